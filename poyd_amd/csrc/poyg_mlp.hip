@@ -113,12 +113,6 @@ __global__ __launch_bounds__(256) void pair_feature_any_kernel(const float *__re
 // C[4*(l/16) + r][l%16], r = 0..3.  Rows i >= M, columns j >= N and k >= K
 // read as zero and are not stored.
 // ---------------------------------------------------------------------------
-enum GemmEpi : int {
-  kEpiBiasReluBf16 = 0,   // out bf16 = relu(acc + bias[j])
-  kEpiMaskBf16 = 1,       // out bf16 = acc where mask(i, j) > 0, else 0
-  kEpiF32 = 2,            // out f32 = acc
-};
-
 constexpr int kTM = 64, kTN = 64, kTK = 32, kLdsK = kTK + 8;   // row pad: 16 bytes
 
 __device__ __forceinline__ void load_tile(uint16_t (*dst)[kLdsK], const uint16_t *__restrict__ src, int64_t rs,
@@ -141,30 +135,23 @@ __device__ __forceinline__ void load_tile(uint16_t (*dst)[kLdsK], const uint16_t
   }
 }
 
-template <int kEpi>
 __global__ __launch_bounds__(256) void gemm_bf16_kernel(int M, int N, int K, const uint16_t *__restrict__ A,
                                                         int64_t a_rs, int64_t a_cs, const uint16_t *__restrict__ B,
-                                                        int64_t b_rs, int64_t b_cs, const float *__restrict__ bias,
-                                                        const uint16_t *__restrict__ mask, int64_t ldm,
-                                                        void *__restrict__ out, int64_t ldc, int kchunk,
-                                                        int64_t split_stride) {
+                                                        int64_t b_rs, int64_t b_cs, float *__restrict__ out,
+                                                        int64_t ldc) {
   __shared__ __attribute__((aligned(16))) uint16_t As[kTM][kLdsK];
   __shared__ __attribute__((aligned(16))) uint16_t Bs[kTN][kLdsK];
   const int i0 = blockIdx.x * kTM, j0 = blockIdx.y * kTN;
   const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
   const int qi = (wv >> 1) * 32, qj = (wv & 1) * 32;
-  // split K: workgroup z takes k in [z kchunk, (z + 1) kchunk) and writes
-  // its partial product split_stride elements further (f32 output only)
-  const int kz0 = blockIdx.z * kchunk, kz1 = min(K, kz0 + kchunk);
-  if (kEpi == kEpiF32) out = (float *)out + blockIdx.z * split_stride;
   f32x4 acc[2][2];
   for (int a = 0; a < 2; ++a)
     for (int b = 0; b < 2; ++b) acc[a][b] = f32x4{0.f, 0.f, 0.f, 0.f};
-  for (int k0 = kz0; k0 < kz1; k0 += kTK) {
+  for (int k0 = 0; k0 < K; k0 += kTK) {
     __syncthreads();
-    load_tile(As, A, a_rs, a_cs, i0, M, k0, kz1);
+    load_tile(As, A, a_rs, a_cs, i0, M, k0, K);
     // B(k, j): rows of the LDS tile are columns j, k contiguous
-    load_tile(Bs, B, b_cs, b_rs, j0, N, k0, kz1);
+    load_tile(Bs, B, b_cs, b_rs, j0, N, k0, K);
     __syncthreads();
     const int kk = 8 * (lane >> 4);
     bf16x8 av[2], bv[2];
@@ -178,16 +165,7 @@ __global__ __launch_bounds__(256) void gemm_bf16_kernel(int M, int N, int K, con
       for (int r = 0; r < 4; ++r) {
         const int i = i0 + qi + 16 * a + 4 * (lane >> 4) + r;
         const int j = j0 + qj + 16 * b + (lane & 15);
-        if (i >= M || j >= N) continue;
-        const float v = acc[a][b][r];
-        if (kEpi == kEpiBiasReluBf16) {
-          ((uint16_t *)out)[(int64_t)i * ldc + j] = f2bf(fmaxf(v + bias[j], 0.f));
-        } else if (kEpi == kEpiMaskBf16) {
-          const bool on = bf2f(mask[(int64_t)i * ldm + j]) > 0.f;
-          ((uint16_t *)out)[(int64_t)i * ldc + j] = on ? f2bf(v) : (uint16_t)0;
-        } else {
-          ((float *)out)[(int64_t)i * ldc + j] = v;
-        }
+        if (i < M && j < N) out[(int64_t)i * ldc + j] = acc[a][b][r];
       }
 }
 
@@ -210,17 +188,23 @@ __global__ __launch_bounds__(256) void gemm_bf16_kernel(int M, int N, int K, con
 constexpr int kNetWaves = 8;
 constexpr int kRowPad = kH + 8;   // LDS row of 256 bf16 and 16 bytes of padding
 
-// A wave's 32 columns of one layer: A operands W[n][k..k+7] of two 16-column
-// blocks, from rows of 256 k-contiguous weights.
+// The bf16 copies of the hidden layers' weights lie in MFMA operand order:
+// element (n, k) of the operand A(n, k) = W[k][n] (W[n][k] for the backward
+// product) at the place of its 16 x 32 block, lane and half word, so that a
+// wave reads an operand as one contiguous kilobyte.
+__device__ __forceinline__ int frag_at(int n, int k) {
+  return ((n >> 4) * 8 + (k >> 5)) * 512 + (((k >> 3) & 3) * 16 + (n & 15)) * 8 + (k & 7);
+}
+
+// A wave's 32 columns of one layer: the A operands of two 16-column blocks.
 struct NetSlice {
   bf16x8 a[2][8];
   __device__ __forceinline__ void load(const uint16_t *__restrict__ w, int n0) {
-    const int lane = threadIdx.x & 63;
 #pragma unroll
     for (int b = 0; b < 2; ++b)
 #pragma unroll
       for (int k = 0; k < 8; ++k)
-        a[b][k] = *(const bf16x8 *)(w + (n0 + 16 * b + (lane & 15)) * kH + 32 * k + 8 * (lane >> 4));
+        a[b][k] = *(const bf16x8 *)(w + ((n0 >> 4) + b) * 4096 + 512 * k + 8 * (threadIdx.x & 63));
   }
   // acc[b] = the slice's block b times the 16 rows at `rows` (LDS)
   __device__ __forceinline__ void mul(const uint16_t (*rows)[kRowPad], f32x4 (&acc)[2]) const {
@@ -327,81 +311,179 @@ __global__ __launch_bounds__(64 * kNetWaves, 2) void net_forward_kernel(
   }
 }
 
-// Output layer and loss.  y[m] = sum_k H2[m][k] w3[k] + b3; with targets,
-// dy[m] = 2 (y[m] - t[m]) / n (mean squared error), dZ2[m][k] =
-// bf16(dy[m] w3[k]) where H2[m][k] > 0, and loss[m] = (y - t)^2 / n.
-// One workgroup of 256 threads per row.
-__global__ __launch_bounds__(256) void head_kernel(int n, const uint16_t *__restrict__ H2,
-                                                   const uint16_t *__restrict__ w3, const float *__restrict__ b3,
-                                                   const float *__restrict__ t, float *__restrict__ y,
-                                                   float *__restrict__ dy, float *__restrict__ loss,
-                                                   uint16_t *__restrict__ dZ2) {
-  __shared__ float part[4];
-  const int k = threadIdx.x, lane = k & 63, wv = k >> 6;
-  const float wk = bf2f(w3[k]);
-  for (int m = blockIdx.x; m < n; m += gridDim.x) {
-    const float h = bf2f(H2[(int64_t)m * kH + k]);
-    float s = h * wk;
-    for (int d = 32; d >= 1; d >>= 1) s += __shfl_xor(s, d);
-    if (lane == 0) part[wv] = s;
-    __syncthreads();
-    const float ym = ((part[0] + part[1]) + (part[2] + part[3])) + b3[0];
-    __syncthreads();
-    if (k == 0 && y) y[m] = ym;
-    if (t) {
-      const float e = ym - t[m];
-      const float g = 2.f * e / (float)n;
-      if (k == 0) {
-        dy[m] = g;
-        loss[m] = e * e / (float)n;
-      }
-      dZ2[(int64_t)m * kH + k] = h > 0.f ? f2bf(g * wk) : (uint16_t)0;
+// ---------------------------------------------------------------------------
+// One training step in four launches: net_grad (forward, loss, back-propagated
+// errors), net_wgrad (both weight gradients), net_reduce (their partial sums
+// and the biases', in a fixed order) and adam (below).  A batch of 4,096 rows
+// is too little work for the chip to hide 17 dependent launches (170 us a
+// step; the weight gradients' products alone 47 us, reading both operands
+// against their layout one element at a time).  Now 38 us: net_grad 16 (bound
+// by the 384 KB of weights every workgroup reads from L2; 23 while each product
+// waited for its own in 64-byte pieces), net_wgrad 10, net_reduce 7, adam 4.
+//
+// net_grad: a workgroup of eight waves takes 16 rows (256 workgroups for 4,096
+// rows) as net_forward does, keeps both layers' activations in LDS, and goes
+// back: with e = y - t, dy = 2 e / n (mean squared error), dZ2[m][k] =
+// bf16(dy[m] w3[k]) where H2[m][k] > 0, dZ1 = bf16(dZ2 W2^T) where H1 > 0.
+// X, H1, dZ1 and dZ2 are stored transposed (column k: ldt rows, contiguous),
+// so that the weight gradients read both operands along their sum; rows n ..
+// 16 gridDim.x - 1 are stored as zeros.  Per workgroup, the sums over its rows
+// of dZ1, dZ2 and H2 dy go to colpart[block][3][256], those of dy and of the
+// loss e^2 / n to rowpart[block][2].
+// ---------------------------------------------------------------------------
+__global__ __launch_bounds__(64 * kNetWaves, 2) void net_grad_kernel(
+    int n, const uint16_t *__restrict__ x, const float *__restrict__ t, const uint16_t *__restrict__ w1t,
+    const float *__restrict__ b1, const uint16_t *__restrict__ w2t, const float *__restrict__ b2,
+    const uint16_t *__restrict__ w2b, const uint16_t *__restrict__ w3, const float *__restrict__ b3,
+    uint16_t *__restrict__ xT, uint16_t *__restrict__ h1T, uint16_t *__restrict__ dz1T, uint16_t *__restrict__ dz2T,
+    int64_t ldt, float *__restrict__ colpart, float *__restrict__ rowpart) {
+  __shared__ __attribute__((aligned(16))) uint16_t xs[16][kRowPad], h1[16][kRowPad], h2[16][kRowPad],
+      d1[16][kRowPad], d2[16][kRowPad];
+  __shared__ float part[kNetWaves][16], dy[16];
+  const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
+  const int n0 = 32 * wv, c0 = n0 + 4 * (lane >> 4), row = lane & 15;
+  const int r0 = 16 * blockIdx.x;
+  const bool live = r0 + row < n;
+  NetSlice s1, s2, s3;   // one round of loads for the three products
+  s1.load(w1t, n0);
+  s2.load(w2t, n0);
+  s3.load(w2b, n0);
+  {
+    const int r = tid >> 5;
+    *(uint4 *)&xs[r][8 * (tid & 31)] =
+        r0 + r < n ? *(const uint4 *)(x + (int64_t)(r0 + r) * kH + 8 * (tid & 31)) : make_uint4(0, 0, 0, 0);
+  }
+  __syncthreads();
+  f32x4 acc[2];
+  s1.mul(xs, acc);
+#pragma unroll
+  for (int b = 0; b < 2; ++b)
+    *(uint2 *)&h1[row][c0 + 16 * b] = live ? pack_relu(acc[b], load4_f(b1 + c0 + 16 * b)) : make_uint2(0, 0);
+  __syncthreads();
+  s2.mul(h1, acc);
+  float4 wo[2];
+  uint2 h[2];
+  float p = 0.f;
+#pragma unroll
+  for (int b = 0; b < 2; ++b) {
+    wo[b] = load4_bf(w3 + c0 + 16 * b);
+    h[b] = live ? pack_relu(acc[b], load4_f(b2 + c0 + 16 * b)) : make_uint2(0, 0);
+    *(uint2 *)&h2[row][c0 + 16 * b] = h[b];
+    p += dot4(h[b], wo[b]);
+  }
+  p += __shfl_xor(p, 16);
+  p += __shfl_xor(p, 32);
+  if (lane < 16) part[wv][row] = p;
+  __syncthreads();
+  float y = b3[0];
+#pragma unroll
+  for (int w = 0; w < kNetWaves; ++w) y += part[w][row];
+  const float e = live ? y - t[r0 + row] : 0.f;
+  const float g = 2.f * e / (float)n;
+  if (wv == 0) {
+    if (lane < 16) dy[row] = g;
+    float sg = g, sl = e * e / (float)n;
+#pragma unroll
+    for (int d = 8; d >= 1; d >>= 1) {
+      sg += __shfl_xor(sg, d);
+      sl += __shfl_xor(sl, d);
+    }
+    if (lane == 0) {
+      rowpart[2 * blockIdx.x] = sg;
+      rowpart[2 * blockIdx.x + 1] = sl;
     }
   }
-}
-
-// Column sums over the batch: out[j] = sum_m X[m][j] (X bf16), or
-// sum_m X[m][j] * w[m] when w is given.  Two passes with a fixed order, so
-// that the sums are deterministic: workgroup b sums rows
-// [b * rows, (b + 1) * rows) of every column into part[b][j] (one thread
-// per column, four row streams interleaved to keep loads in flight); then
-// one thread per column adds the kColParts partials in order.
-constexpr int kColParts = 64;
-__global__ __launch_bounds__(256) void colsum_part_kernel(int n, const uint16_t *__restrict__ X,
-                                                          const float *__restrict__ w, float *__restrict__ part) {
-  const int j = threadIdx.x;   // kH == 256 columns
-  const int rows = (n + kColParts - 1) / kColParts;
-  const int m0 = blockIdx.x * rows, m1 = min(n, m0 + rows);
-  float s[4] = {0.f, 0.f, 0.f, 0.f};
-  int m = m0;
-  for (; m + 3 < m1; m += 4) {
 #pragma unroll
-    for (int r = 0; r < 4; ++r) s[r] += bf2f(X[(int64_t)(m + r) * kH + j]) * (w ? w[m + r] : 1.f);
+  for (int b = 0; b < 2; ++b) {
+    auto q = [&](float hv, float w) { return hv > 0.f ? (uint32_t)f2bf(g * w) : 0u; };   // (h is 0 past the last row)
+    *(uint2 *)&d2[row][c0 + 16 * b] =
+        make_uint2(q(bf_lo(h[b].x), wo[b].x) | (q(bf_hi(h[b].x), wo[b].y) << 16),
+                   q(bf_lo(h[b].y), wo[b].z) | (q(bf_hi(h[b].y), wo[b].w) << 16));
   }
-  for (; m < m1; ++m) s[0] += bf2f(X[(int64_t)m * kH + j]) * (w ? w[m] : 1.f);
-  part[blockIdx.x * kH + j] = (s[0] + s[1]) + (s[2] + s[3]);
-}
-
-__global__ __launch_bounds__(256) void colsum_fin_kernel(const float *__restrict__ part, float *__restrict__ out) {
-  const int j = threadIdx.x;
-  float s = 0.f;
-  for (int b = 0; b < kColParts; ++b) s += part[b * kH + j];
-  out[j] = s;
-}
-
-// sum of a vector (one workgroup, deterministic order per thread then a
-// fixed tree)
-__global__ __launch_bounds__(256) void vsum_kernel(int n, const float *__restrict__ v, float *__restrict__ out) {
-  __shared__ float part[256];
-  float s = 0.f;
-  for (int m = threadIdx.x; m < n; m += 256) s += v[m];
-  part[threadIdx.x] = s;
   __syncthreads();
-  for (int d = 128; d >= 1; d >>= 1) {
-    if ((int)threadIdx.x < d) part[threadIdx.x] += part[threadIdx.x + d];
-    __syncthreads();
+  s3.mul(d2, acc);
+#pragma unroll
+  for (int b = 0; b < 2; ++b) {
+    const uint2 m = *(const uint2 *)&h1[row][c0 + 16 * b];
+    auto q = [&](float hv, float v) { return hv > 0.f ? (uint32_t)f2bf(v) : 0u; };
+    *(uint2 *)&d1[row][c0 + 16 * b] = make_uint2(q(bf_lo(m.x), acc[b][0]) | (q(bf_hi(m.x), acc[b][1]) << 16),
+                                                 q(bf_lo(m.y), acc[b][2]) | (q(bf_hi(m.y), acc[b][3]) << 16));
   }
-  if (threadIdx.x == 0) out[0] = part[0];
+  __syncthreads();
+  // columns: thread 2c + half takes rows 8 half .. +7 of column c
+  const int c = tid >> 1, q0 = 8 * (tid & 1);
+  const int64_t at = c * ldt + r0 + q0;
+  auto column = [&](const uint16_t (*m)[kRowPad], uint16_t *out) {
+    uint32_t v[4];
+    float sum = 0.f;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const uint32_t lo = m[q0 + 2 * r][c], hi = m[q0 + 2 * r + 1][c];
+      v[r] = lo | (hi << 16);
+      sum += bf2f((uint16_t)lo) + bf2f((uint16_t)hi);
+    }
+    *(uint4 *)(out + at) = make_uint4(v[0], v[1], v[2], v[3]);
+    return sum + __shfl_xor(sum, 1);
+  };
+  column(xs, xT);
+  column(h1, h1T);
+  const float sb1 = column(d1, dz1T), sb2 = column(d2, dz2T);
+  float sw = 0.f;
+#pragma unroll
+  for (int r = 0; r < 8; ++r) sw += bf2f(h2[q0 + r][c]) * dy[q0 + r];
+  sw += __shfl_xor(sw, 1);
+  if (q0 == 0) {
+    float *o = colpart + (int64_t)blockIdx.x * 3 * kH + c;
+    o[0] = sb1;
+    o[kH] = sb2;
+    o[2 * kH] = sw;
+  }
+}
+
+// Weight gradients dW1 = X^T dZ1 and dW2 = H1^T dZ2 over rows [chunk z,
+// chunk (z + 1)) of `rows` (a multiple of 32) for workgroup (tile, matrix, z):
+// a 64 x 64 tile of one of them, each wave a 32 x 32 quadrant, MFMA operands
+// read straight from the transposed operands (16 contiguous bytes per lane,
+// no LDS: every operand line is used by two waves of the workgroup and comes
+// from L2).  Splitting the rows gives the 32 tiles enough workgroups for the
+// chip.
+constexpr int kWgSplits = 8;
+__global__ __launch_bounds__(256) void net_wgrad_kernel(int rows, int chunk, int64_t ldt,
+                                                        const uint16_t *__restrict__ xT,
+                                                        const uint16_t *__restrict__ h1T,
+                                                        const uint16_t *__restrict__ dz1T,
+                                                        const uint16_t *__restrict__ dz2T,
+                                                        float *__restrict__ part) {
+  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+  const int i0 = (blockIdx.x >> 2) * 64 + (wv >> 1) * 32, j0 = (blockIdx.x & 3) * 64 + (wv & 1) * 32;
+  const bool second = blockIdx.y == 1;
+  const int64_t off = (lane & 15) * ldt + 8 * (lane >> 4);
+  const uint16_t *A = (second ? h1T : xT) + i0 * ldt + off, *B = (second ? dz2T : dz1T) + j0 * ldt + off;
+  const int k1 = min(rows, (int)(blockIdx.z + 1) * chunk);
+  f32x4 acc[2][2];
+  for (int a = 0; a < 2; ++a)
+    for (int b = 0; b < 2; ++b) acc[a][b] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll 4
+  for (int k = blockIdx.z * chunk; k < k1; k += 32) {
+    bf16x8 av[2], bv[2];
+#pragma unroll
+    for (int a = 0; a < 2; ++a) {
+      av[a] = *(const bf16x8 *)(A + 16 * a * ldt + k);
+      bv[a] = *(const bf16x8 *)(B + 16 * a * ldt + k);
+    }
+#pragma unroll
+    for (int a = 0; a < 2; ++a)
+#pragma unroll
+      for (int b = 0; b < 2; ++b) acc[a][b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(av[a], bv[b], acc[a][b], 0, 0, 0);
+  }
+  float *o = part + ((int64_t)blockIdx.z * 2 + blockIdx.y) * kH * kH;
+#pragma unroll
+  for (int a = 0; a < 2; ++a)
+#pragma unroll
+    for (int b = 0; b < 2; ++b)
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+        o[(i0 + 16 * a + 4 * (lane >> 4) + r) * kH + j0 + 16 * b + (lane & 15)] = acc[a][b][r];
 }
 
 // dst row r = src row idx[r] (rows of `words` 32-bit words): batch
@@ -416,38 +498,106 @@ __global__ __launch_bounds__(256) void gather_rows_kernel(const uint32_t *__rest
   }
 }
 
-// Adam over the flat parameter vector, then the bf16 copies the products
-// read: W1t[n][k] = W1[k][n], W2t[n][k] = W2[k][n], W2b = W2, w3b = w3.
+// Adam over the flat parameter vector, and the bf16 copies the products read
+// (frag_at): w1t(n, k) = W1[k][n], w2t(n, k) = W2[k][n], w2b(k, n) = W2[k][n],
+// w3b = w3.
 struct MlpLayout {
   static constexpr int64_t W1 = 0, B1 = W1 + kH * kH, W2 = B1 + kH, B2 = W2 + kH * kH, W3 = B2 + kH,
                            B3 = W3 + kH, N = B3 + 1;
 };
 
+// Sums of a step's partials, each in a fixed order: workgroups 0 .. 511 the
+// weight gradients (one element per thread over the splits), the next 48 the
+// column sums of b1, b2 and w3 (16 columns by 16 interleaved groups of net_grad
+// workgroups, then the groups in order), the last one b3's and the loss.
+constexpr int kReduceBlocks = 2 * kH + 3 * kH / 16 + 1;
+__global__ __launch_bounds__(256) void net_reduce_kernel(int splits, int tiles, const float *__restrict__ part,
+                                                         const float *__restrict__ colpart,
+                                                         const float *__restrict__ rowpart, float *__restrict__ g,
+                                                         float *__restrict__ loss) {
+  __shared__ float sum[2][256];
+  const int t = threadIdx.x;
+  int b = blockIdx.x;
+  if (b < 2 * kH) {
+    const int64_t e = (int64_t)(b & (kH - 1)) * 256 + t;
+    const float *q = part + (b >> 8) * kH * kH + e;
+    float s = 0.f;
+    for (int z = 0; z < splits; ++z) s += q[(int64_t)z * 2 * kH * kH];
+    g[(b >> 8 ? MlpLayout::W2 : MlpLayout::W1) + e] = s;
+    return;
+  }
+  b -= 2 * kH;
+  if (b < 3 * kH / 16) {
+    const int sec = b >> 4, c = (b & 15) * 16 + (t & 15), grp = t >> 4;
+    float s = 0.f;
+    for (int m = grp; m < tiles; m += 16) s += colpart[((int64_t)m * 3 + sec) * kH + c];
+    sum[0][t] = s;
+    __syncthreads();
+    if (t < 16) {
+      float r = 0.f;
+      for (int q = 0; q < 16; ++q) r += sum[0][16 * q + t];
+      g[(sec == 0 ? MlpLayout::B1 : sec == 1 ? MlpLayout::B2 : MlpLayout::W3) + c] = r;
+    }
+    return;
+  }
+  float s0 = 0.f, s1 = 0.f;
+  for (int m = t; m < tiles; m += 256) {
+    s0 += rowpart[2 * m];
+    s1 += rowpart[2 * m + 1];
+  }
+  sum[0][t] = s0;
+  sum[1][t] = s1;
+  __syncthreads();
+  for (int d = 128; d >= 1; d >>= 1) {
+    if (t < d) {
+      sum[0][t] += sum[0][t + d];
+      sum[1][t] += sum[1][t + d];
+    }
+    __syncthreads();
+  }
+  if (t == 0) {
+    g[MlpLayout::B3] = sum[0][0];
+    loss[0] = sum[1][0];
+  }
+}
+
+// The bf16 copies of parameter i that the products read.
+__device__ __forceinline__ void cast_param(int64_t i, float v, uint16_t *w1t, uint16_t *w2t, uint16_t *w2b,
+                                           uint16_t *w3b) {
+  const uint16_t h = f2bf(v);
+  if (i < MlpLayout::B1) {
+    w1t[frag_at((int)(i % kH), (int)(i / kH))] = h;
+  } else if (i >= MlpLayout::W2 && i < MlpLayout::B2) {
+    const int e = (int)(i - MlpLayout::W2), in = e / kH, out = e % kH;
+    w2t[frag_at(out, in)] = h;
+    w2b[frag_at(in, out)] = h;
+  } else if (i >= MlpLayout::W3 && i < MlpLayout::B3) {
+    w3b[i - MlpLayout::W3] = h;
+  }
+}
+
 __global__ __launch_bounds__(256) void adam_kernel(int64_t n, float *__restrict__ p, const float *__restrict__ g,
                                                    float *__restrict__ m1, float *__restrict__ m2, float lr,
-                                                   float b1, float b2, float eps, float c1, float c2) {
+                                                   float b1, float b2, float eps, float c1, float c2,
+                                                   uint16_t *__restrict__ w1t, uint16_t *__restrict__ w2t,
+                                                   uint16_t *__restrict__ w2b, uint16_t *__restrict__ w3b) {
   for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x) {
     const float gi = g[i];
     const float a = b1 * m1[i] + (1.f - b1) * gi;
     const float b = b2 * m2[i] + (1.f - b2) * gi * gi;
     m1[i] = a;
     m2[i] = b;
-    p[i] -= lr * (a / c1) / (sqrtf(b / c2) + eps);
+    const float v = p[i] - lr * (a / c1) / (sqrtf(b / c2) + eps);
+    p[i] = v;
+    cast_param(i, v, w1t, w2t, w2b, w3b);
   }
 }
 
 __global__ __launch_bounds__(256) void cast_params_kernel(const float *__restrict__ p, uint16_t *__restrict__ w1t,
                                                           uint16_t *__restrict__ w2t, uint16_t *__restrict__ w2b,
                                                           uint16_t *__restrict__ w3b) {
-  const int64_t e = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-  if (e < kH * kH) {
-    const int k = (int)(e / kH), j = (int)(e % kH);
-    w1t[(int64_t)j * kH + k] = f2bf(p[MlpLayout::W1 + e]);
-    const uint16_t v = f2bf(p[MlpLayout::W2 + e]);
-    w2t[(int64_t)j * kH + k] = v;
-    w2b[e] = v;
-  }
-  if (e < kH) w3b[e] = f2bf(p[MlpLayout::W3 + e]);
+  const int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
+  if (i < MlpLayout::N) cast_param(i, p[i], w1t, w2t, w2b, w3b);
 }
 
 }  // namespace poyg
@@ -472,80 +622,21 @@ struct poyg_mlp {
   // f32: params, grads, Adam moments; bf16 copies; batch scratch
   float *p = nullptr, *g = nullptr, *m1 = nullptr, *m2 = nullptr;
   uint16_t *w1t = nullptr, *w2t = nullptr, *w2b = nullptr, *w3b = nullptr;
-  uint16_t *h1 = nullptr, *h2 = nullptr, *dz2 = nullptr, *dz1 = nullptr;
-  float *y = nullptr, *dy = nullptr, *loss = nullptr, *lsum = nullptr;
-  float *cpart = nullptr;   // column-sum partials, kColParts x kH per sum
-  float *wpart = nullptr;   // split-K partials of a weight gradient
+  uint16_t *xT = nullptr, *h1T = nullptr, *dz2T = nullptr, *dz1T = nullptr;   // transposed, ldt rows a column
+  int64_t ldt = 0;
+  float *lsum = nullptr;
+  float *cpart = nullptr, *rpart = nullptr;   // net_grad's partial sums per workgroup
+  float *wpart = nullptr;                     // net_wgrad's partial products
   ~poyg_mlp() {
     for (void *q : {(void *)p, (void *)g, (void *)m1, (void *)m2, (void *)w1t, (void *)w2t, (void *)w2b,
-                    (void *)w3b, (void *)h1, (void *)h2, (void *)dz2, (void *)dz1, (void *)y, (void *)dy,
-                    (void *)loss, (void *)lsum, (void *)cpart, (void *)wpart})
+                    (void *)w3b, (void *)xT, (void *)h1T, (void *)dz2T, (void *)dz1T, (void *)lsum, (void *)cpart,
+                    (void *)rpart, (void *)wpart})
       if (q) (void)hipFree(q);
   }
 };
 
 extern "C" void *poyg_ctx_stream(poyg_ctx *ctx);
 extern "C" int poyg_ctx_device(poyg_ctx *ctx);
-
-static hipError_t gemm(int epi, int M, int N, int K, const uint16_t *A, int64_t a_rs, int64_t a_cs,
-                       const uint16_t *B, int64_t b_rs, int64_t b_cs, const float *bias, const uint16_t *mask,
-                       int64_t ldm, void *C, int64_t ldc, hipStream_t s) {
-  if (M <= 0 || N <= 0) return hipSuccess;
-  dim3 grid((M + kTM - 1) / kTM, (N + kTN - 1) / kTN);
-  const int kall = std::max(K, 1);
-  if (epi == kEpiBiasReluBf16)
-    hipLaunchKernelGGL(gemm_bf16_kernel<kEpiBiasReluBf16>, grid, dim3(256), 0, s, M, N, K, A, a_rs, a_cs, B, b_rs,
-                       b_cs, bias, mask, ldm, C, ldc, kall, (int64_t)0);
-  else if (epi == kEpiMaskBf16)
-    hipLaunchKernelGGL(gemm_bf16_kernel<kEpiMaskBf16>, grid, dim3(256), 0, s, M, N, K, A, a_rs, a_cs, B, b_rs,
-                       b_cs, bias, mask, ldm, C, ldc, kall, (int64_t)0);
-  else
-    hipLaunchKernelGGL(gemm_bf16_kernel<kEpiF32>, grid, dim3(256), 0, s, M, N, K, A, a_rs, a_cs, B, b_rs, b_cs,
-                       bias, mask, ldm, C, ldc, kall, (int64_t)0);
-  return hipGetLastError();
-}
-
-// C (f32, M x N, ldc) = sum over z of part[z] (M x N each), in order.
-__global__ __launch_bounds__(256) void split_sum_kernel(int M, int N, int splits, const float *__restrict__ part,
-                                                        float *__restrict__ C, int64_t ldc) {
-  const int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (e >= (int64_t)M * N) return;
-  float s = 0.f;
-  for (int z = 0; z < splits; ++z) s += part[z * (int64_t)M * N + e];
-  C[(e / N) * ldc + e % N] = s;
-}
-
-// Weight gradients (M = N = kH, K = the batch): K split into kWgSplits
-// chunks so that 16 output tiles become 16 * kWgSplits workgroups; the
-// partial products go to `part` (kWgSplits x M x N floats) and are added
-// in a fixed order, so the result does not depend on scheduling.
-constexpr int kWgSplits = 32;
-static hipError_t gemm_wgrad(int M, int N, int K, const uint16_t *A, int64_t a_rs, int64_t a_cs, const uint16_t *B,
-                             int64_t b_rs, int64_t b_cs, float *part, float *C, int64_t ldc, hipStream_t s) {
-  if (M <= 0 || N <= 0) return hipSuccess;
-  const int chunk = std::max(kTK, (K + kWgSplits - 1) / kWgSplits + kTK - 1) / kTK * kTK;
-  const int splits = std::max(1, (K + chunk - 1) / chunk);
-  dim3 grid((M + kTM - 1) / kTM, (N + kTN - 1) / kTN, splits);
-  hipLaunchKernelGGL(gemm_bf16_kernel<kEpiF32>, grid, dim3(256), 0, s, M, N, K, A, a_rs, a_cs, B, b_rs, b_cs,
-                     (const float *)nullptr, (const uint16_t *)nullptr, (int64_t)0, (void *)part, (int64_t)N, chunk,
-                     (int64_t)M * N);
-  const int64_t tot = (int64_t)M * N;
-  hipLaunchKernelGGL(split_sum_kernel, dim3((unsigned)((tot + 255) / 256)), dim3(256), 0, s, M, N, splits, part, C,
-                     ldc);
-  return hipGetLastError();
-}
-
-// forward of n <= batch_max rows into m->h1, m->h2 and (optionally) y
-static int mlp_forward_batch(poyg_mlp *m, const uint16_t *x, int n, float *y, const float *t, hipStream_t s) {
-  HIP_TRYM(gemm(kEpiBiasReluBf16, n, kH, kH, x, kH, 1, m->w1t, 1, kH, m->p + MlpLayout::B1, nullptr, 0, m->h1, kH,
-                s));
-  HIP_TRYM(gemm(kEpiBiasReluBf16, n, kH, kH, m->h1, kH, 1, m->w2t, 1, kH, m->p + MlpLayout::B2, nullptr, 0, m->h2,
-                kH, s));
-  hipLaunchKernelGGL(head_kernel, dim3(std::min(n, 65536)), dim3(256), 0, s, n, m->h2, m->w3b, m->p + MlpLayout::B3,
-                     t, y, m->dy, m->loss, m->dz2);
-  HIP_TRYM(hipGetLastError());
-  return POYG_OK;
-}
 
 extern "C" {
 
@@ -564,7 +655,10 @@ int poyg_mlp_create(poyg_ctx *ctx, int batch_max, uint64_t seed, poyg_mlp **out)
   m->batch_max = batch_max;
   m->cus = ctx_cus(ctx);
   hipError_t e = hipSetDevice(m->device);
-  const size_t np = (size_t)MlpLayout::N, nb = (size_t)batch_max;
+  // rows of a batch, rounded to the weight gradients' 32, and 32 more so that
+  // the columns do not all start in the same memory channel
+  const size_t np = (size_t)MlpLayout::N, nb = ((size_t)batch_max + 31) / 32 * 32;
+  m->ldt = (int64_t)nb + 32;
   auto A = [&](void **q, size_t bytes) {
     if (e == hipSuccess) e = hipMalloc(q, std::max<size_t>(bytes, 16));
   };
@@ -576,16 +670,11 @@ int poyg_mlp_create(poyg_ctx *ctx, int batch_max, uint64_t seed, poyg_mlp **out)
   A((void **)&m->w2t, 2 * kH * kH);
   A((void **)&m->w2b, 2 * kH * kH);
   A((void **)&m->w3b, 2 * kH);
-  A((void **)&m->h1, 2 * nb * kH);
-  A((void **)&m->h2, 2 * nb * kH);
-  A((void **)&m->dz2, 2 * nb * kH);
-  A((void **)&m->dz1, 2 * nb * kH);
-  A((void **)&m->y, 4 * nb);
-  A((void **)&m->dy, 4 * nb);
-  A((void **)&m->loss, 4 * nb);
+  for (uint16_t **q : {&m->xT, &m->h1T, &m->dz2T, &m->dz1T}) A((void **)q, 2 * (size_t)m->ldt * kH);
   A((void **)&m->lsum, 16);
-  A((void **)&m->cpart, 4 * 3 * kColParts * kH);
-  A((void **)&m->wpart, 4 * (size_t)kWgSplits * kH * kH);
+  A((void **)&m->cpart, 4 * 3 * (nb / 16) * kH);
+  A((void **)&m->rpart, 4 * 2 * (nb / 16));
+  A((void **)&m->wpart, 4 * 2 * (size_t)kWgSplits * kH * kH);
   if (e != hipSuccess) {
     delete m;
     set_error("poyg_mlp_create: hipMalloc failed: %s", hipGetErrorString(e));
@@ -624,8 +713,8 @@ int poyg_mlp_set_params(poyg_mlp *m, const float *host, int64_t n) {
   HIP_TRYM(hipMemcpyAsync(m->p, host, 4 * (size_t)n, hipMemcpyHostToDevice, m->stream));
   HIP_TRYM(hipMemsetAsync(m->m1, 0, 4 * (size_t)n, m->stream));
   HIP_TRYM(hipMemsetAsync(m->m2, 0, 4 * (size_t)n, m->stream));
-  hipLaunchKernelGGL(cast_params_kernel, dim3((kH * kH + 255) / 256), dim3(256), 0, m->stream, m->p, m->w1t, m->w2t,
-                     m->w2b, m->w3b);
+  hipLaunchKernelGGL(cast_params_kernel, dim3((MlpLayout::N + 255) / 256), dim3(256), 0, m->stream, m->p, m->w1t,
+                     m->w2t, m->w2b, m->w3b);
   HIP_TRYM(hipGetLastError());
   HIP_TRYM(hipStreamSynchronize(m->stream));
   m->step = 0;
@@ -672,26 +761,20 @@ int poyg_mlp_grad(poyg_mlp *m, const uint16_t *d_x, const float *d_t, int n, flo
     return POYG_EINVAL;
   }
   hipStream_t s = m->stream;
-  int rc = mlp_forward_batch(m, d_x, n, m->y, d_t, s);
-  if (rc) return rc;
-  float *g = m->g;
-  // dZ1 = (dZ2 W2^T) where H1 > 0: B(k', j) = W2[j][k'] (W2b is [in][out])
-  HIP_TRYM(gemm(kEpiMaskBf16, n, kH, kH, m->dz2, kH, 1, m->w2b, 1, kH, nullptr, m->h1, kH, m->dz1, kH, s));
-  // dW2[k][j] = sum_m H1[m][k] dZ2[m][j]; dW1[k][j] = sum_m X[m][k] dZ1[m][j]
-  HIP_TRYM(gemm_wgrad(kH, kH, n, m->h1, 1, kH, m->dz2, kH, 1, m->wpart, g + MlpLayout::W2, kH, s));
-  HIP_TRYM(gemm_wgrad(kH, kH, n, d_x, 1, kH, m->dz1, kH, 1, m->wpart, g + MlpLayout::W1, kH, s));
-  float *cp = m->cpart;
-  hipLaunchKernelGGL(colsum_part_kernel, dim3(kColParts), dim3(kH), 0, s, n, m->dz2, nullptr, cp);
-  hipLaunchKernelGGL(colsum_part_kernel, dim3(kColParts), dim3(kH), 0, s, n, m->dz1, nullptr, cp + kColParts * kH);
-  hipLaunchKernelGGL(colsum_part_kernel, dim3(kColParts), dim3(kH), 0, s, n, m->h2, m->dy, cp + 2 * kColParts * kH);
-  hipLaunchKernelGGL(colsum_fin_kernel, dim3(1), dim3(kH), 0, s, cp, g + MlpLayout::B2);
-  hipLaunchKernelGGL(colsum_fin_kernel, dim3(1), dim3(kH), 0, s, cp + kColParts * kH, g + MlpLayout::B1);
-  hipLaunchKernelGGL(colsum_fin_kernel, dim3(1), dim3(kH), 0, s, cp + 2 * kColParts * kH, g + MlpLayout::W3);
-  hipLaunchKernelGGL(vsum_kernel, dim3(1), dim3(256), 0, s, n, m->dy, g + MlpLayout::B3);
+  const float *p = m->p;
+  const int rows = (n + 31) / 32 * 32, tiles = rows / 16;
+  hipLaunchKernelGGL(net_grad_kernel, dim3(tiles), dim3(64 * kNetWaves), 0, s, n, d_x, d_t, m->w1t, p + MlpLayout::B1,
+                     m->w2t, p + MlpLayout::B2, m->w2b, m->w3b, p + MlpLayout::B3, m->xT, m->h1T, m->dz1T, m->dz2T,
+                     m->ldt, m->cpart, m->rpart);
+  // at least four steps of 32 rows per split
+  const int want = std::max(1, std::min(kWgSplits, rows / 128));
+  const int chunk = (rows / 32 + want - 1) / want * 32, splits = (rows + chunk - 1) / chunk;
+  hipLaunchKernelGGL(net_wgrad_kernel, dim3(16, 2, splits), dim3(256), 0, s, rows, chunk, m->ldt, m->xT, m->h1T,
+                     m->dz1T, m->dz2T, m->wpart);
+  hipLaunchKernelGGL(net_reduce_kernel, dim3(kReduceBlocks), dim3(256), 0, s, splits, tiles, m->wpart, m->cpart,
+                     m->rpart, m->g, m->lsum);
   HIP_TRYM(hipGetLastError());
   if (loss) {
-    hipLaunchKernelGGL(vsum_kernel, dim3(1), dim3(256), 0, s, n, m->loss, m->lsum);
-    HIP_TRYM(hipGetLastError());
     HIP_TRYM(hipMemcpyAsync(loss, m->lsum, 4, hipMemcpyDeviceToHost, s));
     HIP_TRYM(hipStreamSynchronize(s));
   }
@@ -704,9 +787,7 @@ int poyg_mlp_adam(poyg_mlp *m, float lr, float beta1, float beta2, float eps) {
   m->step += 1;
   const float c1 = 1.f - powf(beta1, (float)m->step), c2 = 1.f - powf(beta2, (float)m->step);
   hipLaunchKernelGGL(adam_kernel, dim3(256), dim3(256), 0, m->stream, MlpLayout::N, m->p, m->g, m->m1, m->m2, lr,
-                     beta1, beta2, eps, c1, c2);
-  hipLaunchKernelGGL(cast_params_kernel, dim3((kH * kH + 255) / 256), dim3(256), 0, m->stream, m->p, m->w1t,
-                     m->w2t, m->w2b, m->w3b);
+                     beta1, beta2, eps, c1, c2, m->w1t, m->w2t, m->w2b, m->w3b);
   HIP_TRYM(hipGetLastError());
   return POYG_OK;
 }
@@ -754,13 +835,16 @@ int poyg_gather_rows(poyg_ctx *ctx, const void *d_src, int64_t row_bytes, const 
   return POYG_OK;
 }
 
-// A plain bf16 product for tests of the MFMA tiles: C (f32, ldc) = A B with
-// the strides above.
+// A plain bf16 product for tests of the MFMA operand layout: C (f32, ldc) = A B
+// with the strides above.
 int poyg_gemm_bf16_f32(poyg_ctx *ctx, int M, int N, int K, const uint16_t *d_a, int64_t a_rs, int64_t a_cs,
                        const uint16_t *d_b, int64_t b_rs, int64_t b_cs, float *d_c, int64_t ldc, void *stream) {
   if (!ctx || M < 0 || N < 0 || K < 0) return POYG_EINVAL;
   hipStream_t s = stream ? (hipStream_t)stream : (hipStream_t)poyg_ctx_stream(ctx);
-  HIP_TRYM(gemm(kEpiF32, M, N, K, d_a, a_rs, a_cs, d_b, b_rs, b_cs, nullptr, nullptr, 0, d_c, ldc, s));
+  if (M == 0 || N == 0) return POYG_OK;
+  hipLaunchKernelGGL(gemm_bf16_kernel, dim3((M + kTM - 1) / kTM, (N + kTN - 1) / kTN), dim3(256), 0, s, M, N, K, d_a,
+                     a_rs, a_cs, d_b, b_rs, b_cs, d_c, ldc);
+  HIP_TRYM(hipGetLastError());
   return POYG_OK;
 }
 

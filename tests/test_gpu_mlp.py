@@ -271,3 +271,28 @@ def test_features_of_unaligned_buffers(ctx):
         got = np.empty((37, 256), np.uint16)
         engine._check(engine.load().poyg_dev_download(ctx.h, got.ctypes.data, d_x.ptr + x_off, got.nbytes), "download")
         assert np.array_equal(got, want)
+
+
+def test_gradient_at_tile_edges(ctx):
+    """Batches around the 16-row tiles and the 32-row steps of the weight
+    gradients, a large one first (the scratch keeps its rows).  A rounding
+    that tips moves one term of a sum by one bf16 ulp, 2^-8 of it; two allowed."""
+    from poyd_amd import engine, surrogate
+    rng = np.random.default_rng(8)
+    sc = surrogate.Scorer(ctx, batch_max=5000, seed=6)
+    p = sc.params()
+    p[B1:W2] = rng.uniform(-0.1, 0.1, H)
+    sc.set_params(p)
+    for n in (5000, 1, 15, 16, 17, 31, 32, 33, 127, 129, 1023):
+        note(f"gradient of {n} rows")
+        xb = bf16(np.abs(rng.standard_normal((n, H))).astype(np.float32))
+        t = rng.standard_normal(n).astype(np.float32)
+        dx, dt = engine.DeviceBuffer.from_array(ctx, xb), engine.DeviceBuffer.from_array(ctx, t)
+        loss = sc.grad(dx.ptr, dt.ptr, n, True)
+        g = sc.grads().astype(np.float64)
+        want, wloss = reference_grads(p, xb, t.astype(np.float64))
+        assert abs(loss - wloss) <= 2 ** -7 * max(1.0, wloss)
+        for name, (a, b) in segments().items():
+            rel = np.linalg.norm(g[a:b] - want[a:b]) / max(np.linalg.norm(want[a:b]), 1e-12)
+            assert rel < 2 ** -7, (n, name, rel)
+    sc.close()
