@@ -665,3 +665,46 @@ def test_fitch_widths_match_oracle(ctx, oracle, width):
         assert L.poyg_nonadd_median_3_w(ctx.h, width, a.ctypes.data, b.ctypes.data, c.ctypes.data, d.ctypes.data,
                                         res.ctypes.data, length) == 0
         assert np.array_equal(res, oracle.nonadd_median_3_w(a, b, c, d, width)), length
+
+
+@pytest.mark.parametrize("width", [1, 2, 4])
+def test_fitch_ragged_levels(ctx, oracle, width):
+    """A level of several nodes whose rows start at any byte: row lengths
+    around the 16-byte vectors and the workgroups' share, the result written
+    over an input too, the bytes before and after the rows left alone."""
+    import ctypes as C
+    from poyd_amd import engine
+    dt = {1: np.uint8, 2: np.uint16, 4: np.uint32}[width]
+    rng = np.random.default_rng(90 + width)
+    L = engine.load()
+    for length in (1, 3, 15, 16, 17, 31, 4095, 4097, 65537):
+        note(f"fitch level width {width} length {length}")
+        rows = (np.uint64(1) << rng.integers(0, 8 * width, size=(9, length)).astype(np.uint64)).astype(dt)
+        rows |= (rng.random((9, length)) < 0.3) * (np.uint64(1) << rng.integers(0, 8 * width, size=(9, length)).astype(
+            np.uint64)).astype(dt)
+        host = np.concatenate([np.full(3, 7, dt), rows.ravel(), np.full(5, 9, dt)])
+        d = engine.DeviceBuffer.from_array(ctx, host)
+        at = d.ptr + 3 * width
+        jobs = np.array([[0, 1, 4], [2, 3, 5], [6, 7, 7]], np.int32)   # the last one in place
+        d_jobs = engine.DeviceBuffer.from_array(ctx, np.ascontiguousarray(jobs.T))
+        d_added = engine.DeviceBuffer.from_array(ctx, np.zeros(3, np.int64))
+        assert L.poyg_fitch_down_w(ctx.h, width, at, length, 3, d_jobs.ptr, d_jobs.ptr + 12, d_jobs.ptr + 24,
+                                   d_added.ptr, None) == 0
+        ctx.sync()
+        got = d.download(dt, len(host))
+        added = d_added.download(np.int64, 3)
+        want = rows.copy()
+        for k, (a, b, r) in enumerate(jobs):
+            want[r], n = oracle.nonadd_median_w(rows[a], rows[b], width)
+            assert added[k] == n, (length, k)
+        assert np.array_equal(got[3:-5].reshape(9, length), want), length
+        up = np.array([[8, 4, 0, 1, 6], [8, 5, 2, 3, 5]], np.int32)
+        d_up = engine.DeviceBuffer.from_array(ctx, np.ascontiguousarray(up.T))
+        assert L.poyg_fitch_up_w(ctx.h, width, at, length, 2, *[d_up.ptr + 8 * c for c in range(5)], None) == 0
+        ctx.sync()
+        got = d.download(dt, len(host))
+        final = want.copy()
+        for A, N, D1, D2, F in up:
+            final[F] = oracle.nonadd_median_3_w(want[A], want[N], want[D1], want[D2], width)
+        assert np.array_equal(got[3:-5].reshape(9, length), final), length
+        assert (got[:3] == 7).all() and (got[-5:] == 9).all()
