@@ -13,6 +13,7 @@
 #include "poyg_band.h"
 #include "poyg_ukk.h"
 #include "poyg_internal.h"
+#include "poyg_lindiag.h"
 
 namespace poyg {
 hipError_t launch_reset(int *counters, int n, hipStream_t s);
@@ -62,6 +63,10 @@ hipError_t launch_lin_cost16(bool with_dm, int grid_waves, const PairMeta *meta,
 hipError_t launch_lin_fill(bool with_dm, bool glb, int grid, const PairMeta *meta, const int32_t *order, int n,
                            int *counter, const uint8_t *seq, const DevTcm *tcm, uint8_t *dm, int *aux,
                            int32_t *cost, int *rowscratch, int row_width, hipStream_t s);
+int lin_diag_blocks_per_cu(bool with_dm);
+hipError_t launch_lin_diag(bool with_dm, int waves, int grid, const PairMeta *meta, const int32_t *order, int n,
+                           int *counter, const uint8_t *seq, const DevTcm *tcm, const LinDiagCosts &costs, uint8_t *dm,
+                           int32_t *cost, uint8_t *out, int32_t *out_len, int32_t *status, hipStream_t s);
 int lin_trace_blocks_per_cu();
 hipError_t launch_lin_trace(int grid, const PairMeta *meta, const int32_t *order, int n, int *counter,
                             const uint8_t *seq, const DevTcm *tcm, const uint8_t *dm, uint8_t *out, int32_t *out_len,
@@ -99,9 +104,10 @@ using namespace poyg;
 
 // Launch-shape knobs a tuner may set per context (-1: the built-in choice).
 // lin_cost_kernel: 1 = the 32-bit systolic fill for every linear pair that
-// fits it; the packed 16-bit fill wherever a pair allows it with 2 = one
-// pair per wave for large batches and four waves per pair for small ones
-// (built-in), 3 = one pair per wave, 4 = four waves per pair.
+// fits it; 2 (built-in) = the diagonal fill wherever a pair allows it, else
+// the packed 16-bit strips (one pair per wave for large batches, four waves
+// per pair for small ones); the strips for every pair they take with 3 = one
+// pair per wave, 4 = four waves per pair.
 // aff_narrow_kernel: 1 = the 32-bit four-pair fill for the narrow affine
 // bands, 2 = the packed eight-pair fill (built-in).
 enum TuneKnob : int {
@@ -403,10 +409,16 @@ struct poyg_plan {
   // (linear pairs: the systolic kernel takes every pair whose column
   // sequence fits its LDS row, the row kernels the rest)
   DevBuf tcm, meta, order_all, order_lds, order_glb, order_sys, order_c16, order_quad, order_diag[3], order_rows,
+      order_ldiag,
       dm, aux, rows, counters, status, sink, pure, trout, blob, redo, tlist;
   int n_lds = 0, n_glb = 0, n_sys = 0, n_quad = 0, n_diag[3] = {0, 0, 0}, n_rows = 0;
   int n_c16 = 0, grid_c16 = 0, c16_nmax = 0;   // linear pairs of the packed 16-bit fill
   bool c16_mw = false;                          // ... four waves per pair (grid_c16 counts workgroups)
+  // linear pairs of the diagonal fill (it traces them too): waves of a
+  // workgroup per pair, or 0 for one pair per wave
+  int n_ldiag = 0, grid_ldiag = 0, ldiag_waves = 0;
+  LinDiagCosts ldiag_costs{0, 0, 0};
+  int n_trace = 0;   // linear pairs of the separate backtrace (order_all)
   // the narrow affine bands (order_quad) go to the packed eight-pair fill;
   // its pairs whose cost saturates 16 bits are listed in `redo` for the
   // 32-bit four-pair fill (grid_redo workgroups), launched after it
@@ -431,7 +443,7 @@ struct poyg_plan {
   hipEvent_t fork = nullptr, join = nullptr, join2 = nullptr;   // hand-off to and from the side streams
   ~poyg_plan() {
     if (triple) poyg_triple_plan_destroy(triple);
-    for (DevBuf *b : {&tcm, &meta, &order_all, &order_lds, &order_glb, &order_sys, &order_c16, &order_quad, &order_diag[0],
+    for (DevBuf *b : {&tcm, &meta, &order_all, &order_lds, &order_glb, &order_sys, &order_c16, &order_quad, &order_diag[0], &order_ldiag,
                       &order_diag[1], &order_diag[2], &order_rows, &dm, &aux, &rows, &counters, &status,
                       &sink, &pure, &trout, &blob, &redo, &tlist})
       b->release(idle);
@@ -710,6 +722,7 @@ struct PerCallSeqs {
   // lengths: small_words words; the output sequences)
   int32_t *small_dev = nullptr;
   uint8_t *out_dev = nullptr;
+  bool byte_band = false;   // the caller reads the direction band, one byte per cell
   int64_t small_words = 0;
 };
 
@@ -757,7 +770,10 @@ static int plan_pairs_impl(poyg_ctx *ctx, const poyg_cm *cm, int mode, int32_t n
                                                  : lin_trace_blocks_per_cu();
   std::vector<PairMeta> meta(n);
   std::vector<int64_t> cells(n);
-  std::vector<char> glb(n, 0), diag(n, 0), quad(n, 0), sys(n, 0), c16(n, 0);
+  std::vector<char> glb(n, 0), diag(n, 0), quad(n, 0), sys(n, 0), c16(n, 0), ldiag(n, 0);
+  std::vector<int> widest(affine ? 0 : n);
+  int64_t diag_waves = 0;   // waves the batch's diagonal pairs would take
+  bool diag_multi = false;
   DevTcm dt;
   to_dev_tcm(cm, &dt);
   // the packed 16-bit fill: linear plans whose tail costs equal the
@@ -773,6 +789,12 @@ static int plan_pairs_impl(poyg_ctx *ctx, const poyg_cm *cm, int mode, int32_t n
     c16_matrix = c16_matrix && dt.cost[x] >= 0;
     c16_cmax = std::max<int64_t>(c16_cmax, dt.cost[x]);
   }
+  // the diagonal fill: also row 0's costs equal the insertion costs, and the
+  // caller does not read the band one byte per cell
+  bool ldiag_matrix = c16_matrix && ctx->tune[kTuneLinCost] <= 2 && dt.cost[kGap * 32 + kGap] == 0 &&
+                      !(pc && pc->byte_band);
+  for (int x = 0; x < 32; ++x) ldiag_matrix = ldiag_matrix && dt.prepend[x] == dt.cost[kGap * 32 + x];
+  if (ldiag_matrix) P->ldiag_costs = lin_diag_costs(dt, align ? 4 : 1);
   // tuned launch shapes (see poyg_ctx_set_tuning)
   // (a per-call pair runs alone: the one-pair-per-wave kernel steps one
   // diagonal pair per lane instead of three, a shorter latency)
@@ -857,40 +879,88 @@ static int plan_pairs_impl(poyg_ctx *ctx, const poyg_cm *cm, int mode, int32_t n
       int64_t c = 0;
       lin_band_extent(m.lr, m.lc, g, maxw, c);
       cells[k] = c;
-      m.stride = lin_dm_stride(maxw);   // room for a row start phase of up to 3 bytes (systolic fill)
-      if (align && !lin_dm_fits(m.lr, maxw)) {
-        delete P;
-        set_error("poyg_plan_pairs: pair %d (%d x %d) has a direction band of %lld bytes, beyond the linear "
-                  "kernels' 32-bit band offsets", k, m.lr, m.lc, (long long)m.lr * m.stride);
-        return POYG_EUNSUPPORTED;
-      }
-      m.aux_off = aux_ints;
-      aux_ints += (2 * (int64_t)m.lc + 63) & ~(int64_t)63;
-      if (align) {
-        m.dm_off = dm_bytes;
-        dm_bytes += (int64_t)m.lr * m.stride;
-      }
-      if (c16_matrix && m.lc >= 2 && m.lc <= kLinStageHost &&
-          ((int64_t)m.lr + m.lc + 2) * std::max<int64_t>(c16_cmax, 1) < 0xfff0) {
-        c16[k] = 1;
-        m.p3 = 1;
-      } else if (m.lc <= kLinStageHost) {
-        sys[k] = 1;
-      } else if (maxw > kLinRBHost) {
-        glb[k] = 1;
-        row_width = std::max(row_width, (m.lc + 1 + 63) & ~63);
+      widest[k] = maxw;
+      if (ldiag_matrix && lin_diag_fits(m.lr, m.lc, g) &&
+          ((int64_t)m.lr + m.lc + 2) * std::max<int64_t>(c16_cmax, 1) * (align ? 4 : 1) < 0xfff0) {
+        int dlo, dhi;
+        lin_diag_range(m.lr, m.lc, g, dlo, dhi);
+        ldiag[k] = 1;
+        const int w = lin_diag_waves(dlo, dhi);
+        diag_waves += w ? w : 1 << 20;
+        diag_multi = diag_multi || w > 1;
       }
     }
     P->cells += cells[k];
+  }
+  // Linear pairs: the diagonal fill, with several waves on a pair where pairs
+  // need more than one register per lane and the batch leaves SIMDs idle (a
+  // wave's step is shortest with one register; past that the wave per pair
+  // wins, which computes no shared diagonals); the strips, the systolic fill or
+  // the row kernels for the pairs it does not take.  Pairs of 1,500-2,000
+  // (2.4 waves each), several waves against one: costs of 256 / 768 / 1,024
+  // pairs 186 / 364 / 442 us against 374 / 382 / 385; alignments of 256 / 512 /
+  // 1,024 pairs 283 / 370 / 398 against 353 / 356 / 361.
+  const bool diag_group = diag_multi && diag_waves <= (align ? 4 : 8) * ctx->cus;
+  int max_waves = 0;
+  for (int k = 0; !affine && k < n; ++k) {
+    PairMeta &m = meta[k];
+    const LinGeom g{m.p0, m.p1, m.p2};
+    if (ldiag[k]) {
+      int dlo, dhi;
+      lin_diag_range(m.lr, m.lc, g, dlo, dhi);
+      const int f = diag_group ? lin_diag_waves(dlo, dhi) : lin_diag_regs(dlo, dhi);
+      ldiag[k] = f > 0;
+      if (f) {
+        m.p0 = dlo;
+        m.p1 = dhi;
+        m.p2 = f;
+        m.p3 = 2;
+        m.stride = lin_diag_cols(diag_group, f);
+        if (align) {
+          m.dm_off = (dm_bytes + 7) & ~(int64_t)7;
+          dm_bytes = m.dm_off + lin_diag_bytes(m.lr, m.lc, dlo, m.stride);
+        }
+        max_waves = std::max(max_waves, f);
+        continue;
+      }
+    }
+    m.stride = lin_dm_stride(widest[k]);   // room for a row start phase of up to 3 bytes (systolic fill)
+    if (align && !lin_dm_fits(m.lr, widest[k])) {
+      delete P;
+      set_error("poyg_plan_pairs: pair %d (%d x %d) has a direction band of %lld bytes, beyond the linear "
+                "kernels' 32-bit band offsets", k, m.lr, m.lc, (long long)m.lr * m.stride);
+      return POYG_EUNSUPPORTED;
+    }
+    m.aux_off = aux_ints;
+    aux_ints += (2 * (int64_t)m.lc + 63) & ~(int64_t)63;
+    if (align) {
+      m.dm_off = dm_bytes;
+      dm_bytes += (int64_t)m.lr * m.stride;
+    }
+    if (c16_matrix && m.lc >= 2 && m.lc <= kLinStageHost &&
+        ((int64_t)m.lr + m.lc + 2) * std::max<int64_t>(c16_cmax, 1) < 0xfff0) {
+      c16[k] = 1;
+      m.p3 = 1;
+    } else if (m.lc <= kLinStageHost) {
+      sys[k] = 1;
+    } else if (widest[k] > kLinRBHost) {
+      glb[k] = 1;
+      row_width = std::max(row_width, (m.lc + 1 + 63) & ~63);
+    }
   }
   P->out_bytes = out_bytes;
   // longest-first work lists
   std::vector<int32_t> order(n);
   std::iota(order.begin(), order.end(), 0);
   std::stable_sort(order.begin(), order.end(), [&](int a, int b) { return cells[a] > cells[b]; });
-  std::vector<int32_t> o_lds, o_glb, o_sys, o_c16, o_quad, o_diag[3], o_rows;
+  std::vector<int32_t> o_lds, o_glb, o_sys, o_c16, o_quad, o_diag[3], o_rows, o_ldiag, o_trace;
   int64_t c_quad3 = 0, c_diag1 = 0;
   for (int k : order) {
+    if (ldiag[k]) {
+      o_ldiag.push_back(k);
+      continue;
+    }
+    if (!affine) o_trace.push_back(k);
     if (quad[k]) {
       o_quad.push_back(k);
       c_quad3 += cells[k];
@@ -932,11 +1002,17 @@ static int plan_pairs_impl(poyg_ctx *ctx, const poyg_cm *cm, int mode, int32_t n
   P->grid_lds = std::max(1, std::min((P->n_lds + 3) / 4, ctx->cus * per_cu));
   P->grid_glb = std::max(1, std::min(P->n_glb, 256));
   if (P->n_sys) P->grid_sys = std::max(1, std::min(P->n_sys, ctx->cus * sys_bpc));
+  P->n_trace = (int)o_trace.size();
+  P->n_ldiag = (int)o_ldiag.size();
+  if (P->n_ldiag) {
+    P->ldiag_waves = diag_group ? max_waves : 0;
+    P->grid_ldiag = diag_group ? P->n_ldiag
+                               : std::max(1, std::min((P->n_ldiag + 3) / 4, ctx->cus * lin_diag_blocks_per_cu(align)));
+  }
   P->n_c16 = (int)o_c16.size();
   if (P->n_c16) {
-    // a batch that one pair per wave leaves far from filling the chip (tree
-    // levels, per-call entries) gets four waves per pair: each pair's
-    // latency is about a third
+    // a batch that one pair per wave leaves far from filling the chip gets
+    // four waves per pair: each pair's latency is about a third
     const int lk = ctx->tune[kTuneLinCost];
     P->c16_mw = lk == 4 || (lk != 3 && P->n_c16 <= 2 * ctx->cus);
     if (P->c16_mw)   // grid_c16 counts workgroups
@@ -1022,7 +1098,7 @@ static int plan_pairs_impl(poyg_ctx *ctx, const poyg_cm *cm, int mode, int32_t n
   std::vector<std::pair<DevBuf *, std::pair<const void *, size_t>>> sections = {
       {&P->tcm, {&dt, sizeof dt}},
       {&P->meta, {meta.data(), sizeof(PairMeta) * (size_t)n}},
-      {&P->order_all, {order.data(), sizeof(int32_t) * (size_t)n}},
+      {&P->order_all, {o_trace.data(), sizeof(int32_t) * o_trace.size()}},
       {&P->order_lds, {o_lds.data(), sizeof(int32_t) * o_lds.size()}},
       {&P->order_glb, {o_glb.data(), sizeof(int32_t) * o_glb.size()}},
       {&P->order_sys, {o_sys.data(), sizeof(int32_t) * o_sys.size()}},
@@ -1031,7 +1107,8 @@ static int plan_pairs_impl(poyg_ctx *ctx, const poyg_cm *cm, int mode, int32_t n
       {&P->order_diag[0], {o_diag[0].data(), sizeof(int32_t) * o_diag[0].size()}},
       {&P->order_diag[1], {o_diag[1].data(), sizeof(int32_t) * o_diag[1].size()}},
       {&P->order_diag[2], {o_diag[2].data(), sizeof(int32_t) * o_diag[2].size()}},
-      {&P->order_rows, {o_rows.data(), sizeof(int32_t) * o_rows.size()}}};
+      {&P->order_rows, {o_rows.data(), sizeof(int32_t) * o_rows.size()}},
+      {&P->order_ldiag, {o_ldiag.data(), sizeof(int32_t) * o_ldiag.size()}}};
   std::vector<size_t> sec_off;
   size_t blob_bytes = 0;
   for (auto &sec : sections) {
@@ -1191,7 +1268,7 @@ extern "C" int poyg_plan_run(poyg_plan *P, const uint8_t *d_seq, int32_t *d_cost
     HIP_TRY(launch_plan_start(ctr, kPlanCounters, (int *)P->status.p, kStatusFlags + P->n,
                               affine && align ? (TraceOut *)P->trout.p : nullptr, d_out, d_out_len, s));
   P->last_stream = s;
-  if (!affine || P->n_lds + P->n_glb)
+  if (affine ? P->n_lds + P->n_glb : P->n_trace)
     HIP_TRY(launch_prep(affine, std::max(1, std::min((P->n + 3) / 4, P->ctx->cus * 8)), meta, P->n, d_seq, tcm,
                         (int *)P->aux.p, s));
   if (affine) {
@@ -1262,6 +1339,10 @@ extern "C" int poyg_plan_run(poyg_plan *P, const uint8_t *d_seq, int32_t *d_cost
                               dm, d_cost, sink, (const uint8_t *)P->pure.p, (const TraceOut *)P->trout.p, ctr + 5,
                               s));
   } else {
+    if (P->n_ldiag)
+      HIP_TRY(launch_lin_diag(align, P->ldiag_waves, P->grid_ldiag, meta, (const int32_t *)P->order_ldiag.p, P->n_ldiag,
+                              ctr + 10, d_seq, tcm, P->ldiag_costs, (uint8_t *)P->dm.p, d_cost, d_out, d_out_len,
+                              (int32_t *)P->status.p, s));
     if (P->n_c16 && P->c16_mw)
       HIP_TRY(launch_lin_c16mw(align, P->grid_c16, meta, (const int32_t *)P->order_c16.p, P->n_c16, ctr + 4, d_seq,
                                tcm, (const int *)P->aux.p, d_cost, (uint8_t *)P->dm.p, P->c16_nmax, s));
@@ -1292,9 +1373,9 @@ extern "C" int poyg_plan_run(poyg_plan *P, const uint8_t *d_seq, int32_t *d_cost
         HIP_TRY(launch_aff_trace(meta, (const int32_t *)P->order_rows.p, P->n_rows, d_seq, tcm,
                                  (const uint8_t *)P->dm.p, d_out, d_out_len, (int32_t *)P->status.p, s));
     }
-    else
-      HIP_TRY(launch_lin_trace(std::max(1, std::min((P->n + 3) / 4, P->ctx->cus * P->trace_bpc)), meta,
-                               (const int32_t *)P->order_all.p, P->n, ctr + 3, d_seq, tcm, (const uint8_t *)P->dm.p,
+    else if (P->n_trace)
+      HIP_TRY(launch_lin_trace(std::max(1, std::min((P->n_trace + 3) / 4, P->ctx->cus * P->trace_bpc)), meta,
+                               (const int32_t *)P->order_all.p, P->n_trace, ctr + 3, d_seq, tcm, (const uint8_t *)P->dm.p,
                                d_out, d_out_len, (int32_t *)P->status.p, s));
   }
   if (P->timing) {
@@ -1379,13 +1460,14 @@ struct HostRun {
 struct OnePair : HostRun {
   int32_t h_cost1 = 0;
   int run(poyg_ctx *ctx, const poyg_cm *cm, int mode, const uint8_t *a, int la, const uint8_t *b, int lb,
-          int dw) {
+          int dw, bool byte_band = false) {
     if (!a || !b || la < 1 || lb < 1) {
       set_error("sequence arguments must be non-empty (leading gap included)");
       return POYG_EINVAL;
     }
     int64_t offa = 0, offb = round16(la);
     PerCallSeqs in{a, b, la, lb, offb};
+    in.byte_band = byte_band;
     int rc = HostRun::run(ctx, cm, mode, 1, in, &offa, &la, &offb, &lb, &dw);
     if (rc) return rc;
     h_cost1 = h_cost[0];
@@ -1496,7 +1578,7 @@ int poyg_algn_direction_matrix(poyg_ctx *ctx, const poyg_cm *cm, const uint8_t *
     return POYG_EINVAL;
   }
   OnePair op;
-  int rc = op.run(ctx, cm, POYG_MODE_LINEAR_ALIGN, s1, l1, s2, l2, deltawh);
+  int rc = op.run(ctx, cm, POYG_MODE_LINEAR_ALIGN, s1, l1, s2, l2, deltawh, true);
   if (rc) return rc;
   poyg_plan *P = op.plan;
   const LinGeom g = lin_geom(l1, l2, deltawh);

@@ -253,3 +253,44 @@ def test_direction_matrix_equals_oracle(ctx, oracle, kernel):
             assert np.array_equal(dm, wdm), (la, lb, np.argwhere(dm != wdm)[:5])
     finally:
         ctx.set_tuning("lin_cost_kernel", -1)
+
+
+@pytest.mark.parametrize("sub,indel,alphabet", [(1, 2, "dna"), (1, 1, "ambig"), (2, 1, "any"), (3, 2, "ambig")])
+def test_diagonal_fill_sizes_equal_strips(ctx, sub, indel, alphabet):
+    """The diagonal fill at the edges of its forms: bands of 256, 448, 512 and
+    640 diagonals (one to four registers or waves a pair) and their neighbours,
+    times of 1 .. 17 (a group is eight, a halo exchange sixteen), windows of 64,
+    equal lengths and swapped pairs, both forms of the launch, costs and
+    alignments; every result equal to the strips'.  Symbols without base bits
+    or the gap alone take the table costs."""
+    from poyd_amd import engine
+    rng = np.random.default_rng(70 + sub)
+    A, B, dws = [], [], []
+    for m, n, dw in ([(k, k, 0) for k in list(range(2, 20)) + [63, 64, 65, 66, 128, 129, 130]] +
+                     [(900, 900 - k, w) for w in (76, 77, 78, 79, 172, 173, 174, 205, 206, 267, 268, 269) for k in (0, 1, 3)] +
+                     [(300, 280, 26), (257, 256, 24), (130, 60, 3), (60, 130, 3), (700, 655, 120), (655, 700, 118)]):
+        a = rand_seq(rng, m - 1, alphabet)
+        b = (mutate(rng, a, 0.2, 0.05) if alphabet == "dna" else a.copy())
+        b = np.concatenate([b, rand_seq(rng, max(n - len(b), 1), alphabet)[1:]])[:n]
+        if len(A) % 3 == 2:
+            b[1 + int(rng.integers(0, max(1, len(b) - 2)))] = GAP
+        A.append(a)
+        B.append(b)
+        dws.append(dw)
+    cm = engine.CostMatrix.of_sub_indel(sub, indel)
+    dws = np.array(dws, np.int32)
+    note(f"diagonal fill sub={sub} indel={indel} alphabet={alphabet}: {len(A)} pairs, alone and 40 times over")
+    for reps in (1, 40):   # several waves per pair, then one
+        for mode in (engine.POYG_MODE_LINEAR_COST, engine.POYG_MODE_LINEAR_ALIGN):
+            got = {}
+            for knob in (-1, 3):
+                ctx.set_tuning("lin_cost_kernel", knob)
+                try:
+                    got[knob] = engine.run_pairs(ctx, cm, mode, batch_of(A * reps), batch_of(B * reps), np.tile(dws, reps))
+                finally:
+                    ctx.set_tuning("lin_cost_kernel", -1)
+            assert np.array_equal(got[-1].cost, got[3].cost), (reps, np.nonzero(got[-1].cost != got[3].cost)[0][:5])
+            if mode == engine.POYG_MODE_LINEAR_ALIGN:
+                for k in range(len(A) * (2 if reps > 1 else 1)):
+                    for slot in range(3):
+                        assert np.array_equal(got[-1].seq(k, slot), got[3].seq(k, slot)), (reps, k, slot)
