@@ -59,7 +59,8 @@ int poyg_ctx_sync(poyg_ctx *ctx);
  * "aff_side_div" (2..64, default 4: the side streams get at most
  * CUs / value compute units), "lin_sys_blocks_per_cu" and
  * "lin_trace_blocks_per_cu" (1..occupancy: resident workgroups per CU of the
- * linear fill and backtrace), "cube_waves_per_cu" (1..64, default 8),
+ * linear fill and backtrace), "cube_waves_per_cu" (1..64, default
+ * 16: resident waves per CU of the three-way fill, whose workgroups have eight),
  * "lin_cost_kernel" (1: the 32-bit systolic linear fill for every pair it
  * takes; 2, the default: the 16-bit fill over the band's diagonals where a
  * pair's costs and band allow it, else the packed 16-bit strips, one wave per

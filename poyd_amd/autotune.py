@@ -28,7 +28,7 @@ KNOBS = {
                ("aff_narrow_kernel", [1])],
     "linear": [("lin_cost_kernel", [3, 4]), ("lin_sys_blocks_per_cu", [1, 2, 3, 4]),
                ("lin_trace_blocks_per_cu", [2, 4, 7])],
-    "cube": [("cube_waves_per_cu", [4, 6, 8, 12, 16])],
+    "cube": [("cube_waves_per_cu", [8, 16, 24])],
 }
 
 

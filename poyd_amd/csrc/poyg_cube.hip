@@ -14,6 +14,7 @@
 
 #include <algorithm>
 #include <numeric>
+#include <type_traits>
 #include <vector>
 
 #include "poyg_internal.h"
@@ -292,26 +293,36 @@ __global__ __launch_bounds__(64) void cube_fill_kernel(const TripleMeta *__restr
 }
 
 // ---------------------------------------------------------------------------
-// Row kernel: lane L owns the R consecutive cells k = L*R .. L*R+R-1 of every
-// row (n3 <= 64*R), so a row is one pass: six candidate moves per cell as
-// ranked keys (value*8 + move index; the minimum key is the reference's
-// first minimum), then the self pass along s3 as one prefix minimum
-// (mm[k] = min(v[k], mm[k-1] + g[k]) equals G3[k] + min_{j<=k}(v[j] - G3[j])
-// with G3 the prefix sums of g; the self move wins exactly where
+// Block kernel: a workgroup of kCubeWaves waves fills one cube, a wave two
+// consecutive rows at a time.  Lane L owns the R consecutive cells k = L*R ..
+// L*R+R-1 of a row (n3 <= 64*R), so a row is one pass: six candidate moves per
+// cell as ranked keys (value*8 + move index; the minimum key is the
+// reference's first minimum), then the self pass along s3 as one prefix
+// minimum (mm[k] = min(v[k], mm[k-1] + g[k]) equals G3[k] + min_{j<=k}(v[j] -
+// G3[j]) with G3 the prefix sums of g; the self move wins exactly where
 // mm[k-1] + g[k] < v[k]).
 //
 // The reference's row pointers lag (see the top of this file): row `out` of
 // plane p >= 1 reads rows out-(n2+p-1) ("upper", or "diagonal" on line 0),
-// out-(n2+p) ("diagonal") and out-(p+1) ("previous").  Every input of row
-// out+1 is therefore complete once row out-1 is stored, so the loads of the
-// next row are issued before the current row is computed, and the
-// "diagonal" row of line r is the "upper" row of line r-1 (line 1 reuses the
-// row of line 0), already in registers.  Rows live in a per-wave ring of
-// n1+n2 rows; T is int16_t when every cell value is provably below 2^15
+// out-(n2+p) ("diagonal") and out-(p+1) ("previous").  So p + 1 consecutive
+// lines of plane p depend on none of each other: the workgroup computes chunks
+// of min(p + 1, 2 kCubeWaves) lines, one barrier a chunk, and from plane
+// kCubeAhead on the inputs of the next chunk are stored before the current one
+// starts and are loaded while it is computed.  Plane 0 (each line reads the
+// one before) is the first wave's.  Rows live in a ring of n1 + n2 + 2
+// kCubeWaves rows per workgroup (a chunk's stores never reach a row another
+// wave still reads); T is int16_t when every cell value is provably below 2^15
 // (checked on the host), else int32_t.
+//
+// Bound by VALU issue (about 25 operations a cell) and, where the longest
+// triples run out, by their chunks.  One wave per triple, row after row, took 1
+// us a row whatever the batch: 1,024 triples of 100-500 took 268 ms, here 67 (for
+// costs that leave the packed kernel's range), 53 in the packed kernel below.
 constexpr int kBig3 = 1 << 28;
 constexpr int kTop3 = 0x7fffffff;
-constexpr int kAhead = 4;   // rows whose inputs are in flight
+constexpr int kCubeWaves = 8;
+constexpr int kCubeLines = 2 * kCubeWaves;   // lines of a full chunk
+constexpr int kCubeAhead = 3 * kCubeLines;   // first plane whose chunks' inputs are three chunks old
 
 __device__ __forceinline__ int c_shr1(int v, int fill) {
   return __builtin_amdgcn_update_dpp(fill, v, 0x138 /* wave_shr:1 */, 0xf, 0xf, false);
@@ -379,12 +390,13 @@ __device__ __forceinline__ void store_codes(uint8_t *p, const uint32_t (&c)[(R +
 // One row.  kKind 0: plane 0, line >= 1 (previous-row moves only); 1: line 0
 // of a plane >= 1 (upper moves only, the upper row being the reference's
 // diagonal pointer there); 2: every other row.  U, D, P: raw values of the
-// upper, diagonal and previous rows; tab: the LDS cost table row of s2[r].
+// upper, diagonal and previous rows; tab: the LDS cost table row of s2[r]; z: the
+// cells' S3 terms.
 // Out: mm (raw values) and the packed move codes.
 template <int R, int kKind>
 __device__ __forceinline__ void cube_row(const int (&U)[R], const int (&D)[R], const int (&P)[R],
-                                         const int (&G3s)[R], const int (&yo)[R], const int4 *tab, int cP3,
-                                         int cP1, int cP2, int (&mm)[R], uint32_t (&codes)[(R + 7) / 8]) {
+                                         const int (&G3s)[R], const int (&yo)[R], const int2 *tab, const int (&z)[R],
+                                         int cP3, int cP1, int cP2, int (&mm)[R], uint32_t (&codes)[(R + 7) / 8]) {
   // cell k-1 of lane 0's first cell does not exist: the fill value makes its
   // moves lose to every real key
   constexpr int kNone = kBig3 >> 3;
@@ -396,16 +408,17 @@ __device__ __forceinline__ void cube_row(const int (&U)[R], const int (&D)[R], c
   int key[R];
 #pragma unroll
   for (int j = 0; j < R; ++j) {
-    const int4 tb = tab[yo[j]];
+    int2 tb = make_int2(0, 0);
+    if (kKind != 1) tb = tab[yo[j]];
     const int ul = j ? U[j - 1] : Ul, dl = j ? D[j - 1] : Dl, pl = j ? P[j - 1] : Pl;
     int k;
     if (kKind == 0) {
       k = min((P[j] << 3) + cP1, (pl << 3) + tb.x);
     } else if (kKind == 1) {
-      k = min((U[j] << 3) + cP3, (ul << 3) + tb.z);
+      k = min((U[j] << 3) + cP3, (ul << 3) + z[j]);
     } else {
       k = min(min((U[j] << 3) + cP3, (P[j] << 3) + cP1), (D[j] << 3) + cP2);
-      k = min(min(k, (ul << 3) + tb.z), min((pl << 3) + tb.x, (dl << 3) + tb.y));
+      k = min(min(k, (ul << 3) + z[j]), min((pl << 3) + tb.x, (dl << 3) + tb.y));
     }
     key[j] = k;
   }
@@ -454,9 +467,9 @@ __device__ __forceinline__ int c_prefix_min_ng(int v) {
 // interleave.  The second row's diagonal row is the first row's upper row.
 template <int R>
 __device__ __forceinline__ void cube_row_pair(const int (&U0)[R], const int (&D0)[R], const int (&P0)[R],
-                                              const int4 *tab0, int cP1a, int cP2a, const int (&U1)[R],
-                                              const int (&P1)[R], const int4 *tab1, int cP1b, int cP2b,
-                                              const int (&G3s)[R], const int (&yo)[R], int cP3,
+                                              const int2 *tab0, int cP1a, int cP2a, const int (&U1)[R],
+                                              const int (&P1)[R], const int2 *tab1, int cP1b, int cP2b,
+                                              const int (&G3s)[R], const int (&yo)[R], const int (&z)[R], int cP3,
                                               int (&mm0)[R], uint32_t (&codes0)[(R + 7) / 8], int (&mm1)[R],
                                               uint32_t (&codes1)[(R + 7) / 8]) {
   constexpr int kNone = kBig3 >> 3;
@@ -466,13 +479,13 @@ __device__ __forceinline__ void cube_row_pair(const int (&U0)[R], const int (&D0
   int key0[R], key1[R];
 #pragma unroll
   for (int j = 0; j < R; ++j) {
-    const int4 ta = tab0[yo[j]], tb = tab1[yo[j]];
+    const int2 ta = tab0[yo[j]], tb = tab1[yo[j]];
     const int ul0 = j ? U0[j - 1] : Ul0, dl0 = j ? D0[j - 1] : Dl0, pl0 = j ? P0[j - 1] : Pl0;
     const int ul1 = j ? U1[j - 1] : Ul1, dl1 = ul0, pl1 = j ? P1[j - 1] : Pl1;
     int k0 = min(min((U0[j] << 3) + cP3, (P0[j] << 3) + cP1a), (D0[j] << 3) + cP2a);
-    k0 = min(min(k0, (ul0 << 3) + ta.z), min((pl0 << 3) + ta.x, (dl0 << 3) + ta.y));
+    k0 = min(min(k0, (ul0 << 3) + z[j]), min((pl0 << 3) + ta.x, (dl0 << 3) + ta.y));
     int k1 = min(min((U1[j] << 3) + cP3, (P1[j] << 3) + cP1b), (U0[j] << 3) + cP2b);
-    k1 = min(min(k1, (ul1 << 3) + tb.z), min((pl1 << 3) + tb.x, (dl1 << 3) + tb.y));
+    k1 = min(min(k1, (ul1 << 3) + z[j]), min((pl1 << 3) + tb.x, (dl1 << 3) + tb.y));
     key0[j] = k0;
     key1[j] = k1;
   }
@@ -506,25 +519,27 @@ __device__ __forceinline__ void cube_row_pair(const int (&U0)[R], const int (&D0
 }
 
 template <typename T, int R>
-__global__ __launch_bounds__(64) void cube_rows_kernel(const TripleMeta *__restrict__ meta,
-                                                       const int32_t *__restrict__ order, int n, int *counter,
-                                                       const uint8_t *__restrict__ seq,
-                                                       const DevTcm3 *__restrict__ tcm, uint8_t *dm_base,
-                                                       T *scratch, int64_t scratch_per_wave,
-                                                       int32_t *cost_out) {
-  // [b][y]: x = cost(gap, b, y)*8 + S1, y = cost(a, b, y)*8 + S2, z = cost(a, gap, y)*8 + S3 for the
-  // plane's s1 symbol a
-  __shared__ int4 s_tab[32 * 32];
+__global__ __launch_bounds__(64 * kCubeWaves) void cube_block_kernel(
+    const TripleMeta *__restrict__ meta, const int32_t *__restrict__ order, int n, int *counter,
+    const uint8_t *__restrict__ seq, const DevTcm3 *__restrict__ tcm, uint8_t *dm_base, T *scratch,
+    int64_t scratch_per_group, int32_t *cost_out) {
+  // [b][y] of the planes of one parity: x = cost(gap, b, y)*8 + S1, y = cost(a, b, y)*8 + S2 for the plane's s1
+  // symbol a; s_z: cost(a, gap, y)*8 + S3
+  __shared__ int2 s_tab[2][32 * 32];
+  __shared__ int s_z[2][32];
+  __shared__ int s_item;
   constexpr int RS = 64 * R;   // ring row stride (elements)
-  const int lane = c_lane();
-  T *ring = scratch + (size_t)blockIdx.x * scratch_per_wave;
+  constexpr int kPer = 1024 / (64 * kCubeWaves);   // table entries per thread
+  const int lane = c_lane(), wv = __builtin_amdgcn_readfirstlane((int)threadIdx.x / 64);
+  T *const ring = scratch + (size_t)blockIdx.x * scratch_per_group;
   const int gap = tcm->gap;
-  for (int e = lane; e < 1024; e += 64) s_tab[e].x = (tcm->cost[gap * 1024 + e] << 3) | kS1;
-  c_lds_sync();
+  for (int e = threadIdx.x; e < 1024; e += 64 * kCubeWaves)
+    s_tab[0][e].x = s_tab[1][e].x = (tcm->cost[gap * 1024 + e] << 3) | kS1;
   for (;;) {
-    int kk = 0;
-    if (lane == 0) kk = atomicAdd(counter, 1);
-    kk = __builtin_amdgcn_readfirstlane(kk);
+    __syncthreads();   // the previous triple is done in every wave
+    if (threadIdx.x == 0) s_item = atomicAdd(counter, 1);
+    __syncthreads();
+    const int kk = __builtin_amdgcn_readfirstlane(s_item);
     if (kk >= n) break;
     const int t = __builtin_amdgcn_readfirstlane(order[kk]);
     const int64_t off1 = c_uniform64(meta[t].off1), off2 = c_uniform64(meta[t].off2),
@@ -539,12 +554,26 @@ __global__ __launch_bounds__(64) void cube_rows_kernel(const TripleMeta *__restr
     else __builtin_amdgcn_s_setprio(0);
     const uint8_t *s1 = seq + off1, *s2 = seq + off2, *s3 = seq + off3;
     uint8_t *dm = dm_base + dm_off;
-    const int W = n1 + n2;
+    const int W = n1 + n2 + kCubeLines;
     const int s30 = __builtin_amdgcn_readfirstlane((int)(s3[0] & 31));
     const bool act = lane * R < n3;   // lane holds at least one cell
+    // the table of plane p (its part of 1,024 entries per thread)
+    int tv[kPer], tz = 0;
+    auto table_load = [&](int p) {
+      const int a = __builtin_amdgcn_readfirstlane((int)(s1[p] & 31));
+#pragma unroll
+      for (int q = 0; q < kPer; ++q) tv[q] = tcm->cost[a * 1024 + q * 64 * kCubeWaves + (int)threadIdx.x];
+      tz = tcm->cost[(a * 32 + gap) * 32 + (lane & 31)];
+    };
+    auto table_store = [&](int p) {
+#pragma unroll
+      for (int q = 0; q < kPer; ++q) s_tab[p & 1][q * 64 * kCubeWaves + (int)threadIdx.x].y = (tv[q] << 3) | kS2;
+      if (threadIdx.x < 32) s_z[p & 1][lane] = (tz << 3) | kS3;
+    };
+    if (n1 > 1) table_load(1);
     // per-cell symbols of s3 (inactive cells: the gap) and prefix sums of
     // cost(gap, gap, s3[k]) for k >= 1
-    int yo[R], G3s[R];
+    int yo[R], G3s[R], z[R];
     {
       int g[R], sum = 0;
 #pragma unroll
@@ -552,9 +581,10 @@ __global__ __launch_bounds__(64) void cube_rows_kernel(const TripleMeta *__restr
         const int k = lane * R + j;
         const int y = k < n3 ? (int)(s3[k] & 31) : gap;
         yo[j] = y;
-        g[j] = (k >= 1 && k < n3) ? (s_tab[gap * 32 + y].x >> 3) : 0;
+        g[j] = (k >= 1 && k < n3) ? (s_tab[0][gap * 32 + y].x >> 3) : 0;
         sum += g[j];
         G3s[j] = sum;
+        z[j] = 0;
       }
       const int ex = c_prefix_sum(sum) - sum;
 #pragma unroll
@@ -562,224 +592,580 @@ __global__ __launch_bounds__(64) void cube_rows_kernel(const TripleMeta *__restr
     }
     int mm[R];
     uint32_t codes[(R + 7) / 8];
-    // plane 0, line 0: the self pass from 0
-#pragma unroll
-    for (int j = 0; j < R; ++j) mm[j] = G3s[j] >> 3;
-#pragma unroll
-    for (int j = 0; j < (R + 7) / 8; ++j) codes[j] = kSS * 0x11111111u;
-    if (lane == 0) codes[0] = (codes[0] & ~0xfu) | kS2;   // the origin's code is never read
-    if (act) {
-      store_ring<T, R>(ring + lane * R, mm);
-      store_codes<R>(dm + lane * (R / 2), codes);
-    }
-    int cur = 0;   // ring row of the row just written
-    // plane 0, lines r >= 1 (the previous row is the one just computed)
-    for (int r = 1; r < n2; ++r) {
-      const int b = s2[r] & 31;
-      const int4 *tab = s_tab + b * 32;
-      const int cP1 = __builtin_amdgcn_readfirstlane(tab[s30].x) - (kS1 - kP1);
-      int P[R];
-#pragma unroll
-      for (int j = 0; j < R; ++j) P[j] = mm[j];
-      cube_row<R, 0>(P, P, P, G3s, yo, tab, 0, cP1, 0, mm, codes);
-      cur = cur + 1 == W ? 0 : cur + 1;
+    // row f (ring row rr) from mm and codes; the last row's last cell is the cost
+    const int total = n1 * n2;
+    auto store_row = [&](int rr, int f) {
       if (act) {
-        store_ring<T, R>(ring + (size_t)cur * RS + lane * R, mm);
-        store_codes<R>(dm + (size_t)r * dstride + lane * (R / 2), codes);
+        store_ring<T, R>(ring + (size_t)rr * RS + lane * R, mm);
+        store_codes<R>(dm + (size_t)f * dstride + lane * (R / 2), codes);
+      }
+      if (f == total - 1) {
+        const int jl = (n3 - 1) % R;
+        int v = 0;
+#pragma unroll
+        for (int j = 0; j < R; ++j) v = j == jl ? mm[j] : v;
+        cost_out[t] = __builtin_amdgcn_readlane(v, (n3 - 1) / R);   // every lane stores the same value
+      }
+    };
+    if (wv == 0) {
+      // plane 0, line 0: the self pass from 0
+#pragma unroll
+      for (int j = 0; j < R; ++j) mm[j] = G3s[j] >> 3;
+#pragma unroll
+      for (int j = 0; j < (R + 7) / 8; ++j) codes[j] = kSS * 0x11111111u;
+      if (lane == 0) codes[0] = (codes[0] & ~0xfu) | kS2;   // the origin's code is never read
+      store_row(0, 0);
+      // lines r >= 1 (the previous row is the one just computed)
+      for (int r = 1; r < n2; ++r) {
+        const int b = __builtin_amdgcn_readfirstlane((int)(s2[r] & 31));
+        const int2 *tab = s_tab[0] + b * 32;
+        const int cP1 = __builtin_amdgcn_readfirstlane(tab[s30].x) - (kS1 - kP1);
+        int P[R];
+#pragma unroll
+        for (int j = 0; j < R; ++j) P[j] = mm[j];
+        cube_row<R, 0>(P, P, P, G3s, yo, tab, z, 0, cP1, 0, mm, codes);
+        store_row(r, r);
       }
     }
-    int last = 0;   // cost: cell n3-1 of the last row
-    {
-      const int jl = (n3 - 1) % R;
-      int v = 0;
-#pragma unroll
-      for (int j = 0; j < R; ++j) v = j == jl ? mm[j] : v;
-      last = __builtin_amdgcn_readlane(v, (n3 - 1) / R);
-    }
-    if (n1 > 1) {
-      // planes p >= 1 as one stream of rows f = p*n2 + r.  The inputs of row
-      // g are loaded kAhead rows early (register slot (g - n2) % kAhead) when
-      // every row they read is stored by then even if two rows are computed
-      // together, i.e. g - (p+1) and g - (n2+p-1) are at most g - kAhead - 2;
-      // other rows (the first planes) load their inputs when they are
-      // computed.  A wave's own stores are seen by its later loads in program
-      // order.
-      RingRow<T, R> xs[kAhead], ps[kAhead];
-      int bs[kAhead];
-      bool pre[kAhead];
-      int U[R], D[R];
-#pragma unroll
-      for (int j = 0; j < R; ++j) U[j] = D[j] = 0;
-#pragma unroll
-      for (int i = 0; i < kAhead; ++i) {
-        xs[i].zero();
-        ps[i].zero();
-        bs[i] = 0;
-        pre[i] = false;
+    if (n1 > 1) table_store(1);
+    __syncthreads();
+    // planes p >= 1.  in: the inputs of the wave's lines r, r + 1 of a chunk
+    // (d: the diagonal row of line r; that of line r + 1 is u0).
+    struct Inputs {
+      RingRow<T, R> d, u0, u1, p0, p1;
+      int b0, b1;
+    } in;
+    in.d.zero();
+    in.u0.zero();
+    in.u1.zero();
+    in.p0.zero();
+    in.p1.zero();
+    in.b0 = in.b1 = 0;
+    // the chunk's first ring row; lines of the wave
+    auto load_inputs = [&](int p, int r, int rr, int lines) {
+      if (lines <= 0) return;
+      auto row = [&](RingRow<T, R> &x, int back) {
+        int i = rr - back;
+        i += i < 0 ? W : 0;
+        i -= i >= W ? W : 0;
+        if (act) x.load(ring + (size_t)i * RS + lane * R);
+      };
+      row(in.u0, n2 + p - 1);
+      if (r >= 1) {
+        row(in.d, n2 + p);
+        row(in.p0, p + 1);
       }
-      const int total = n1 * n2;
-      // row g's ring index and (plane, line), kAhead rows ahead of f
-      int f = n2, p = 1, r = 0, cur_ring = n2;
-      int g = f, gp = 1, gr = 0, g_ring = n2;
-      auto issue = [&](int i) {
-        // loads of row g into slot i when allowed, then advance g
-        pre[i] = false;
-        bs[i] = s2[gr];   // gr < n2 on every call: loaded unconditionally, used kAhead rows later
-        if (g < total && gp >= kAhead + 1 && n2 + gp >= kAhead + 3) {
-          int xi = g_ring - (n2 + gp - 1);
-          xi += xi < 0 ? W : 0;
-          if (act) xs[i].load(ring + (size_t)xi * RS + lane * R);
-          if (gr >= 1) {
-            int pi = g_ring - (gp + 1);
-            pi += pi < 0 ? W : 0;
-            if (act) ps[i].load(ring + (size_t)pi * RS + lane * R);
+      in.b0 = s2[r];
+      if (lines > 1) {
+        row(in.u1, n2 + p - 2);
+        row(in.p1, p);
+        in.b1 = s2[r + 1];
+      }
+    };
+    int rb = n2;         // ring row of the chunk's first line
+    bool ready = false;   // `in` holds the chunk's inputs
+    for (int p = 1; p < n1; ++p) {
+      const int buf = p & 1;
+#pragma unroll
+      for (int j = 0; j < R; ++j) z[j] = s_z[buf][yo[j]];
+      const int cP3 = __builtin_amdgcn_readfirstlane(s_z[buf][s30]) - (kS3 - kP3);
+      if (p + 1 < n1) table_load(p + 1);
+      const int B = min(p + 1, kCubeLines);
+      for (int r0 = 0; r0 < n2; r0 += B) {
+        const int len = min(B, n2 - r0);
+        const int r = r0 + 2 * wv, lines = len - 2 * wv;
+        int rr = rb + 2 * wv;
+        rr -= rr >= W ? W : 0;
+        if (!ready) load_inputs(p, r, rr, lines);
+        Inputs now = in;
+        // the next chunk
+        int np = p, nr0 = r0 + B, nrb = rb + len;
+        nrb -= nrb >= W ? W : 0;
+        if (nr0 >= n2) {
+          np = p + 1;
+          nr0 = 0;
+        }
+        ready = np < n1 && np >= kCubeAhead;
+        if (ready) {
+          const int nlen = min(kCubeLines, n2 - nr0);
+          int nrr = nrb + 2 * wv;
+          nrr -= nrr >= W ? W : 0;
+          load_inputs(np, nr0 + 2 * wv, nrr, nlen - 2 * wv);
+        }
+        if (lines > 0) {
+          const int b0 = __builtin_amdgcn_readfirstlane(now.b0) & 31;
+          const int b1 = __builtin_amdgcn_readfirstlane(now.b1) & 31;
+          const int2 *tab0 = s_tab[buf] + b0 * 32, *tab1 = s_tab[buf] + b1 * 32;
+          const int2 c0 = tab0[s30], c1 = tab1[s30];
+          const int cP1a = __builtin_amdgcn_readfirstlane(c0.x) - (kS1 - kP1);
+          const int cP2a = __builtin_amdgcn_readfirstlane(c0.y) - (kS2 - kP2);
+          const int cP1b = __builtin_amdgcn_readfirstlane(c1.x) - (kS1 - kP1);
+          const int cP2b = __builtin_amdgcn_readfirstlane(c1.y) - (kS2 - kP2);
+          int U0[R], D0[R], P0[R], U1[R], P1[R];
+#pragma unroll
+          for (int j = 0; j < R; ++j) {
+            U0[j] = now.u0.get(j);
+            D0[j] = now.d.get(j);
+            P0[j] = now.p0.get(j);
+            U1[j] = now.u1.get(j);
+            P1[j] = now.p1.get(j);
           }
-          pre[i] = true;
-        }
-        ++g;
-        g_ring = g_ring + 1 == W ? 0 : g_ring + 1;
-        if (++gr == n2) { gr = 0; ++gp; }
-      };
-#pragma unroll
-      for (int i = 0; i < kAhead; ++i) issue(i);
-      int cP3 = 0;
-      // the contents of slot i; true when they hold the row's inputs
-      auto inputs = [&](int i, RingRow<T, R> &xc, RingRow<T, R> &pc, int &b) {
-        xc = xs[i];
-        pc = ps[i];
-        b = bs[i];
-        return pre[i];
-      };
-      auto load_now = [&](int pp, int rr, int rg, RingRow<T, R> &xc, RingRow<T, R> &pc, int &b) {
-        int xi = rg - (n2 + pp - 1);
-        xi += xi < 0 ? W : 0;
-        if (act) xc.load(ring + (size_t)xi * RS + lane * R);
-        if (rr >= 1) {
-          int pi = rg - (pp + 1);
-          pi += pi < 0 ? W : 0;
-          if (act) pc.load(ring + (size_t)pi * RS + lane * R);
-        }
-        b = s2[rr];
-      };
-      auto store_row = [&](int rg, int ff) {
-        if (act) {
-          store_ring<T, R>(ring + (size_t)rg * RS + lane * R, mm);
-          store_codes<R>(dm + (size_t)ff * dstride + lane * (R / 2), codes);
-        }
-      };
-      auto advance = [&]() {
-        ++f;
-        cur_ring = cur_ring + 1 == W ? 0 : cur_ring + 1;
-        if (++r == n2) { r = 0; ++p; }
-      };
-      auto single = [&](int i) {
-        RingRow<T, R> xc, pc;
-        int b;
-        const bool had = inputs(i, xc, pc, b);
-        issue(i);
-        if (!had) {
-          load_now(p, r, cur_ring, xc, pc, b);
-          // complete these loads here, so that the rows computed from
-          // prefetched slots do not wait for the loads just issued
-          __builtin_amdgcn_s_waitcnt(0x0F70);   // vmcnt(0)
-        }
-        b = __builtin_amdgcn_readfirstlane(b) & 31;
-#pragma unroll
-        for (int j = 0; j < R; ++j) {
-          D[j] = U[j];
-          U[j] = xc.get(j);
-        }
-        if (r == 0) {
-          // plane table: cost(a, b, y) and cost(a, gap, y); all loads first
-          const int a = __builtin_amdgcn_readfirstlane((int)(s1[p] & 31));
-          int v[16];
-#pragma unroll
-          for (int q = 0; q < 16; ++q) v[q] = tcm->cost[a * 1024 + q * 64 + lane];
-          const int z = (tcm->cost[(a * 32 + gap) * 32 + (lane & 31)] << 3) | kS3;
-#pragma unroll
-          for (int q = 0; q < 16; ++q) {
-            s_tab[q * 64 + lane].y = (v[q] << 3) | kS2;
-            s_tab[q * 64 + lane].z = z;
-          }
-          c_lds_sync();
-          cP3 = __builtin_amdgcn_readfirstlane(s_tab[gap * 32 + s30].z) - (kS3 - kP3);
-          cube_row<R, 1>(U, U, U, G3s, yo, s_tab + gap * 32, cP3, 0, 0, mm, codes);
-        } else {
-          const int4 *tab = s_tab + b * 32;
-          const int4 c0 = tab[s30];
-          const int cP1 = __builtin_amdgcn_readfirstlane(c0.x) - (kS1 - kP1);
-          const int cP2 = __builtin_amdgcn_readfirstlane(c0.y) - (kS2 - kP2);
-          int P[R];
-#pragma unroll
-          for (int j = 0; j < R; ++j) P[j] = pc.get(j);
-          cube_row<R, 2>(U, D, P, G3s, yo, tab, cP3, cP1, cP2, mm, codes);
-        }
-        store_row(cur_ring, f);
-        advance();
-      };
-      while (f < total) {
-#pragma unroll
-        for (int i = 0; i < kAhead; i += 2) {
-          if (f + 1 < total && r >= 1 && r + 1 < n2) {
-            // rows f and f+1: lines r and r+1 of plane p
-            RingRow<T, R> xa, pa, xb, pb;
-            int ba, bb;
-            const int ring_b = cur_ring + 1 == W ? 0 : cur_ring + 1;
-            const bool ha = inputs(i, xa, pa, ba);
-            const bool hb = inputs(i + 1, xb, pb, bb);
-            issue(i);
-            issue(i + 1);
-            if (!ha) load_now(p, r, cur_ring, xa, pa, ba);
-            if (!hb) load_now(p, r + 1, ring_b, xb, pb, bb);
-            if (!ha || !hb) __builtin_amdgcn_s_waitcnt(0x0F70);   // vmcnt(0)
-            ba = __builtin_amdgcn_readfirstlane(ba) & 31;
-            bb = __builtin_amdgcn_readfirstlane(bb) & 31;
-            int U1[R], P0[R], P1[R];
-#pragma unroll
-            for (int j = 0; j < R; ++j) {
-              D[j] = U[j];
-              U[j] = xa.get(j);
-              P0[j] = pa.get(j);
-              U1[j] = xb.get(j);
-              P1[j] = pb.get(j);
-            }
-            const int4 *tab0 = s_tab + ba * 32, *tab1 = s_tab + bb * 32;
-            const int4 c0 = tab0[s30], c1 = tab1[s30];
-            const int cP1a = __builtin_amdgcn_readfirstlane(c0.x) - (kS1 - kP1);
-            const int cP2a = __builtin_amdgcn_readfirstlane(c0.y) - (kS2 - kP2);
-            const int cP1b = __builtin_amdgcn_readfirstlane(c1.x) - (kS1 - kP1);
-            const int cP2b = __builtin_amdgcn_readfirstlane(c1.y) - (kS2 - kP2);
+          const int f = p * n2 + r;
+          int rr1 = rr + 1;
+          rr1 -= rr1 >= W ? W : 0;
+          if (r >= 1 && lines > 1) {
             int mm1[R];
             uint32_t codes1[(R + 7) / 8];
-            cube_row_pair<R>(U, D, P0, tab0, cP1a, cP2a, U1, P1, tab1, cP1b, cP2b, G3s, yo, cP3, mm, codes, mm1,
+            cube_row_pair<R>(U0, D0, P0, tab0, cP1a, cP2a, U1, P1, tab1, cP1b, cP2b, G3s, yo, z, cP3, mm, codes, mm1,
                              codes1);
-            store_row(cur_ring, f);
-            advance();
+            store_row(rr, f);
 #pragma unroll
-            for (int j = 0; j < R; ++j) {
-              D[j] = U[j];
-              U[j] = U1[j];
-              mm[j] = mm1[j];
-            }
+            for (int j = 0; j < R; ++j) mm[j] = mm1[j];
 #pragma unroll
             for (int q = 0; q < (R + 7) / 8; ++q) codes[q] = codes1[q];
-            store_row(cur_ring, f);
-            advance();
+            store_row(rr1, f + 1);
           } else {
-            if (f < total) single(i);
-            if (f < total) single(i + 1);
+            if (r == 0) cube_row<R, 1>(U0, U0, U0, G3s, yo, tab0, z, cP3, 0, 0, mm, codes);
+            else cube_row<R, 2>(U0, D0, P0, G3s, yo, tab0, z, cP3, cP1a, cP2a, mm, codes);
+            store_row(rr, f);
+            if (lines > 1) {
+              cube_row<R, 2>(U1, U0, P1, G3s, yo, tab1, z, cP3, cP1b, cP2b, mm, codes);
+              store_row(rr1, f + 1);
+            }
           }
         }
+        if (r0 + B >= n2 && p + 1 < n1) table_store(p + 1);   // (its buffer was plane p - 1's)
+        rb = nrb;
+        __syncthreads();
       }
-      const int jl = (n3 - 1) % R;
-      int v = 0;
-#pragma unroll
-      for (int j = 0; j < R; ++j) v = j == jl ? mm[j] : v;
-      last = __builtin_amdgcn_readlane(v, (n3 - 1) / R);
     }
-    // every lane stores the same value (keeps the item loop scalar)
-    cost_out[t] = last;
-    c_wave_fence();
+  }
+}
+
+// ---------------------------------------------------------------------------
+// The block kernel in packed 16-bit halves, for triples whose every cell value
+// stays below kPackMax: a register holds one cell of the wave's two lines (the
+// first in the low half), so that the six candidates, the minima and the
+// prefix minimum serve both.  A line without previous or diagonal rows (line 0
+// of a plane, plane 0) reads kPackNone in their place, whose candidates lose to
+// every real one.  At R = 8 a chunk of two lines takes 307 vector and 117
+// scalar instructions of a wave (VALU in use 55% of the time, with two waves a
+// SIMD; the rows, 175 GB to and from memory for 1,024 triples, are not the
+// bound).  What it took: 66 ms with the same waits as the unpacked kernel (the
+// barrier of every chunk then waited for its stores), 55 with counted waits,
+// 52 with the chunk's loop free of branches and copies.
+// ---------------------------------------------------------------------------
+constexpr int kPackMax = 8000, kPackCost = 64, kPackNone = 8100;   // 8 kPackNone + 8 kPackCost + 7 < 2^16
+typedef short c3s __attribute__((ext_vector_type(2)));
+typedef unsigned short c3u __attribute__((ext_vector_type(2)));
+__device__ __forceinline__ uint32_t p3_min_u(uint32_t a, uint32_t b) {
+  return __builtin_bit_cast(uint32_t, __builtin_elementwise_min(__builtin_bit_cast(c3u, a), __builtin_bit_cast(c3u, b)));
+}
+__device__ __forceinline__ uint32_t p3_min_i(uint32_t a, uint32_t b) {
+  return __builtin_bit_cast(uint32_t, __builtin_elementwise_min(__builtin_bit_cast(c3s, a), __builtin_bit_cast(c3s, b)));
+}
+__device__ __forceinline__ uint32_t p3_add(uint32_t a, uint32_t b) {
+  return __builtin_bit_cast(uint32_t, __builtin_bit_cast(c3u, a) + __builtin_bit_cast(c3u, b));
+}
+__device__ __forceinline__ uint32_t p3_sub(uint32_t a, uint32_t b) {
+  return __builtin_bit_cast(uint32_t, __builtin_bit_cast(c3u, a) - __builtin_bit_cast(c3u, b));
+}
+// per half: 8 v + c (c may be uniform)
+__device__ __forceinline__ uint32_t p3_key(uint32_t v, uint32_t c) {
+  uint32_t r;
+  asm("v_pk_mad_u16 %0, %1, 8, %2 op_sel_hi:[1,0,1]" : "=v"(r) : "v"(v), "v"(c));
+  return r;
+}
+__device__ __forceinline__ uint32_t p3_key_s(uint32_t v, uint32_t c) {
+  uint32_t r;
+  asm("v_pk_mad_u16 %0, %1, 8, %2 op_sel_hi:[1,0,1]" : "=v"(r) : "v"(v), "s"(c));
+  return r;
+}
+// per half: all ones where a < b, signed (written out: the compiler makes two
+// compares and selects of it)
+__device__ __forceinline__ uint32_t p3_lt(uint32_t a, uint32_t b) {
+  uint32_t r;
+  asm("v_pk_sub_i16 %0, %1, %2 clamp" : "=v"(r) : "v"(a), "v"(b));
+  asm("v_pk_ashrrev_i16 %0, 15, %0 op_sel_hi:[0,1]" : "+v"(r));
+  return r;
+}
+__device__ __forceinline__ uint32_t p3_lo(uint32_t first, uint32_t second) {   // low halves
+  return __builtin_amdgcn_perm(second, first, 0x05040100u);
+}
+__device__ __forceinline__ uint32_t p3_hi(uint32_t first, uint32_t second) {
+  return __builtin_amdgcn_perm(second, first, 0x07060302u);
+}
+__device__ __forceinline__ uint32_t p3_prefix_min(uint32_t v) {
+  constexpr int I = 0x7fff7fff;
+  v = p3_min_i(v, (uint32_t)__builtin_amdgcn_update_dpp(I, (int)v, 0x111, 0xf, 0xf, false));
+  v = p3_min_i(v, (uint32_t)__builtin_amdgcn_update_dpp(I, (int)v, 0x112, 0xf, 0xf, false));
+  v = p3_min_i(v, (uint32_t)__builtin_amdgcn_update_dpp(I, (int)v, 0x114, 0xf, 0xf, false));
+  v = p3_min_i(v, (uint32_t)__builtin_amdgcn_update_dpp(I, (int)v, 0x118, 0xf, 0xf, false));
+  v = p3_min_i(v, (uint32_t)__builtin_amdgcn_update_dpp(I, (int)v, 0x142, 0xa, 0xf, false));
+  v = p3_min_i(v, (uint32_t)__builtin_amdgcn_update_dpp(I, (int)v, 0x143, 0xc, 0xf, false));
+  return v;
+}
+
+// Two lines.  U, D, P: their upper, diagonal and previous rows; tab0 / tab1:
+// the table rows of their s2 symbols (S1 term | S2 term << 16); mm: the values;
+// codes[q]: move codes of cells 4q .. 4q + 3 of both lines.
+template <int R>
+__device__ __forceinline__ void cube_lines(const uint32_t (&U)[R], const uint32_t (&D)[R], const uint32_t (&P)[R],
+                                           const uint32_t (&G3)[R], const uint32_t (&z)[R], const int (&yo)[R],
+                                           const uint32_t *tab0, const uint32_t *tab1, uint32_t cP3, uint32_t cP1,
+                                           uint32_t cP2, uint32_t (&mm)[R], uint32_t (&codes)[R / 4]) {
+  constexpr int kNone = kPackNone * 0x00010001;
+  c_dpp_guard();
+  const uint32_t Ul = (uint32_t)c_shr1((int)U[R - 1], kNone), Dl = (uint32_t)c_shr1((int)D[R - 1], kNone),
+                 Pl = (uint32_t)c_shr1((int)P[R - 1], kNone);
+  uint32_t key[R], wv[R], lp[R];
+#pragma unroll
+  for (int j = 0; j < R; ++j) {
+    const uint32_t e0 = *(const uint32_t *)((const char *)tab0 + yo[j]), e1 = *(const uint32_t *)((const char *)tab1 + yo[j]);
+    const uint32_t ul = j ? U[j ? j - 1 : 0] : Ul, dl = j ? D[j ? j - 1 : 0] : Dl, pl = j ? P[j ? j - 1 : 0] : Pl;
+    const uint32_t a = p3_min_u(p3_min_u(p3_key_s(U[j], cP3), p3_key_s(P[j], cP1)), p3_key_s(D[j], cP2));
+    const uint32_t b = p3_min_u(p3_min_u(p3_key(ul, z[j]), p3_key(pl, p3_lo(e0, e1))), p3_key(dl, p3_hi(e0, e1)));
+    key[j] = p3_min_u(a, b);
+  }
+  // self pass along s3
+  uint32_t run = 0x7fff7fffu;
+#pragma unroll
+  for (int j = 0; j < R; ++j) {
+    const c3u v = __builtin_bit_cast(c3u, key[j]) >> (c3u){3, 3};
+    wv[j] = p3_sub(__builtin_bit_cast(uint32_t, v), G3[j]);
+    run = p3_min_i(run, wv[j]);
+    lp[j] = run;
+  }
+  const uint32_t excl = (uint32_t)c_shr1((int)p3_prefix_min(run), 0x7fff7fff);
+  uint32_t prev = excl;
+#pragma unroll
+  for (int j = 0; j < R / 4; ++j) codes[j] = 0;
+#pragma unroll
+  for (int j = 0; j < R; ++j) {
+    const uint32_t pm = p3_min_i(excl, lp[j]);
+    // all ones where the cell before plus the self cost is smaller
+    const uint32_t m = p3_lt(prev, wv[j]);
+    mm[j] = p3_add(G3[j], pm);
+    const uint32_t code = ((m & (kSS * 0x00010001u)) | (~m & key[j])) & 0x00070007u;
+    codes[j >> 2] |= code << (4 * (j & 3));
+    prev = pm;
+  }
+}
+
+// LDS of a workgroup.  tab: [b][y] of the planes of one parity, cost(gap, b,
+// y)*8 + S1 | (cost(a, b, y)*8 + S2) << 16 for the plane's s1 symbol a; z:
+// cost(a, gap, y)*8 + S3.
+struct CubeLds {
+  uint32_t tab[2][32 * 32];
+  uint32_t z[2][32];
+  int item;
+  uint8_t s2[kPackMax];   // (n2 < kPackMax: every cost bound is at least 1)
+};
+constexpr int kCubePer = 1024 / (64 * kCubeWaves);   // table entries per thread
+
+// One triple by the workgroup; tx: the S1 terms of this thread's table entries.
+template <int R>
+__device__ __forceinline__ void cube_packed_triple(int t, const TripleMeta *__restrict__ meta,
+                                                   const uint8_t *__restrict__ seq, const DevTcm3 *__restrict__ tcm,
+                                                   uint8_t *dm_base, uint16_t *const ring, int32_t *cost_out, CubeLds &L,
+                                                   const uint32_t (&tx)[kCubePer], int gap) {
+  constexpr int RS = 64 * R;   // ring row stride (elements)
+  constexpr int kPer = kCubePer;
+  uint32_t(&s_tab)[2][32 * 32] = L.tab;
+  uint32_t(&s_z)[2][32] = L.z;
+  const int lane = c_lane(), wv = __builtin_amdgcn_readfirstlane((int)threadIdx.x / 64);
+  const int64_t off1 = c_uniform64(meta[t].off1), off2 = c_uniform64(meta[t].off2),
+                off3 = c_uniform64(meta[t].off3), dm_off = c_uniform64(meta[t].dm_off);
+  const int n1 = __builtin_amdgcn_readfirstlane(meta[t].l1), n2 = __builtin_amdgcn_readfirstlane(meta[t].l2),
+            n3 = __builtin_amdgcn_readfirstlane(meta[t].l3),
+            dstride = __builtin_amdgcn_readfirstlane(meta[t].dstride);
+  // the triples with the most rows bound the launch: their waves issue first
+  const int prio = (__builtin_amdgcn_readfirstlane(meta[t].flags) >> 1) & 3;
+  if (prio >= 2) __builtin_amdgcn_s_setprio(2);
+  else if (prio == 1) __builtin_amdgcn_s_setprio(1);
+  else __builtin_amdgcn_s_setprio(0);
+  const uint8_t *s1 = seq + off1, *s2 = seq + off2, *s3 = seq + off3;
+  uint8_t *dm = dm_base + dm_off;
+  const int W = n1 + n2 + kCubeLines;
+  const int s30 = __builtin_amdgcn_readfirstlane((int)(s3[0] & 31));
+  const bool act = lane * R < n3;   // lane holds at least one cell
+  int tv[kPer], tz = 0;
+  auto table_load = [&](int p) {
+    const int a = __builtin_amdgcn_readfirstlane((int)(s1[p] & 31));
+#pragma unroll
+    for (int q = 0; q < kPer; ++q) tv[q] = tcm->cost[a * 1024 + q * 64 * kCubeWaves + (int)threadIdx.x];
+    tz = tcm->cost[(a * 32 + gap) * 32 + (lane & 31)];
+  };
+  auto table_store = [&](int p) {
+#pragma unroll
+    for (int q = 0; q < kPer; ++q)
+      s_tab[p & 1][q * 64 * kCubeWaves + (int)threadIdx.x] = tx[q] | ((uint32_t)((tv[q] << 3) | kS2) << 16);
+    if (threadIdx.x < 32) s_z[p & 1][lane] = (uint32_t)((tz << 3) | kS3) & 0xffffu;
+  };
+  for (int k = threadIdx.x; k < n2; k += 64 * kCubeWaves) L.s2[k] = s2[k];   // (read after the next barrier)
+  if (n1 > 1) table_load(1);
+  // byte offsets of the cells' s3 symbols in a table row (inactive cells:
+  // the gap), prefix sums of cost(gap, gap, s3[k]) for k >= 1, S3 terms
+  int yo[R];
+  uint32_t G3[R], z[R];
+  {
+    int g[R], sum = 0;
+#pragma unroll
+    for (int j = 0; j < R; ++j) {
+      const int k = lane * R + j;
+      const int y = k < n3 ? (int)(s3[k] & 31) : gap;
+      yo[j] = 4 * y;
+      sum += (k >= 1 && k < n3) ? (int)((s_tab[0][gap * 32 + y] & 0xffffu) >> 3) : 0;
+      g[j] = sum;
+      z[j] = 0;
+    }
+    const int ex = c_prefix_sum(sum) - sum;
+#pragma unroll
+    for (int j = 0; j < R; ++j) G3[j] = (uint32_t)(g[j] + ex) * 0x00010001u;
+  }
+  constexpr uint32_t kNone2 = kPackNone * 0x00010001u;
+  uint32_t mm[R], codes[R / 4];
+  const int total = n1 * n2;
+  using Low = std::integral_constant<int, 0>;
+  using High = std::integral_constant<int, 1>;
+  // the last cell of a line of mm
+  auto last_cell = [&](auto half) {
+    const int jl = (n3 - 1) % R;
+    int v = 0;
+#pragma unroll
+    for (int j = 0; j < R; ++j) v = j == jl ? (int)((mm[j] >> (16 * decltype(half)::value)) & 0xffffu) : v;
+    return __builtin_amdgcn_readlane(v, (n3 - 1) / R);
+  };
+  // plane 0's line f (the low halves)
+  auto store_line = [&](int f) {
+    uint32_t w[R / 2], c[(R + 7) / 8];
+#pragma unroll
+    for (int i = 0; i < R / 2; ++i) w[i] = p3_lo(mm[2 * i], mm[2 * i + 1]);
+#pragma unroll
+    for (int i = 0; i < (R + 7) / 8; ++i) c[i] = p3_lo(codes[2 * i], 2 * i + 1 < R / 4 ? codes[2 * i + 1 < R / 4 ? 2 * i + 1 : 0] : 0u);
+    if (act) {
+      uint2 *q = (uint2 *)(ring + (size_t)f * RS + lane * R);
+#pragma unroll
+      for (int i = 0; i < R / 4; ++i) q[i] = make_uint2(w[2 * i], w[2 * i + 1]);
+      store_codes<R>(dm + (size_t)f * dstride + lane * (R / 2), c);
+    }
+    if (f == total - 1) cost_out[t] = last_cell(Low{});   // every lane stores the same value
+  };
+  if (wv == 0) {
+    uint32_t none[R];
+    // plane 0, line 0: the self pass from 0
+#pragma unroll
+    for (int j = 0; j < R; ++j) {
+      none[j] = kNone2;
+      mm[j] = G3[j];
+    }
+#pragma unroll
+    for (int j = 0; j < R / 4; ++j) codes[j] = kSS * 0x11111111u;
+    if (lane == 0) codes[0] = (codes[0] & ~0xfu) | kS2;   // the origin's code is never read
+    store_line(0);
+    // lines r >= 1 (the previous row is the one just computed)
+    for (int r = 1; r < n2; ++r) {
+      const int b = __builtin_amdgcn_readfirstlane((int)(s2[r] & 31));
+      const uint32_t *tab = s_tab[0] + b * 32;
+      const uint32_t cP1 = (__builtin_amdgcn_readfirstlane(tab[s30]) & 0xffffu) - (kS1 - kP1);
+      uint32_t P[R];
+#pragma unroll
+      for (int j = 0; j < R; ++j) P[j] = mm[j];
+      cube_lines<R>(none, none, P, G3, z, yo, tab, tab, 0u, cP1, 0u, mm, codes);
+      store_line(r);
+    }
+  }
+  if (n1 > 1) table_store(1);
+  __syncthreads();
+  // Planes p >= 1.  Every chunk of every wave issues the same loads and stores
+  // (lanes and lines it does not have are dropped by their offsets), so that the
+  // waits can count them: with the next chunk's inputs three chunks old (from
+  // plane kCubeAhead on) a wave waits, before its stores, for those of the chunk
+  // before -- all older than the loads just issued -- and the barrier waits for
+  // nothing else.
+  constexpr int kW = R / 2;                  // words of a row per lane
+  constexpr int kRowLoads = R <= 8 ? 1 : 2;   // loads of a row
+  constexpr int kDrop = 0x7ffffff0;
+  const __amdgpu_buffer_rsrc_t rring = __builtin_amdgcn_make_buffer_rsrc(ring, 0, W * RS * 2, 0x00020000);
+  const int vring = act ? lane * R * 2 : kDrop, vcode = act ? lane * (R / 2) : kDrop;
+  // the inputs of the wave's lines r, r + 1 of a chunk (d: the diagonal row of
+  // line r; that of line r + 1 is u0)
+  uint32_t iu0[kW], iu1[kW], id[kW], ip0[kW], ip1[kW];
+  int ib0 = 0, ib1 = 0;
+  auto up = [&](int i) { return i + ((i >> 31) & W); };          // -W .. W - 1 to 0 .. W - 1
+  auto down = [&](int i) { return i >= W ? i - W : i; };          // 0 .. 2 W - 1 to 0 .. W - 1
+  auto load_row = [&](uint32_t (&w)[kW], int row) {
+    typedef uint32_t u2 __attribute__((ext_vector_type(2)));
+    typedef uint32_t u4 __attribute__((ext_vector_type(4)));
+    const int at = row * (RS * 2);
+    if constexpr (R == 4) {
+      const u2 v = __builtin_amdgcn_raw_buffer_load_b64(rring, vring, at, 0);
+      w[0] = v.x;
+      w[1] = v.y;
+    } else {
+      const u4 v = __builtin_amdgcn_raw_buffer_load_b128(rring, vring, at, 0);
+      w[0] = v.x;
+      w[1] = v.y;
+      w[2] = v.z;
+      w[3] = v.w;
+      if constexpr (R == 12) {
+        const u2 x = __builtin_amdgcn_raw_buffer_load_b64(rring, vring + 16, at, 0);
+        w[4] = x.x;
+        w[5] = x.y;
+      } else if constexpr (R == 16) {
+        const u4 x = __builtin_amdgcn_raw_buffer_load_b128(rring, vring + 16, at, 0);
+        w[4] = x.x;
+        w[5] = x.y;
+        w[6] = x.z;
+        w[7] = x.w;
+      }
+    }
+  };
+  auto load_inputs = [&](int p, int r, int rr) {
+    const int u = up(rr - (n2 + p - 1)), q = up(rr - (p + 1));
+    load_row(iu0, u);
+    load_row(id, up(u - 1));
+    load_row(ip0, q);
+    load_row(iu1, down(u + 1));
+    load_row(ip1, down(q + 1));
+    ib0 = L.s2[min(r, n2 - 1)];
+    ib1 = L.s2[min(r + 1, n2 - 1)];
+  };
+  // line kHalf of mm and codes: ring row rr, line r of the plane (dropped: off)
+  auto store_half = [&](auto half, __amdgpu_buffer_rsrc_t rcode, int rr, int r, bool on) {
+    constexpr int kHalf = decltype(half)::value;
+    typedef uint32_t u2 __attribute__((ext_vector_type(2)));
+    typedef uint32_t u4 __attribute__((ext_vector_type(4)));
+    uint32_t w[kW], c[(R + 7) / 8];
+#pragma unroll
+    for (int i = 0; i < kW; ++i) w[i] = kHalf ? p3_hi(mm[2 * i], mm[2 * i + 1]) : p3_lo(mm[2 * i], mm[2 * i + 1]);
+#pragma unroll
+    for (int i = 0; i < (R + 7) / 8; ++i) {
+      const uint32_t second = 2 * i + 1 < R / 4 ? codes[2 * i + 1 < R / 4 ? 2 * i + 1 : 0] : 0u;
+      c[i] = kHalf ? p3_hi(codes[2 * i], second) : p3_lo(codes[2 * i], second);
+    }
+    const int vr = on ? vring : kDrop, vc = on ? vcode : kDrop, at = rr * (RS * 2), ac = r * dstride;
+    if constexpr (R == 4) __builtin_amdgcn_raw_buffer_store_b64(u2{w[0], w[1]}, rring, vr, at, 0);
+    else __builtin_amdgcn_raw_buffer_store_b128(u4{w[0], w[1], w[2], w[3]}, rring, vr, at, 0);
+    if constexpr (R == 12) __builtin_amdgcn_raw_buffer_store_b64(u2{w[4], w[5]}, rring, vr + 16, at, 0);
+    if constexpr (R == 16) __builtin_amdgcn_raw_buffer_store_b128(u4{w[4], w[5], w[6], w[7]}, rring, vr + 16, at, 0);
+    if constexpr (R == 4) {
+      __builtin_amdgcn_raw_buffer_store_b16((uint16_t)c[0], rcode, vc, ac, 0);
+    } else if constexpr (R == 12) {   // (lanes' codes start at multiples of 6 bytes)
+      __builtin_amdgcn_raw_buffer_store_b16((uint16_t)c[0], rcode, vc, ac, 0);
+      __builtin_amdgcn_raw_buffer_store_b16((uint16_t)(c[0] >> 16), rcode, vc + 2, ac, 0);
+      __builtin_amdgcn_raw_buffer_store_b16((uint16_t)c[1], rcode, vc + 4, ac, 0);
+    } else if constexpr (R == 8) {
+      __builtin_amdgcn_raw_buffer_store_b32(c[0], rcode, vc, ac, 0);
+    } else {
+      __builtin_amdgcn_raw_buffer_store_b64(u2{c[0], c[1]}, rcode, vc, ac, 0);
+    }
+  };
+  int rb = n2;   // ring row of the chunk's first line
+  // planes p0 .. p1 - 1; kPrefetch: the first chunk's inputs are on their way,
+  // and each chunk issues the loads of the next one (past the last plane: rows
+  // that nothing reads)
+  auto planes = [&](auto prefetch, int first, int last) {
+    constexpr bool kPrefetch = decltype(prefetch)::value;
+    for (int p = first; p < last; ++p) {
+      const int buf = p & 1;
+#pragma unroll
+      for (int j = 0; j < R; ++j) z[j] = *(const uint32_t *)((const char *)s_z[buf] + yo[j]) * 0x00010001u;
+      const uint32_t cP3 = (__builtin_amdgcn_readfirstlane(s_z[buf][s30]) - (kS3 - kP3)) * 0x00010001u;
+      const int cline = (int)s_tab[buf][(lane & 31) * 32 + s30];   // lane b: the table entry of s2 symbol b and s3[0]
+      if (p + 1 < n1) table_load(p + 1);
+      const __amdgpu_buffer_rsrc_t rcode =
+          __builtin_amdgcn_make_buffer_rsrc(dm + (int64_t)p * n2 * dstride, 0, n2 * dstride, 0x00020000);
+      const int B = kPrefetch ? kCubeLines : min(p + 1, kCubeLines);
+      for (int r0 = 0; r0 < n2; r0 += B) {
+        const int len = min(B, n2 - r0);
+        const int r = r0 + 2 * wv, lines = len - 2 * wv;
+        const int rr = down(rb + 2 * wv);
+        if constexpr (!kPrefetch) load_inputs(p, r, rr);
+        // line 0 has no previous and no diagonal row (a branch here would copy every input)
+        const uint32_t keep = r == 0 ? 0u : 0xffffffffu, none = kNone2 & ~keep;
+        uint32_t U[R], D[R], P[R];
+#pragma unroll
+        for (int i = 0; i < kW; ++i) {
+          const uint32_t d = (id[i] & keep) | none, p0 = (ip0[i] & keep) | none;
+          U[2 * i] = p3_lo(iu0[i], iu1[i]);
+          U[2 * i + 1] = p3_hi(iu0[i], iu1[i]);
+          D[2 * i] = p3_lo(d, iu0[i]);
+          D[2 * i + 1] = p3_hi(d, iu0[i]);
+          P[2 * i] = p3_lo(p0, ip1[i]);
+          P[2 * i + 1] = p3_hi(p0, ip1[i]);
+        }
+        const int b0 = __builtin_amdgcn_readfirstlane(ib0) & 31, b1 = __builtin_amdgcn_readfirstlane(ib1) & 31;
+        const int nrb = down(rb + len);
+        if constexpr (kPrefetch) {
+          __builtin_amdgcn_sched_barrier(0);   // the loads reuse the inputs' registers
+          const bool turn = r0 + B >= n2;
+          load_inputs(turn ? p + 1 : p, (turn ? 0 : r0 + B) + 2 * wv, down(nrb + 2 * wv));
+        }
+        if (lines > 0) {
+          const uint32_t c0 = (uint32_t)__builtin_amdgcn_readlane(cline, b0), c1 = (uint32_t)__builtin_amdgcn_readlane(cline, b1);
+          const uint32_t cP1 = ((c0 & 0xffffu) | (c1 << 16)) - (kS1 - kP1) * 0x00010001u;
+          const uint32_t cP2 = ((c0 >> 16) | (c1 & 0xffff0000u)) - (kS2 - kP2) * 0x00010001u;
+          cube_lines<R>(U, D, P, G3, z, yo, s_tab[buf] + b0 * 32, s_tab[buf] + b1 * 32, cP3, cP1, cP2, mm, codes);
+        }
+        if constexpr (kPrefetch) asm volatile("s_waitcnt vmcnt(%0)" ::"i"(5 * kRowLoads) : "memory");
+        store_half(Low{}, rcode, rr, r, lines > 0);
+        store_half(High{}, rcode, down(rr + 1), r + 1, lines > 1);
+        if (r0 + B >= n2 && p + 1 < n1) table_store(p + 1);   // (its buffer was plane p - 1's)
+        rb = nrb;
+        if constexpr (kPrefetch) asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+        else __syncthreads();
+      }
+    }
+  };
+  planes(std::false_type{}, 1, min(n1, kCubeAhead));
+  if (n1 > kCubeAhead) {
+    load_inputs(kCubeAhead, 2 * wv, down(rb + 2 * wv));
+    planes(std::true_type{}, kCubeAhead, n1);
+    __syncthreads();   // the last stores
+  }
+  if (n1 > 1) {   // the last row is still in its wave's mm
+    const int at = (n2 - 1) % min(n1, kCubeLines);
+    if (wv == at >> 1) {
+      const int c = at & 1 ? last_cell(High{}) : last_cell(Low{});
+      cost_out[t] = c;   // every lane stores the same value
+    }
+  }
+}
+
+// Every triple of the plan whose n3 <= 64 kMaxR in one work list, the largest
+// first: workgroups of different row widths in launches of their own, side by
+// side, left a few wide triples waiting for the narrow launch's workgroups (100
+// ms against 70).  kMaxR 8: two workgroups a compute unit, 16: one.
+template <int kMaxR>
+__global__ __launch_bounds__(64 * kCubeWaves, kMaxR <= 8 ? 4 : 2) void cube_packed_kernel(
+    const TripleMeta *__restrict__ meta, const int32_t *__restrict__ order, int n, int *counter,
+    const uint8_t *__restrict__ seq, const DevTcm3 *__restrict__ tcm, uint8_t *dm_base, uint16_t *scratch,
+    int64_t scratch_per_group, int32_t *cost_out) {
+  __shared__ CubeLds L;
+  uint16_t *const ring = scratch + (size_t)blockIdx.x * scratch_per_group;
+  const int gap = tcm->gap;
+  uint32_t tx[kCubePer];
+#pragma unroll
+  for (int q = 0; q < kCubePer; ++q) {
+    const int e = q * 64 * kCubeWaves + (int)threadIdx.x;
+    tx[q] = (uint32_t)((tcm->cost[gap * 1024 + e] << 3) | kS1) & 0xffffu;
+    L.tab[0][e] = tx[q];   // (plane 0 reads no S2 term that counts)
+  }
+  for (;;) {
+    __syncthreads();   // the previous triple is done in every wave
+    if (threadIdx.x == 0) L.item = atomicAdd(counter, 1);
+    __syncthreads();
+    const int kk = __builtin_amdgcn_readfirstlane(L.item);
+    if (kk >= n) break;
+    const int t = __builtin_amdgcn_readfirstlane(order[kk]);
+    const int c = (__builtin_amdgcn_readfirstlane(meta[t].l3) + 255) >> 8;   // cube_class
+    if (c <= 1) cube_packed_triple<4>(t, meta, seq, tcm, dm_base, ring, cost_out, L, tx, gap);
+    else if (c == 2) cube_packed_triple<8>(t, meta, seq, tcm, dm_base, ring, cost_out, L, tx, gap);
+    if constexpr (kMaxR > 8) {
+      if (c == 3) cube_packed_triple<12>(t, meta, seq, tcm, dm_base, ring, cost_out, L, tx, gap);
+      else if (c == 4) cube_packed_triple<16>(t, meta, seq, tcm, dm_base, ring, cost_out, L, tx, gap);
+    }
   }
 }
 
@@ -863,9 +1249,9 @@ using namespace poyg;
 // Triple plans are kept apart from pair plans; the C ABI shares poyg_plan
 // through a tagged wrapper defined here.
 //
-// Row classes: a triple with n3 <= 64*R (R = 4, 8, 12, 16) runs in the row
+// Row classes: a triple with n3 <= 64*R (R = 4, 8, 12, 16) runs in the block
 // kernel of that R; longer s3 fall back to cube_fill_kernel (64-cell chunks).
-constexpr int kCubeClasses = 5;   // 0: chunked fallback, c >= 1: row kernel with R = 4c
+constexpr int kCubeClasses = 5;   // 0: chunked fallback, c >= 1: block kernel with R = 4c
 struct TriplePlan {
   poyg_ctx *ctx;
   int n;
@@ -877,6 +1263,9 @@ struct TriplePlan {
   int64_t scratch_bytes_per_wave = 0;
   int grid = 1;
   bool narrow = false;   // int16 ring rows
+  bool packed = false;   // ... and the packed kernel: one launch for every row class
+  bool wide = false;     // ... with triples of more than 512 cells a row
+  int group(int k) const { return packed ? std::min(cls[k], 1) : cls[k]; }   // launch of triple k
   std::vector<int> cls;  // row class per triple
   void *d_tcm = nullptr, *d_meta = nullptr, *d_order = nullptr, *d_dm = nullptr, *d_scratch = nullptr,
        *d_ctr = nullptr, *d_status = nullptr;
@@ -899,8 +1288,8 @@ static hipError_t launch_rows(const TriplePlan *P, int ri, const int32_t *ord, i
                               const uint8_t *d_seq, int32_t *d_cost, hipStream_t s) {
   const int grid = std::max(1, std::min(P->grid, nb));
   T *scratch = (T *)((uint8_t *)P->d_scratch + (size_t)ri * P->grid * P->scratch_bytes_per_wave);
-  hipLaunchKernelGGL((cube_rows_kernel<T, R>), dim3(grid), dim3(64), 0, s, (const TripleMeta *)P->d_meta, ord, nb,
-                     ctr, d_seq, (const DevTcm3 *)P->d_tcm, (uint8_t *)P->d_dm, scratch,
+  hipLaunchKernelGGL((cube_block_kernel<T, R>), dim3(grid), dim3(64 * kCubeWaves), 0, s, (const TripleMeta *)P->d_meta, ord, nb, ctr,
+                     d_seq, (const DevTcm3 *)P->d_tcm, (uint8_t *)P->d_dm, scratch,
                      (int64_t)(P->scratch_bytes_per_wave / (int64_t)sizeof(T)), d_cost);
   return hipGetLastError();
 }
@@ -914,6 +1303,16 @@ static hipError_t launch_class(const TriplePlan *P, int c, int ri, const int32_t
     case 3: return launch_rows<T, 12>(P, ri, ord, nb, ctr, d_seq, d_cost, s);
     default: return launch_rows<T, 16>(P, ri, ord, nb, ctr, d_seq, d_cost, s);
   }
+}
+
+static hipError_t launch_packed(const TriplePlan *P, int ri, const int32_t *ord, int nb, int *ctr, const uint8_t *d_seq,
+                                int32_t *d_cost, hipStream_t s) {
+  const int grid = std::max(1, std::min(P->grid, nb));
+  uint16_t *scratch = (uint16_t *)((uint8_t *)P->d_scratch + (size_t)ri * P->grid * P->scratch_bytes_per_wave);
+  auto *k = P->wide ? cube_packed_kernel<16> : cube_packed_kernel<8>;
+  hipLaunchKernelGGL(k, dim3(grid), dim3(64 * kCubeWaves), 0, s, (const TripleMeta *)P->d_meta, ord, nb, ctr, d_seq,
+                     (const DevTcm3 *)P->d_tcm, (uint8_t *)P->d_dm, scratch, P->scratch_bytes_per_wave / 2, d_cost);
+  return hipGetLastError();
 }
 
 extern "C" {
@@ -973,17 +1372,19 @@ int poyg_triple_plan_create(poyg_ctx *ctx, const poyg_cm3 *cm3, int32_t n, const
   // for non-negative costs below 2^15, the ring rows fit int16
   const bool rows_ok = minc >= 0 && max_sum * std::max<int64_t>(maxc, 1) < (int64_t(1) << 24);
   P->narrow = rows_ok && max_sum * maxc < 32767;
+  P->packed = rows_ok && maxc <= kPackCost && max_sum * std::max<int64_t>(maxc, 1) < kPackMax;
   int64_t need = 0;
   for (int k = 0; k < n; ++k) {
     TripleMeta &m = P->meta[k];
     const int c = rows_ok ? cube_class(m.l3) : 0;
     P->cls[k] = c;
+    P->wide = P->wide || c > 2;
     // row kernel: 4-bit codes, rows padded to whole lanes' cells; fallback: bytes
     m.dstride = c ? (m.l3 + 4 * c - 1) / (4 * c) * (2 * c) : m.l3;
     m.flags = c ? 1 : 0;
     dmb[k] = (int64_t)m.l1 * m.l2 * m.dstride;
     const int64_t w = (int64_t)m.l1 + m.l2;
-    const int64_t bytes = c ? w * 64 * 4 * c * (P->narrow ? 2 : 4)
+    const int64_t bytes = c ? (w + kCubeLines) * 64 * 4 * c * (P->narrow ? 2 : 4)
                             : 4 * (w * m.l3 + m.l3 + 64);
     need = std::max(need, bytes);
   }
@@ -1001,7 +1402,7 @@ int poyg_triple_plan_create(poyg_ctx *ctx, const poyg_cm3 *cm3, int32_t n, const
   P->order.resize(n);
   std::iota(P->order.begin(), P->order.end(), 0);
   std::stable_sort(P->order.begin(), P->order.end(), [&](int a, int b) {
-    return P->cls[a] != P->cls[b] ? P->cls[a] > P->cls[b] : cells[a] > cells[b];
+    return P->group(a) != P->group(b) ? P->group(a) > P->group(b) : cells[a] > cells[b];
   });
   // split into batches whose direction cubes fit the budget
   int64_t cur = 0;
@@ -1019,8 +1420,10 @@ int poyg_triple_plan_create(poyg_ctx *ctx, const poyg_cm3 *cm3, int32_t n, const
   }
   if (n) P->batches.push_back({begin, n});
   const char *wv = getenv("POYG_CUBE_WAVES_PER_CU");
-  const int waves = waves_per_cu > 0 ? waves_per_cu : (wv ? std::max(1, atoi(wv)) : 8);
-  P->grid = std::max(1, std::min(n, cus * waves));
+  const int waves = waves_per_cu > 0 ? waves_per_cu : (wv ? std::max(1, atoi(wv)) : 16);
+  // workgroups of the block kernel (the chunked fallback: waves)
+  P->grid = std::max(1, std::min(n, cus * std::max(1, P->packed && P->wide ? std::min(1, waves / kCubeWaves)
+                                                                           : waves / kCubeWaves)));
   hipError_t e = hipSuccess;
   auto A = [&](void **p, size_t b) { if (e == hipSuccess) e = hipMalloc(p, b ? b : 16); };
   A(&P->d_tcm, sizeof(DevTcm3));
@@ -1031,7 +1434,7 @@ int poyg_triple_plan_create(poyg_ctx *ctx, const poyg_cm3 *cm3, int32_t n, const
   int n_cls = 0;
   {
     bool seen[kCubeClasses] = {};
-    for (int k = 0; k < n; ++k) seen[P->cls[k]] = true;
+    for (int k = 0; k < n; ++k) seen[P->group(k)] = true;
     for (bool x : seen) n_cls += x;
   }
   A(&P->d_scratch, (size_t)P->scratch_bytes_per_wave * P->grid * std::max(1, n_cls));
@@ -1085,7 +1488,7 @@ int poyg_triple_plan_run(void *pp, const uint8_t *d_seq, int32_t *d_cost, uint8_
     std::vector<std::pair<int, int>> runs;
     for (int q = b.first; q < b.second;) {
       int q2 = q;
-      while (q2 < b.second && P->cls[P->order[q2]] == P->cls[P->order[q]]) ++q2;
+      while (q2 < b.second && P->group(P->order[q2]) == P->group(P->order[q])) ++q2;
       runs.push_back({q, q2});
       q = q2;
     }
@@ -1113,6 +1516,8 @@ int poyg_triple_plan_run(void *pp, const uint8_t *d_seq, int32_t *d_cost, uint8_
                            (int *)P->d_scratch + (size_t)ri * P->grid * (P->scratch_bytes_per_wave / 4),
                            P->scratch_bytes_per_wave / 4, d_cost);
         HIP_TRY3(hipGetLastError());
+      } else if (P->packed) {
+        HIP_TRY3(launch_packed(P, (int)ri, o2, q2 - q, ctr, d_seq, d_cost, ls));
       } else if (P->narrow) {
         HIP_TRY3(launch_class<int16_t>(P, c, ri, o2, q2 - q, ctr, d_seq, d_cost, ls));
       } else {

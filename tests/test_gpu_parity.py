@@ -413,6 +413,22 @@ def test_three_d_row_classes(ctx, oracle):
     check_triples(ctx, oracle, 1, 2, shaped_triples(rng, CUBE_SHAPES))
 
 
+# planes around the chunks' sizes (a plane p computes min(p + 1, 16) lines at a
+# time; from plane 48 on the next chunk's inputs are loaded ahead), lines around
+# multiples of 16, every row width
+CHUNK_SHAPES = [(n1, n2, n3) for n1, n3 in ((15, 40), (17, 260), (47, 30), (48, 257), (49, 520), (50, 70), (66, 20))
+                for n2 in (1, 2, 15, 16, 17, 33)] + [(97, 31, 300), (52, 32, 790), (49, 34, 512), (80, 70, 60),
+                                                     (50, 16, 1000), (49, 47, 513), (60, 48, 256)]
+
+
+@pytest.mark.parametrize("sub,indel", [(1, 2), (20, 30)])
+def test_three_d_chunks(ctx, oracle, sub, indel):
+    """The block kernels, packed (costs 1, 2) and not (20, 30)."""
+    note(f"three-dimensional chunks, costs {sub} {indel}")
+    rng = np.random.default_rng(33)
+    check_triples(ctx, oracle, sub, indel, shaped_triples(rng, CHUNK_SHAPES if indel == 2 else CHUNK_SHAPES[::3]))
+
+
 def test_three_d_wide_costs(ctx, oracle):
     note("three-dimensional row classes, int32 rows (costs past 2^15)")
     rng = np.random.default_rng(32)
