@@ -1707,75 +1707,93 @@ int poyg_algn_align_3d(poyg_ctx *ctx, const poyg_cm3 *cm3, const uint8_t *s1, in
 extern "C++" {
 namespace poyg {
 void uk_model(int mm, int go, int ge, UkModel *M);
-hipError_t launch_ukk_geom(const UkRange &r, int ge, int c0, int c1, UkLevel *lev, UkWalk *w, int reset,
-                           hipStream_t s);
-hipError_t launch_ukk_level(const UkModel *M, const UkRange &r, int c, int64_t diags, const UkLevel *lev, uint32_t *U,
-                            const char *A, const char *B, const char *C, int target_state, int target_dist,
-                            UkWalk *w, hipStream_t s);
-hipError_t launch_ukk_esweep(const UkModel *M, const UkRange &r, int c, int final_cost, int64_t diags,
+hipError_t launch_ukk_level(const UkModel &M, const UkJob *jobs, int n, int t, int64_t diags, const UkLevel *lev,
+                            int stride, uint32_t *U, const char *A, const char *B, const char *C, UkWalk *w, hipStream_t s);
+hipError_t launch_ukk_esweep(const UkModel &M, const UkJob *jobs, int t, int final_cost, int64_t diags,
                              const UkLevel *lev, const uint32_t *U, int *E, int64_t ring_words, int ring_n, int half,
                              UkWalk *w, hipStream_t s);
-hipError_t launch_ukk_walk(const UkModel *M, const UkRange &r, int cpcost, int cpw, const UkLevel *lev,
-                           const uint32_t *U, int first_pass, UkWalk *w, hipStream_t s);
-hipError_t launch_ukk_trace(const UkModel *M, const UkRange &r, const UkLevel *lev, const uint32_t *U, const char *A,
-                            const char *B, const char *C, char *cols, int cap, UkWalk *w, hipStream_t s);
+hipError_t launch_ukk_walk(const UkModel *M, const UkJob *jobs, int n, int cpw, const UkLevel *lev, int stride,
+                           const uint32_t *U, const char *A, const char *B, const char *C, char *cols, int first_pass, UkWalk *w,
+                           hipStream_t s);
 }  // namespace poyg
 }
 
 namespace {
 
-// The level store of one search range on the device: the level boxes
-// (computed on the device by ukk_geom_kernel, mirrored here to size the
-// store) and 16 words per diagonal and level.
+// The level store of a batch of ranges on the device (16 words per diagonal
+// and level), its descriptors (jobs, levels, walk records) and their host
+// copies.
 struct UkStore {
-  DevBuf lev, U;
-  size_t lev_cap = 0, u_words = 0;
-  std::vector<UkLevel> box;   // host mirror of the current range's boxes
+  DevBuf desc, U;
+  size_t desc_bytes = 0, u_words = 0;
+  std::vector<UkJob> job;
+  std::vector<UkLevel> box;    // job i's levels from i * stride
+  std::vector<UkWalk> walk;
+  std::vector<uint8_t> image;  // walk records, jobs and levels as sent
+  int stride = 0;
+  // one buffer: the walk records, the jobs, the levels
+  size_t job_off() const { return round16((int64_t)(job.size() * sizeof(UkWalk))); }
+  size_t lev_off() const { return job_off() + round16((int64_t)(job.size() * sizeof(UkJob))); }
+  size_t bytes() const { return lev_off() + box.size() * sizeof(UkLevel); }
+  UkWalk *walks() const { return (UkWalk *)desc.p; }
+  const UkJob *jobs() const { return (const UkJob *)((const uint8_t *)desc.p + job_off()); }
+  const UkLevel *levels() const { return (const UkLevel *)((const uint8_t *)desc.p + lev_off()); }
   void release() {
-    lev.release();
+    desc.release();
     U.release();
-    lev_cap = u_words = 0;
+    desc_bytes = u_words = 0;
   }
 };
 
 constexpr int64_t kUkStoreLimit = int64_t(24) << 30;   // bytes of cost levels one call may hold
+constexpr size_t kUkBatch = 16384;                     // ranges of one batch
 
-// Boxes of levels [c0, c1] of range r appended to the host mirror; returns
-// the store's words after level c1.
-int64_t uk_boxes(std::vector<UkLevel> &box, const UkRange &r, int ge, int c0, int c1) {
-  int64_t base = 0;
-  if (c0 > r.scost) base = box[c0 - 1 - r.scost].base + (int64_t)box[c0 - 1 - r.scost].nab * box[c0 - 1 - r.scost].nac * kUkStates;
-  box.resize((size_t)(c1 - r.scost + 1));
+// Appends levels [c0, c1] of range r to the boxes, the first word at `base`;
+// returns the word after level c1.
+int64_t uk_boxes(std::vector<UkLevel> &box, const UkRange &r, int ge, int c0, int c1, int64_t base) {
   for (int c = c0; c <= c1; ++c) {
-    box[c - r.scost] = uk_level_box(r, ge, c, base);
-    base += (int64_t)box[c - r.scost].nab * box[c - r.scost].nac * kUkStates;
+    box.push_back(uk_level_box(r, ge, c, base));
+    base += (int64_t)box.back().nab * box.back().nac * kUkStates;
   }
   return base;
 }
 
-// Room for `words` level words (keep: copy what the store holds).
-int uk_reserve(UkStore &st, size_t levels, int64_t words, bool keep, hipStream_t s) {
-  if (words * 4 > kUkStoreLimit) {
-    set_error("powell_3d: the search needs %lld bytes of cost levels, above the %lld-byte limit", (long long)words * 4,
-              (long long)kUkStoreLimit);
+// Words of levels [scost, c1] of range r.
+int64_t uk_words(const UkRange &r, int ge, int c1) {
+  int64_t n = 0;
+  for (int c = r.scost; c <= c1; ++c) {
+    const UkLevel L = uk_level_box(r, ge, c, 0);
+    n += (int64_t)L.nab * L.nac * kUkStates;
+  }
+  return n;
+}
+
+// Room for the batch's descriptors and for `words` level words (the pad
+// included; keep: copy the words the store holds).
+int uk_reserve(UkStore &st, int64_t words, bool keep, hipStream_t s) {
+  if ((words - kUkPad) * 4 > kUkStoreLimit) {
+    set_error("powell_3d: the search needs %lld bytes of cost levels, above the %lld-byte limit",
+              (long long)(words - kUkPad) * 4, (long long)kUkStoreLimit);
     return POYG_ENOMEM;
   }
-  if (levels > st.lev_cap) {
-    DevBuf nl;
-    const size_t cap = std::max(levels, 2 * st.lev_cap);
-    if (nl.alloc(cap * sizeof(UkLevel))) return POYG_ENOMEM;
-    if (keep && st.lev_cap && hipMemcpyAsync(nl.p, st.lev.p, st.lev_cap * sizeof(UkLevel), hipMemcpyDeviceToDevice, s) != hipSuccess)
-      return POYG_EDEVICE;
-    st.lev.release();
-    st.lev = nl;
-    st.lev_cap = cap;
+  if (st.bytes() > st.desc_bytes) {
+    const size_t cap = std::max(st.bytes(), 2 * st.desc_bytes);
+    st.desc.release();
+    st.desc_bytes = 0;
+    if (st.desc.alloc(cap)) return POYG_ENOMEM;
+    st.desc_bytes = cap;
   }
   if ((size_t)words > st.u_words) {
     DevBuf nu;
     const size_t cap = std::max((size_t)words, 2 * st.u_words);
     if (nu.alloc(cap * 4)) return POYG_ENOMEM;
-    if (keep && st.u_words && hipMemcpyAsync(nu.p, st.U.p, st.u_words * 4, hipMemcpyDeviceToDevice, s) != hipSuccess)
+    const hipError_t e = keep && st.u_words
+                             ? hipMemcpyAsync(nu.p, st.U.p, st.u_words * 4, hipMemcpyDeviceToDevice, s)
+                             : hipMemsetAsync(nu.p, 0, kUkPad * 4, s);
+    if (e != hipSuccess) {
+      nu.release();
       return POYG_EDEVICE;
+    }
     st.U.release();
     st.U = nu;
     st.u_words = cap;
@@ -1783,17 +1801,27 @@ int uk_reserve(UkStore &st, size_t levels, int64_t words, bool keep, hipStream_t
   return POYG_OK;
 }
 
+// A range of the recursion, in the order of the alignment's columns from the
+// last to the first; once traced, its columns.
+struct UkNode {
+  UkRange r;
+  bool traced = false;
+  int col0 = 0, ncols = 0;
+};
+
 }  // namespace
 
 // The check-point Ukkonen search of powell_3D_align (doUkk,
 // src/ukk.checkp.c:113-214): the first pass over costs 1, 2, ... on the
 // device in chunks of levels until the end diagonal's best state reaches
 // |A|; the check-point cost from the evaluated cells (ukk_esweep_kernel);
-// then doUkkInLimits ranges (src/ukk.checkp.c:216-322) from a stack in the
-// reference's order (a split range's later half first), each its levels,
-// then its traceback (base case, at most CPwidth costs) or its split; the
-// columns come back in reverse and go out after the common prefix
-// (printTraceBack, src/ukk.checkp.c:456-500).
+// then doUkkInLimits ranges (src/ukk.checkp.c:216-322), each its levels,
+// then its traceback (base case, at most CPwidth costs) or its split.  The
+// reference takes the ranges one by one, a split range's later half first;
+// they do not depend on each other, so all ranges of a depth of the recursion
+// are one batch, which shares the launches of their levels, and the reference's
+// order is that of the list.  The columns come back in reverse and go out after the
+// common prefix (printTraceBack, src/ukk.checkp.c:456-500).
 int poyg_powell_3d(poyg_ctx *ctx, const uint8_t *a, int la, const uint8_t *b, int lb, const uint8_t *c, int lc,
                    int mm, int go, int ge, uint8_t *ra, uint8_t *rb, uint8_t *rc, int cap, int *rlen, int *cost) {
   if (!ctx || !a || !b || !c || !ra || !rb || !rc || la < 1 || lb < 1 || lc < 1) return POYG_EINVAL;
@@ -1841,16 +1869,16 @@ int poyg_powell_3d(poyg_ctx *ctx, const uint8_t *a, int la, const uint8_t *b, in
   const int cost_bound = (LA + LB + LC + 1) * (M.max_step + 2 * mm) + 8;
 
   hipStream_t s = ctx->stream;
-  DevBuf dx[3], dM, dW, dCols, dE;
+  DevBuf dx[3], dM, dCols, dE;
   UkStore st;
   auto cleanup = [&]() {
     for (auto &d : dx) d.release();
-    dM.release(); dW.release(); dCols.release(); dE.release();
+    dM.release(); dCols.release(); dE.release();
     st.release();
   };
   for (int q = 0; q < 3; ++q)
     if (dx[q].alloc(x[q].size())) { cleanup(); return POYG_ENOMEM; }
-  if (dM.alloc(sizeof(UkModel)) || dW.alloc(sizeof(UkWalk)) || dCols.alloc((size_t)3 * col_cap)) {
+  if (dM.alloc(sizeof(UkModel)) || dCols.alloc((size_t)3 * col_cap)) {
     cleanup();
     return POYG_ENOMEM;
   }
@@ -1860,8 +1888,6 @@ int poyg_powell_3d(poyg_ctx *ctx, const uint8_t *a, int la, const uint8_t *b, in
   if (e == hipSuccess) e = hipMemcpyAsync(dM.p, &M, sizeof M, hipMemcpyHostToDevice, s);
   const char *A = (const char *)dx[0].p, *B = (const char *)dx[1].p, *C = (const char *)dx[2].p;
   const UkModel *dm = (const UkModel *)dM.p;
-  UkWalk *dw = (UkWalk *)dW.p;
-  UkWalk hw;
   int rc_ = POYG_OK;
   auto fail = [&](int code, const char *what) {
     if (code == POYG_EDEVICE) set_error("powell_3d: %s: %s", what, hipGetErrorString(e));
@@ -1869,29 +1895,44 @@ int poyg_powell_3d(poyg_ctx *ctx, const uint8_t *a, int la, const uint8_t *b, in
     rc_ = code;
     return code;
   };
-  auto read_walk = [&]() -> bool {
-    if (e == hipSuccess) e = hipMemcpyAsync(&hw, dw, sizeof hw, hipMemcpyDeviceToHost, s);
+  // the batch's descriptors to the device (in one copy), its walk records back
+  auto send = [&](bool fresh) {
+    if (fresh) st.walk.assign(st.job.size(), UkWalk{INT_MAX, INT_MAX, 0, 0, -1, 0, 0, -1, 0, 0});
+    st.image.resize(st.bytes());
+    memcpy(st.image.data(), st.walk.data(), st.walk.size() * sizeof(UkWalk));
+    memcpy(st.image.data() + st.job_off(), st.job.data(), st.job.size() * sizeof(UkJob));
+    memcpy(st.image.data() + st.lev_off(), st.box.data(), st.box.size() * sizeof(UkLevel));
+    if (e == hipSuccess) e = hipMemcpyAsync(st.desc.p, st.image.data(), st.image.size(), hipMemcpyHostToDevice, s);
+  };
+  auto read_walks = [&]() -> bool {
+    if (e == hipSuccess)
+      e = hipMemcpyAsync(st.walk.data(), st.desc.p, st.walk.size() * sizeof(UkWalk), hipMemcpyDeviceToHost, s);
     if (e == hipSuccess) e = hipStreamSynchronize(s);
     return e == hipSuccess;
+  };
+  auto level = [&](int t, int64_t diags) {
+    if (e == hipSuccess)
+      e = launch_ukk_level(M, st.jobs(), (int)st.job.size(), t, diags, st.levels(), st.stride, (uint32_t *)st.U.p, A,
+                           B, C, st.walks(), s);
   };
   // ---- first pass: levels 0, 1, ... until the end's best state reaches |A|
   UkRange r0{0, 0, 0, 0, start, LA - LB, LA - LC, 0, 0, LA, LA, LB, LC};
   int final_cost = -1;
   {
     const int chunk = 32;
-    st.box.clear();
+    int64_t words = kUkPad;
     for (int c0 = 0; e == hipSuccess && final_cost < 0; c0 += chunk) {
       if (c0 > cost_bound) { cleanup(); return fail(POYG_EBAND, "the first pass did not reach the end"); }
       const int c1 = c0 + chunk - 1;
-      const int64_t words = uk_boxes(st.box, r0, ge, c0, c1);
-      const int rr = uk_reserve(st, (size_t)(c1 + 1), words, true, s);
+      words = uk_boxes(st.box, r0, ge, c0, c1, words);
+      st.job.assign(1, UkJob{r0, c1 + 1, -1, 0, 0, 0, 0});
+      st.stride = c1 + 1;
+      const int rr = uk_reserve(st, words, true, s);
       if (rr) { cleanup(); return rr; }
-      if (e == hipSuccess) e = launch_ukk_geom(r0, ge, c0, c1, (UkLevel *)st.lev.p, dw, c0 == 0 ? 1 : -1, s);
-      for (int cc = c0; cc <= c1 && e == hipSuccess; ++cc)
-        e = launch_ukk_level(dm, r0, cc, (int64_t)st.box[cc].nab * st.box[cc].nac, (const UkLevel *)st.lev.p,
-                             (uint32_t *)st.U.p, A, B, C, -1, LA, dw, s);
-      if (!read_walk()) break;
-      if (hw.reached <= c1) final_cost = hw.reached;
+      send(c0 == 0);
+      for (int cc = c0; cc <= c1; ++cc) level(cc, (int64_t)st.box[cc].nab * st.box[cc].nac);
+      if (!read_walks()) break;
+      if (st.walk[0].reached <= c1) final_cost = st.walk[0].reached;
     }
   }
   if (e != hipSuccess) { cleanup(); return fail(POYG_EDEVICE, "first pass"); }
@@ -1902,65 +1943,107 @@ int poyg_powell_3d(poyg_ctx *ctx, const uint8_t *a, int la, const uint8_t *b, in
     const int64_t ring_words = (int64_t)st.box[final_cost].nab * st.box[final_cost].nac * kUkStates;
     if (dE.alloc((size_t)(ring_words * ring_n * 4))) { cleanup(); return POYG_ENOMEM; }
     for (int cc = final_cost; cc >= 0 && e == hipSuccess; --cc)
-      e = launch_ukk_esweep(dm, r0, cc, final_cost, (int64_t)st.box[cc].nab * st.box[cc].nac,
-                            (const UkLevel *)st.lev.p, (const uint32_t *)st.U.p, (int *)dE.p, ring_words, ring_n,
-                            LA / 2, dw, s);
+      e = launch_ukk_esweep(M, st.jobs(), cc, final_cost, (int64_t)st.box[cc].nab * st.box[cc].nac, st.levels(),
+                            (const uint32_t *)st.U.p, (int *)dE.p, ring_words, ring_n, LA / 2, st.walks(), s);
     if (e == hipSuccess)
-      e = launch_ukk_walk(dm, r0, 0, cpw, (const UkLevel *)st.lev.p, (const uint32_t *)st.U.p, 1, dw, s);
-    if (!read_walk()) { cleanup(); return fail(POYG_EDEVICE, "check-point walk"); }
+      e = launch_ukk_walk(dm, st.jobs(), 1, cpw, st.levels(), st.stride, (const uint32_t *)st.U.p, A, B, C,
+                          (char *)dCols.p, 1, st.walks(), s);
+    if (!read_walks()) { cleanup(); return fail(POYG_EDEVICE, "check-point walk"); }
     dE.release();
-    if (hw.error) { cleanup(); return fail(POYG_EBAND, "the first pass's walk found no end state"); }
+    if (st.walk[0].error) { cleanup(); return fail(POYG_EBAND, "the first pass's walk found no end state"); }
   }
   // ---- doUkkInLimits ranges, later halves first
-  std::vector<UkRange> stack;
-  r0.fstate = hw.fstate;
-  if (hw.f_cost < 0) {
-    stack.push_back(r0);   // checked too late: the whole range again
-  } else {
-    const UkRange first{0, 0, 0, 0, start, hw.f_ab, hw.f_ac, hw.f_cost, hw.f_state, hw.f_dist, hw.f_dist,
-                        hw.f_dist - hw.f_ab, hw.f_dist - hw.f_ac};
-    const UkRange later{hw.f_ab, hw.f_ac, hw.f_cost, hw.f_state, hw.f_dist, r0.fab, r0.fac, final_cost, r0.fstate,
-                        LA, LA, LB, LC};
-    stack.push_back(first);
-    stack.push_back(later);
-  }
+  std::vector<UkNode> nodes, next;
+  auto split = [&](std::vector<UkNode> &to, const UkRange &r, const UkWalk &w, int fcost) {
+    const UkRange later{w.f_ab, w.f_ac, w.f_cost, w.f_state, w.f_dist, r.fab, r.fac, fcost, r.fstate, r.fdist,
+                        r.endA, r.endB, r.endC};
+    const UkRange first{r.sab, r.sac, r.scost, r.sstate, r.sdist, w.f_ab, w.f_ac, w.f_cost, w.f_state, w.f_dist,
+                        w.f_dist, w.f_dist - w.f_ab, w.f_dist - w.f_ac};
+    to.push_back(UkNode{later});
+    to.push_back(UkNode{first});
+  };
+  r0.fstate = st.walk[0].fstate;
+  if (st.walk[0].f_cost < 0) nodes.push_back(UkNode{r0});   // checked too late: the whole range again
+  else split(nodes, r0, st.walk[0], final_cost);
   size_t ranges = 0;
-  while (!stack.empty() && e == hipSuccess) {
-    const UkRange r = stack.back();
-    stack.pop_back();
-    if (++ranges > (size_t)8 * col_cap + 64) { cleanup(); return fail(POYG_EBAND, "the check-point recursion did not close"); }
-    st.box.clear();
-    const int64_t words = uk_boxes(st.box, r, ge, r.scost, r.fcost);
-    const int rr = uk_reserve(st, (size_t)(r.fcost - r.scost + 1), words, false, s);
-    if (rr) { cleanup(); return rr; }
-    e = launch_ukk_geom(r, ge, r.scost, r.fcost, (UkLevel *)st.lev.p, dw, 0, s);
-    for (int cc = r.scost; cc <= r.fcost && e == hipSuccess; ++cc)
-      e = launch_ukk_level(dm, r, cc, (int64_t)st.box[cc - r.scost].nab * st.box[cc - r.scost].nac,
-                           (const UkLevel *)st.lev.p, (uint32_t *)st.U.p, A, B, C, r.fstate, r.fdist, dw, s);
-    if (e != hipSuccess) break;
-    if (r.fcost - r.scost <= cpw) {
-      e = launch_ukk_trace(dm, r, (const UkLevel *)st.lev.p, (const uint32_t *)st.U.p, A, B, C, (char *)dCols.p,
-                           col_cap, dw, s);
-      continue;
+  int error = 0;
+  for (bool open = true; open && e == hipSuccess;) {
+    open = false;
+    next.clear();
+    size_t i = 0;
+    while (i < nodes.size() && e == hipSuccess) {
+      // the next ranges whose levels fit the store together
+      st.box.clear();
+      st.job.clear();
+      int64_t words = kUkPad;
+      st.stride = 0;
+      const size_t i0 = i;
+      for (; i < nodes.size() && st.job.size() < kUkBatch; ++i) {
+        if (nodes[i].traced) continue;
+        const UkRange &r = nodes[i].r;
+        if (!st.job.empty() && (words - kUkPad + uk_words(r, ge, r.fcost)) * 4 > kUkStoreLimit) break;
+        UkJob j{r, r.fcost - r.scost + 1, r.fstate, r.fcost - r.scost <= cpw,
+                (r.fcost + r.scost - cpw + 1) / 2, 0, 0};
+        // a range's columns lie between its start and end indexes
+        const int sb = r.sdist - r.sab, sc = r.sdist - r.sac;
+        j.col0 = r.sdist + sb + sc - 3 * start;
+        j.col_cap = std::min(r.endA - r.sdist + r.endB - sb + r.endC - sc, col_cap - j.col0);
+        words += uk_words(r, ge, r.fcost);
+        st.stride = std::max(st.stride, j.nlev);
+        st.job.push_back(j);
+      }
+      int64_t base = kUkPad;
+      for (const UkJob &j : st.job) {
+        base = uk_boxes(st.box, j.r, ge, j.r.scost, j.r.fcost, base);
+        st.box.resize(st.box.size() + (size_t)(st.stride - j.nlev));
+      }
+      if (!st.job.empty()) {
+        ranges += st.job.size();
+        if (ranges > (size_t)8 * col_cap + 64) { cleanup(); return fail(POYG_EBAND, "the check-point recursion did not close"); }
+        const int rr = uk_reserve(st, words, false, s);
+        if (rr) { cleanup(); return rr; }
+        send(true);
+        for (int t = 0; t < st.stride; ++t) {
+          int64_t diags = 0;
+          for (size_t k = 0; k < st.job.size(); ++k) {
+            const UkLevel &b = st.box[k * st.stride + t];
+            diags = std::max(diags, (int64_t)b.nab * b.nac);
+          }
+          level(t, diags);
+        }
+        if (e == hipSuccess)
+          e = launch_ukk_walk(dm, st.jobs(), (int)st.job.size(), cpw, st.levels(), st.stride,
+                              (const uint32_t *)st.U.p, A, B, C, (char *)dCols.p, 0, st.walks(), s);
+        if (!read_walks()) break;
+      }
+      for (size_t k = i0, n = 0; k < i; ++k) {
+        if (nodes[k].traced) {
+          next.push_back(nodes[k]);
+          continue;
+        }
+        const UkWalk &w = st.walk[n];
+        const UkJob &j = st.job[n++];
+        if (j.base_case) {
+          error |= w.error;
+          next.push_back(UkNode{j.r, true, j.col0, w.ncols});
+        } else {
+          if (w.error || w.f_cost < 0) { cleanup(); return fail(POYG_EBAND, "a range's end has no check point"); }
+          split(next, j.r, w, w.reached);
+          open = true;
+        }
+      }
     }
-    const int cpcost = (r.fcost + r.scost - cpw + 1) / 2;
-    e = launch_ukk_walk(dm, r, cpcost, cpw, (const UkLevel *)st.lev.p, (const uint32_t *)st.U.p, 0, dw, s);
-    if (!read_walk()) break;
-    if (hw.error || hw.f_cost < 0) { cleanup(); return fail(POYG_EBAND, "a range's end has no check point"); }
-    const UkRange first{r.sab, r.sac, r.scost, r.sstate, r.sdist, hw.f_ab, hw.f_ac, hw.f_cost, hw.f_state, hw.f_dist,
-                        hw.f_dist, hw.f_dist - hw.f_ab, hw.f_dist - hw.f_ac};
-    const UkRange later{hw.f_ab, hw.f_ac, hw.f_cost, hw.f_state, hw.f_dist, r.fab, r.fac, hw.reached, r.fstate,
-                        r.fdist, r.endA, r.endB, r.endC};
-    stack.push_back(first);
-    stack.push_back(later);
+    nodes.swap(next);
   }
+  int ncols = 0;
+  for (const UkNode &k : nodes) ncols += k.ncols;
   std::vector<char> cols((size_t)3 * col_cap);
-  if (read_walk() && hw.ncols > 0)
-    e = hipMemcpy(cols.data(), dCols.p, (size_t)3 * hw.ncols, hipMemcpyDeviceToHost);
+  if (e == hipSuccess && ncols > 0)
+    e = hipMemcpy(cols.data(), dCols.p, (size_t)3 * col_cap, hipMemcpyDeviceToHost);
   if (e != hipSuccess) { cleanup(); return fail(POYG_EDEVICE, "search"); }
   cleanup();
-  if (hw.error) return fail(POYG_EBAND, "a traceback left its range");
-  const int len = 1 + start + hw.ncols;
+  if (error) return fail(POYG_EBAND, "a traceback left its range");
+  const int len = 1 + start + ncols;
   if (len > cap) {
     set_error("powell_3d: alignment of %d columns does not fit", len);
     return POYG_EINVAL;
@@ -1973,7 +2056,9 @@ int poyg_powell_3d(poyg_ctx *ctx, const uint8_t *a, int la, const uint8_t *b, in
     uint8_t *o = dst[q] + cap - len;
     o[0] = 16;
     for (int i = 0; i < start; ++i) o[1 + i] = mask(x[0][i]);
-    for (int i = 0; i < hw.ncols; ++i) o[1 + start + i] = mask(cols[(size_t)3 * (hw.ncols - 1 - i) + q]);
+    int i = 1 + start;
+    for (size_t k = nodes.size(); k-- > 0;)
+      for (int n = nodes[k].ncols; n-- > 0;) o[i++] = mask(cols[3 * ((size_t)nodes[k].col0 + n) + q]);
   }
   if (rlen) *rlen = len;
   if (cost) *cost = final_cost;

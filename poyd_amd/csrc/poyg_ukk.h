@@ -10,7 +10,9 @@
 // here one launch computes a whole cost level: every diagonal within the
 // range's reach at that cost, 16 states each, from the levels below (a
 // transition lowers the cost by at most maxSingleStep) and, for the
-// all-match state, the other states of the same level.  Each stored cell
+// all-match state, the other states of the same level.  Ranges that do not
+// depend on each other (all those of one depth of the check-point recursion)
+// share the launches of their levels.  Each stored cell
 // keeps its dist and which candidate won it (the reference's "from" record
 // follows from that and the check-point band), so the check-point split, the
 // base-case traceback and the reference's choice of check-point cost (the
@@ -32,8 +34,52 @@ constexpr int kUkMaxLen = 65534;    // a dist is stored in 16 bits as dist + 1 (
 //   62         the preset start cell of the range;  63  no candidate
 constexpr int kUkLower = 32, kUkExt = 33, kUkStart = 62, kUkNone = 63;
 
-// The model tables of setup (src/ukkCommon.c:247-330), states in the
-// reference's enumeration order (state 0 = all match).
+// The states in the reference's enumeration order (src/ukkCommon.c:247-330;
+// state 0 = all match): what each sequence does (0 match, 1 delete, 2 insert)
+// where at least one matches and at most one inserts.
+struct UkStateTable {
+  int t[kUkStates][3];
+  int n;
+};
+
+constexpr UkStateTable uk_states() {
+  UkStateTable T{};
+  for (int s = 0; s < 27; ++s) {
+    const int t[3] = {s % 3, (s / 3) % 3, (s / 9) % 3};
+    const int nm = (t[0] == 0) + (t[1] == 0) + (t[2] == 0), ni = (t[0] == 2) + (t[1] == 2) + (t[2] == 2);
+    if (nm == 0 || ni > 1) continue;
+    for (int q = 0; q < 3; ++q) T.t[T.n][q] = t[q];
+    ++T.n;
+  }
+  return T;
+}
+constexpr UkStateTable kUkTable = uk_states();
+static_assert(kUkTable.n == kUkStates, "sixteen states");
+
+// The sequences a state's step advances (bit 0 A, bit 1 B, bit 2 C): no
+// insert: the matching ones; one insert: only that one.
+constexpr int uk_step(int s) {
+  int ins = 0, mat = 0;
+  for (int q = 0; q < 3; ++q) {
+    ins |= (kUkTable.t[s][q] == 2) << q;
+    mat |= (kUkTable.t[s][q] == 0) << q;
+  }
+  return ins ? ins : mat;
+}
+
+// What continuing a state costs: 0 one mismatch (all match), 1 one gap
+// extension, 2 two.
+constexpr int uk_cont_kind(int s) {
+  int nm = 0, nd = 0, ni = 0;
+  for (int q = 0; q < 3; ++q) {
+    nm += kUkTable.t[s][q] == 0;
+    nd += kUkTable.t[s][q] == 1;
+    ni += kUkTable.t[s][q] == 2;
+  }
+  return nm == 3 ? 0 : ni || nd == 1 ? 1 : 2;
+}
+
+// The model tables of setup (src/ukkCommon.c:247-330).
 struct UkModel {
   int ns, mis, go, ge, max_step;
   int nb[kUkStates];       // neighbour step: bit 0 A, bit 1 B, bit 2 C advance
@@ -52,16 +98,33 @@ struct UkRange {
 
 // Where level c (scost <= c) of a range sits in the level store: the box of
 // diagonals within reach of the start at that cost, clipped to the ends.
+constexpr int kUkPad = 16;   // the store's first words, zero: what lies outside a level reads there
 struct UkLevel {
-  int ab_lo, ac_lo, nab, nac;
+  int64_t org;    // word of diagonal (0, 0)'s state 0, were it in the box
+  int nac;
+  int reach;      // how far from the start the level's diagonals lie: inside
+                  // the ends, the box is |ab - sab| <= reach, |ac - sac| <= reach
+  int ab_lo, ac_lo, nab, pad;
   int64_t base;   // first word of the level (16 words per diagonal)
+  int64_t pad2;
+};
+
+// One range of a batch: range i's nlev levels sit at lev[i * stride ..] of the
+// batch's descriptors, its columns start at col0 of the column store.
+struct UkJob {
+  UkRange r;
+  int nlev;
+  int target_state;   // the end condition's state; -1: the best state (doUkk's loop)
+  int base_case;      // traced, not split
+  int cpcost;         // where a split looks for its check point
+  int col0, col_cap;
 };
 
 // Diagonals within the reach of cost c from the start: every diagonal whose
 // cheapest cost (withinMatrix, src/ukk.checkp.c:545-576) is at most c has
 // both |ab - sab| and |ac - sac| at most (c - scost) / ge.
 __host__ __device__ inline UkLevel uk_level_box(const UkRange &r, int ge, int c, int64_t base) {
-  UkLevel L;
+  UkLevel L{};
   const int w = (c - r.scost) / ge;
   const int ab_lo = r.sab - w > -r.endB ? r.sab - w : -r.endB;
   const int ab_hi = r.sab + w < r.endA ? r.sab + w : r.endA;
@@ -72,6 +135,8 @@ __host__ __device__ inline UkLevel uk_level_box(const UkRange &r, int ge, int c,
   L.nab = ab_hi >= ab_lo ? ab_hi - ab_lo + 1 : 0;
   L.nac = ac_hi >= ac_lo ? ac_hi - ac_lo + 1 : 0;
   L.base = base;
+  L.org = base - ((int64_t)ab_lo * L.nac + ac_lo) * kUkStates;
+  L.reach = w;
   return L;
 }
 

@@ -563,6 +563,28 @@ def test_powell_search_choices(ctx, oracle):
             assert np.array_equal(al[q], want[1 + q]), (k, q)
 
 
+@pytest.mark.parametrize("mm,go,ge", [(1, 2, 1), (3, 4, 2), (2, 1, 3)])
+def test_powell_run_lengths(ctx, oracle, mm, go, ge):
+    """Runs of equal characters around a row's sixteen columns, up to the ends
+    of the sequences, and levels whose diagonals fill the last workgroup by
+    one to all of its sixteen rows (the boxes grow by odd squares)."""
+    from poyd_amd import engine
+    note(f"powell_3d run lengths mm={mm} go={go} ge={ge}")
+    rng = np.random.default_rng(61 + mm + 7 * go + 13 * ge)
+    for run in (15, 16, 17, 31, 32, 33, 49):
+        a = rand_seq(rng, 3 * run)
+        b, c = a.copy(), a.copy()
+        b[1 + run] = 1 if b[1 + run] != 1 else 2          # one substitution after the first run
+        c = np.delete(c, 1 + 2 * run)                     # one gap after the second
+        c = c[:len(c) - (run % 3)]                        # and ends of unequal length
+        for t in ([a, b, c], [c, a, b]):
+            cost, al = engine.powell_3d(ctx, *t, mm, go, ge)
+            want = oracle.powell_ukk(*t, mm, go, ge)
+            assert cost == want[0], run
+            for q in range(3):
+                assert np.array_equal(al[q], want[1 + q]), (run, q)
+
+
 def test_powell_rejects_gap_only_characters(ctx):
     from poyd_amd import engine
     x = np.array([16, 1, 16, 2], np.uint8)
