@@ -34,9 +34,9 @@ hipError_t launch_aff_quad(bool bt, int grid, const PairMeta *meta, const int32_
                            const uint8_t *seq, const DevTcm *tcm, uint8_t *dm, int32_t *cost, uint32_t *sink,
                            const uint8_t *pure, const TraceOut *tro, const int *n_dev, hipStream_t s);
 hipError_t launch_aff_pk(bool bt, int grid, const PairMeta *meta, const int32_t *order, int n, int *counter,
-                         const uint8_t *seq, const DevTcm *tcm, uint8_t *dm, int32_t *cost, uint32_t *sink,
+                         const uint8_t *seq, const DevTcm *tcm, uint8_t *dm, int32_t *cost,
                          const uint8_t *pure, int32_t *redo, int *redo_n, int32_t *tlist, int *tlist_n,
-                         hipStream_t s);
+                         const AffUniform &uni, hipStream_t s);
 int aff_pk_blocks_per_cu(bool bt);
 int aff_trace_list_blocks_per_cu();
 hipError_t launch_aff_trace_list(int grid, const PairMeta *meta, const int32_t *list, const int *list_n, int *counter,
@@ -44,7 +44,7 @@ hipError_t launch_aff_trace_list(int grid, const PairMeta *meta, const int32_t *
                                  hipStream_t s);
 hipError_t launch_aff_diag(bool bt, int sets, int grid, const PairMeta *meta, const int32_t *order, int n,
                            int *counter, const uint8_t *seq, const DevTcm *tcm, uint8_t *dm, int32_t *cost,
-                           uint32_t *sink, const TraceOut *tro, hipStream_t s);
+                           uint32_t *sink, const TraceOut *tro, const AffUniform &uni, hipStream_t s);
 hipError_t launch_aff_trace(const PairMeta *meta, const int32_t *order, int n, const uint8_t *seq,
                             const DevTcm *tcm, const uint8_t *dm, uint8_t *out, int32_t *out_len, int32_t *status,
                             hipStream_t s);
@@ -418,6 +418,7 @@ struct poyg_plan {
   // workgroup per pair, or 0 for one pair per wave
   int n_ldiag = 0, grid_ldiag = 0, ldiag_waves = 0;
   LinDiagCosts ldiag_costs{0, 0, 0};
+  AffUniform aff_uniform{0, 0, 0, 0};
   int n_trace = 0;   // linear pairs of the separate backtrace (order_all)
   // the narrow affine bands (order_quad) go to the packed eight-pair fill;
   // its pairs whose cost saturates 16 bits are listed in `redo` for the
@@ -795,6 +796,7 @@ static int plan_pairs_impl(poyg_ctx *ctx, const poyg_cm *cm, int mode, int32_t n
                       !(pc && pc->byte_band);
   for (int x = 0; x < 32; ++x) ldiag_matrix = ldiag_matrix && dt.prepend[x] == dt.cost[kGap * 32 + x];
   if (ldiag_matrix) P->ldiag_costs = lin_diag_costs(dt, align ? 4 : 1);
+  if (affine) P->aff_uniform = uniform_costs(dt);
   // tuned launch shapes (see poyg_ctx_set_tuning)
   // (a per-call pair runs alone: the one-pair-per-wave kernel steps one
   // diagonal pair per lane instead of three, a shorter latency)
@@ -839,11 +841,12 @@ static int plan_pairs_impl(poyg_ctx *ctx, const poyg_cm *cm, int mode, int32_t n
         // to long pairs, whose latency the one-pair-per-wave kernel keeps
         // lower (a lane of it steps one diagonal pair instead of three).
         if (ra > 0 && lanes <= quad_max) quad[k] = 3;
-        m.p1 = lanes;
+        // (whole lanes of three: such a lane stores its group in one access)
+        m.p1 = quad[k] ? (lanes + kQuadH - 1) / kQuadH * kQuadH : lanes;
         m.p2 = 1;
         if (align && ra > 0) {
           m.dm_off = dm_bytes;
-          dm_bytes += (((int64_t)ra + cb + 4) >> 2) * 4 * lanes;
+          dm_bytes += (((int64_t)ra + cb + 4) >> 2) * 4 * m.p1;
         }
       } else {
         m.stride = (int32_t)((std::min(cb + 1, e0 + 41) + 3) & ~3);
@@ -1298,15 +1301,15 @@ extern "C" int poyg_plan_run(poyg_plan *P, const uint8_t *d_seq, int32_t *d_cost
     auto quad = [&](int grid, hipStream_t st) {
       if (P->aff_pk)
         return launch_aff_pk(align, grid, meta, (const int32_t *)P->order_quad.p, P->n_quad, ctr + 6, d_seq, tcm, dm,
-                             d_cost, sink, (const uint8_t *)P->pure.p, (int32_t *)P->redo.p, ctr + 5,
-                             (int32_t *)P->tlist.p, ctr + 8, st);
+                             d_cost, (const uint8_t *)P->pure.p, (int32_t *)P->redo.p, ctr + 5,
+                             (int32_t *)P->tlist.p, ctr + 8, P->aff_uniform, st);
       return launch_aff_quad(align, grid, meta, (const int32_t *)P->order_quad.p, P->n_quad, ctr + 6, d_seq, tcm, dm,
                              d_cost, sink, (const uint8_t *)P->pure.p, (const TraceOut *)P->trout.p, nullptr, st);
     };
     auto diag = [&](int q, int grid, hipStream_t st) {
       return launch_aff_diag(align, q == 0 ? 1 : 2 * q, grid, meta, (const int32_t *)P->order_diag[q].p,
                              P->n_diag[q], ctr + 2 + q, d_seq, tcm, dm, d_cost, sink, (const TraceOut *)P->trout.p,
-                             st);
+                             P->aff_uniform, st);
     };
     for (int q = 2; q >= 1; --q)   // the widest bands: 4 and 2 lane sets
       if (P->n_diag[q]) HIP_TRY(diag(q, P->grid_diag[q], rs2));

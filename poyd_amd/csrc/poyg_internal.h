@@ -24,6 +24,24 @@ struct DevTcm {
   int gap, lcm, gap_open, cost_model, combinations, pad[3];
 };
 
+// An affine cost matrix of three costs: characters without the gap bit that
+// share a symbol cost nothing, others `sub`; a gap against any of them costs
+// `del` in the rows and `ins` in the columns.
+struct AffUniform {
+  int ok, sub, del, ins;
+};
+
+inline AffUniform uniform_costs(const DevTcm &t) {
+  const AffUniform u{1, t.cost[1 * 32 + 2], t.cost[1 * 32 + 16], t.prepend[1]}, no{0, 0, 0, 0};
+  if (u.sub < 0 || u.sub > 63) return no;   // four times it is a byte in the cells' arithmetic
+  for (int a = 1; a < 16; ++a) {
+    if (t.cost[a * 32 + 16] != u.del || t.prepend[a] != u.ins) return no;
+    for (int b = 1; b < 16; ++b)
+      if (t.cost[a * 32 + b] != ((a & b) ? 0 : u.sub)) return no;
+  }
+  return u;
+}
+
 // Three-dimensional cost matrix block for 5-bit alphabets.
 struct DevTcm3 {
   int cost[32 * 32 * 32];

@@ -539,6 +539,113 @@ struct AffDiagLanes {
 };
 
 
+// The steady groups of a pair without gap-bearing characters under a cost
+// matrix of three costs (AffUniform), the usual case: 24 instructions per step
+// and lane set against 132.  A wave alone on its SIMD issues one every 5 to 7
+// cycles whatever they depend on, so a step takes as long as its instructions:
+// * values are held as value << 2 in 32 bits (the plan's bound keeps them below
+//   2^31) with their rank in the final minimum (eh 0, cb 1, ev 2) as the low
+//   bits, so that minimum and the aligned state's need no more than the sums'
+//   constants to rank their candidates;
+// * what closes a cell at the band's edges rides in per-lane constants of the
+//   sums too: a closed cell's states are kHigh or more instead of kHigh (no
+//   path the backtrace follows compares two such values);
+// * the substitution costs of eight steps come from two words of each
+//   sequence's characters, four bytes at a time (nonzero byte of the AND: the
+//   characters share a symbol), so no character travels between lanes;
+// * the moves between lanes are the DPP operands of the sums (zero enters at
+//   the ends, where the constants close the cell);
+// * the direction bytes of four steps are put together byte-wise.
+// One alignment of 1,000 x 1,000, a call: 468 to 254 us (its kernel, with the
+// edge groups and the backtrace, 442 to 225).
+struct AffFree {
+  uint32_t eh1, ev1, cb1, eh2, ev2, cb2;
+};
+
+// Sums and minima of one cell; the four words its direction byte is made of:
+// kf & 3 todo, kc & 3 the aligned state's source (H 0, V 2, none 3), dv and
+// dh negative where the state is extended.
+struct AffFreeOut {
+  uint32_t kf, kc, dv, dh;
+};
+
+__device__ __forceinline__ AffFreeOut aff_free_cell(AffFree &S, uint32_t eh_l, uint32_t cb_l, uint32_t ev_u,
+                                                    uint32_t cb_u, uint32_t go_h, uint32_t go_v, uint32_t gap_h,
+                                                    uint32_t gap_v, uint32_t dg, uint32_t shut) {
+  // go_v: the opening and one (cb's rank to ev's); go_h: less one (to eh's)
+  AffFreeOut o;
+  const uint32_t t_v = cb_u + go_v, t_h = cb_l + go_h;
+  o.dv = ev_u - t_v;
+  o.dh = eh_l - t_h;
+  const uint32_t ev = min(ev_u, t_v) + gap_v, eh = min(eh_l, t_h) + gap_h;
+  o.kc = min(min(S.eh2 + dg + shut, S.ev2 + dg + shut), S.cb2 + dg + (shut + 2));
+  const uint32_t cb = (o.kc & ~3u) | 1;
+  o.kf = min(min(eh, cb), ev);
+  S.eh2 = S.eh1; S.ev2 = S.ev1; S.cb2 = S.cb1;
+  S.eh1 = eh; S.ev1 = ev; S.cb1 = cb;
+  return o;
+}
+
+// The direction bytes of four cells of a lane (even, odd, even, odd step).
+__device__ __forceinline__ uint32_t aff_free_bytes(const AffFreeOut (&o)[4], uint32_t keep, uint32_t edge) {
+  auto low = [](uint32_t a, uint32_t b, uint32_t c, uint32_t d) {   // byte 0 of each
+    return __builtin_amdgcn_perm(b, a, 0x0c0c0400u) | __builtin_amdgcn_perm(d, c, 0x04000c0cu);
+  };
+  auto top = [](uint32_t a, uint32_t b, uint32_t c, uint32_t d) {   // byte 3 of each
+    return __builtin_amdgcn_perm(b, a, 0x0c0c0703u) | __builtin_amdgcn_perm(d, c, 0x07030c0cu);
+  };
+  const uint32_t f = low(o[0].kf, o[1].kf, o[2].kf, o[3].kf) & 0x03030303u;
+  const uint32_t n = ((low(o[0].kc, o[1].kc, o[2].kc, o[3].kc) & 0x03030303u) + 0x01010101u) & 0x03030303u;
+  const uint32_t v = (top(o[0].dv, o[1].dv, o[2].dv, o[3].dv) >> 5) & 0x04040404u;
+  const uint32_t h = (top(o[0].dh, o[1].dh, o[2].dh, o[3].dh) >> 4) & 0x08080808u;
+  // END_V, END_H inverted (set where the opening is no dearer), END_B always
+  const uint32_t bytes = ((n << 5) | f | v | h) ^ 0x1c1c1c1cu;
+  return (bytes & keep) | edge;
+}
+
+__device__ __forceinline__ uint32_t dpp_below0(uint32_t v) {   // lane l <- lane l-1, lane 0 <- 0
+  return (uint32_t)__builtin_amdgcn_mov_dpp((int)v, 0x138, 0xf, 0xf, true);
+}
+__device__ __forceinline__ uint32_t dpp_above0(uint32_t v) {   // lane l <- lane l+1, lane 63 <- 0
+  return (uint32_t)__builtin_amdgcn_mov_dpp((int)v, 0x130, 0xf, 0xf, true);
+}
+// lane l <- lane l-1 of v, lane 0 <- lane 63 of w (the set below)
+__device__ __forceinline__ uint32_t dpp_below_set(uint32_t v, uint32_t w) {
+  const int wrap = __builtin_amdgcn_mov_dpp((int)w, 0x13c /* wave_ror:1 */, 0xf, 0xf, true);
+  return (uint32_t)__builtin_amdgcn_update_dpp(wrap, (int)v, 0x138, 0xf, 0xf, false);
+}
+// lane l <- lane l+1 of v, lane 63 <- lane 0 of w (the set above)
+__device__ __forceinline__ uint32_t dpp_above_set(uint32_t v, uint32_t w) {
+  const int wrap = __builtin_amdgcn_mov_dpp((int)w, 0x134 /* wave_rol:1 */, 0xf, 0xf, true);
+  return (uint32_t)__builtin_amdgcn_update_dpp(wrap, (int)v, 0x130, 0xf, 0xf, false);
+}
+
+// Four bytes of a sequence from any position, as the positions idx.. of it;
+// outside, some four bytes of it (lanes beyond the band, words not used).
+// len >= 3: the last position.
+__device__ __forceinline__ uint32_t load_four(const uint8_t *s, int idx, int len) {
+  uint32_t v;
+  __builtin_memcpy(&v, s + min(max(idx, 0), len - 3), 4);
+  return v;
+}
+
+// Every character of positions 1..len is one or several symbols without the
+// gap bit.  Called by every lane.
+__device__ __forceinline__ bool aff_gap_free(const uint8_t *s, int len) {
+  uint32_t bad = 0;
+  if (len < 4) {
+    const int v = s[min(max(lane_id(), 1), len)];
+    return __ballot(len > 0 && ((v & kGap) || !(v & 15))) == 0;
+  }
+#pragma unroll 4
+  for (int i = 1; i <= len; i += 4 * kWave) {
+    const uint32_t v = load_four(s, i + 4 * lane_id(), len);
+    // (the last words repeat earlier positions, never position 0)
+    bad |= (v & (kGap * 0x01010101u)) | (~((v & 0x0f0f0f0fu) + 0x7f7f7f7fu) & 0x80808080u);
+  }
+  return __ballot(bad != 0) == 0;
+}
+
 template <int K>
 __device__ __forceinline__ void aff_trace_pair(const PairMeta &m, int p, const uint8_t *__restrict__ seq,
                                                const uint8_t *__restrict__ dm_base, const uint8_t *s_med,
@@ -558,7 +665,7 @@ template <bool kBt, int R>
 __global__ __launch_bounds__(kWave * 4) void aff_diag_kernel(
     const PairMeta *__restrict__ meta, const int32_t *__restrict__ order, int n, int *counter,
     const uint8_t *__restrict__ seq, const DevTcm *__restrict__ tcm, uint8_t *dm_base, int32_t *cost_out,
-    uint32_t *sink, const TraceOut *trop) {
+    uint32_t *sink, const TraceOut *trop, AffUniform uni) {
   __shared__ int s_cost[32 * 32];
   __shared__ int s_prep[32];
   __shared__ uint8_t s_med[kBt ? 32 * 32 : 4];
@@ -720,6 +827,105 @@ __global__ __launch_bounds__(kWave * 4) void aff_diag_kernel(
     };
     int g = 0;
     for (; g < g_lo; ++g) group(g, std::false_type{});
+    // two groups at a time while the words read ahead lie inside the sequences
+    // (the band's lanes: eight pair-steps of steady cells)
+    if (uni.ok && g + 4 <= g_hi && aff_gap_free(A, la) && aff_gap_free(B, lb)) {
+      constexpr uint32_t kHigh4 = 4u * kHighNum;
+      const uint32_t go4 = 4u * (uint32_t)go, ins4 = 4u * (uint32_t)uni.ins, del4 = 4u * (uint32_t)uni.del;
+      AffFree S[R];
+      uint32_t go_v0[R], gap_h0[R], gap_v0[R], gap_v1[R], c0[R], c1[R], keep[R], edge[R];
+      uint32_t a0[R], a1[R], b0[R], b1[R];
+#pragma unroll
+      for (int r = 0; r < R; ++r) {
+        S[r] = AffFree{(uint32_t)L.S[r].eh1 * 4, (uint32_t)L.S[r].ev1 * 4 + 2, (uint32_t)L.S[r].cb1 * 4 + 1,
+                       (uint32_t)L.S[r].eh2 * 4, (uint32_t)L.S[r].ev2 * 4 + 2, (uint32_t)L.S[r].cb2 * 4 + 1};
+        const bool left = r == 0 && l0;                          // d = -40: the vertical state only
+        const bool shut0 = r0[r] || !v0[r], shut1 = r1[r] || !v1[r];   // right of the band
+        go_v0[r] = left ? kHigh4 + 1 : go4 + 1;
+        gap_h0[r] = left ? kHigh4 : ins4;
+        gap_v0[r] = shut0 ? kHigh4 : del4;
+        gap_v1[r] = shut1 ? kHigh4 : del4;
+        c0[r] = left || shut0 ? kHigh4 : 0;
+        c1[r] = shut1 ? kHigh4 : 0;
+        const uint32_t k0 = left || shut0 ? 0 : 0x00ff00ffu, k1 = shut1 ? 0 : 0xff00ff00u;
+        keep[r] = k0 | k1;
+        edge[r] = ~keep[r] & ((left ? kAffLeft * 0x00010001u : kAffRight * 0x00010001u) | kAffRight * 0x01000100u);
+        a0[r] = load_four(A, i0[r] + 2 * g, la);
+        b0[r] = load_four(B, j0[r] + 2 * g, lb);
+        a1[r] = load_four(A, i0[r] + 2 * g + 4, la);
+        b1[r] = load_four(B, j0[r] + 2 * g + 4, lb);
+      }
+      uint32_t *dst[R];
+#pragma unroll
+      for (int r = 0; r < R; ++r) dst[r] = dmw[r] + (size_t)g * dmw_step[r];
+      for (; g + 4 <= g_hi; g += 2) {
+        uint32_t zero[R][2];   // per byte 1 where the characters share no symbol: even and odd steps
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+          const uint32_t xe = a0[r] & b0[r] & 0x0f0f0f0fu,
+                         xo = a0[r] & __builtin_amdgcn_alignbyte(b1[r], b0[r], 1) & 0x0f0f0f0fu;
+          zero[r][0] = (~(xe + 0x7f7f7f7fu) >> 7) & 0x01010101u;
+          zero[r][1] = (~(xo + 0x7f7f7f7fu) >> 7) & 0x01010101u;
+          a0[r] = a1[r];
+          b0[r] = b1[r];
+          a1[r] = load_four(A, i0[r] + 2 * g + 8, la);
+          b1[r] = load_four(B, j0[r] + 2 * g + 8, lb);
+        }
+        dpp_exec_guard();
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+          AffFreeOut o[R][4];
+#pragma unroll
+          for (int q = 0; q < 2; ++q) {
+            const uint32_t sub = (uint32_t)(4 * uni.sub) << (8 * (2 * h + q));
+            uint32_t eh_l[R], cb_l[R], ev_u[R], cb_u[R];
+#pragma unroll
+            for (int r = 0; r < R; ++r) {   // even step: left neighbours from lane - 1
+              eh_l[r] = r == 0 ? dpp_below0(S[r].eh1) : dpp_below_set(S[r].eh1, S[r > 0 ? r - 1 : 0].eh1);
+              cb_l[r] = r == 0 ? dpp_below0(S[r].cb1) : dpp_below_set(S[r].cb1, S[r > 0 ? r - 1 : 0].cb1);
+            }
+#pragma unroll
+            for (int r = 0; r < R; ++r)
+              o[r][2 * q] = aff_free_cell(S[r], eh_l[r], cb_l[r], S[r].ev1, S[r].cb1, go4 - 1, go_v0[r], gap_h0[r],
+                                          gap_v0[r], __builtin_amdgcn_udot4(zero[r][0], sub, 0, false), c0[r]);
+#pragma unroll
+            for (int r = 0; r < R; ++r) {   // odd step: upper neighbours from lane + 1
+              ev_u[r] = r == R - 1 ? dpp_above0(S[r].ev1) : dpp_above_set(S[r].ev1, S[r < R - 1 ? r + 1 : 0].ev1);
+              cb_u[r] = r == R - 1 ? dpp_above0(S[r].cb1) : dpp_above_set(S[r].cb1, S[r < R - 1 ? r + 1 : 0].cb1);
+            }
+#pragma unroll
+            for (int r = 0; r < R; ++r)
+              o[r][2 * q + 1] = aff_free_cell(S[r], S[r].eh1, S[r].cb1, ev_u[r], cb_u[r], go4 - 1, go4 + 1, ins4,
+                                              gap_v1[r], __builtin_amdgcn_udot4(zero[r][1], sub, 0, false), c1[r]);
+          }
+          if (kBt) {
+#pragma unroll
+            for (int r = 0; r < R; ++r) {
+              *dst[r] = aff_free_bytes(o[r], keep[r], edge[r]);
+              dst[r] += dmw_step[r];
+            }
+          }
+        }
+      }
+      // the general groups' state
+      const int s = 2 * g - 1, base = 64 * ((g - 1) >> 5);
+      awin = load_or0(A, 20 + base + lane, la);
+      anext = load_or0(A, 84 + base + lane, la);
+      bwin = load_or0(B, bbase + base + lane, lb);
+      bnext = load_or0(B, bbase + base + 64 + lane, lb);
+#pragma unroll
+      for (int r = 0; r < R; ++r) {
+        L.S[r] = AffDiag{(int)(S[r].eh1 >> 2), (int)(S[r].ev1 >> 2), kHigh, (int)(S[r].cb1 >> 2),
+                         (int)(S[r].eh2 >> 2), (int)(S[r].ev2 >> 2), kHigh, (int)(S[r].cb2 >> 2)};
+        L.ic[r] = load_or0(A, i0[r] + s, la);
+        L.ip[r] = load_or0(A, i0[r] + s - 1, la);
+        L.jc[r] = load_or0(B, j0[r] + s + 1, lb);
+        L.jp[r] = load_or0(B, j0[r] + s, lb);
+        L.si_ge[r] = L.sive[r] = s_cost[L.ic[r] * 32 + kGap];
+        L.gap_row[r] = L.hx[r] = s_prep[L.jc[r]];
+        L.si_go[r] = L.sj_go[r] = go;
+      }
+    }
     for (; g < g_hi; ++g) group(g, std::true_type{});
     for (; g < groups; ++g) group(g, std::false_type{});
     // cell (la, lb) sits on diagonal lb - la, i.e. diagonal pair (lb - la + 40) / 2
@@ -1128,6 +1334,13 @@ __device__ __forceinline__ int dpp_row_from_below(int v, int fill) {   // lane q
 __device__ __forceinline__ int dpp_row_from_above(int v, int fill) {   // lane q <- q+1 in the row
   return __builtin_amdgcn_update_dpp(fill, v, 0x101 /* row_shl:1 */, 0xf, 0xf, false);
 }
+// the same with zero entering
+__device__ __forceinline__ uint32_t dpp_row_below0(uint32_t v) {
+  return (uint32_t)__builtin_amdgcn_mov_dpp((int)v, 0x111, 0xf, 0xf, true);
+}
+__device__ __forceinline__ uint32_t dpp_row_above0(uint32_t v) {
+  return (uint32_t)__builtin_amdgcn_mov_dpp((int)v, 0x101, 0xf, 0xf, true);
+}
 // lane q <- lane (q + 1) mod 16 of its row
 __device__ __forceinline__ int dpp_row_rotate_down(int v) {
   return __builtin_amdgcn_update_dpp(0, v, 0x12f /* row_ror:15 */, 0xf, 0xf, false);
@@ -1140,16 +1353,12 @@ __device__ __forceinline__ int dpp_row_rotate_down(int v) {
 __global__ __launch_bounds__(kWave * 4) void pair_pure_kernel(const PairMeta *__restrict__ meta,
                                                             const int32_t *__restrict__ order, int n,
                                                             const uint8_t *__restrict__ seq, uint8_t *pure) {
-  const int lane = lane_id();
   const int waves = gridDim.x * (blockDim.x / kWave);
   for (int w = blockIdx.x * (blockDim.x / kWave) + wave_in_group(); w < n; w += waves) {
     const int p = uniform32(order[w]);
     const PairMeta m = uniform_meta(meta, p);
-    int ga = 0, gb = 0;
-    for (int x = 1 + lane; x < m.lr; x += kWave) ga |= seq[m.off_r + x];
-    for (int x = 1 + lane; x < m.lc; x += kWave) gb |= seq[m.off_c + x];
-    const bool any_a = __ballot(ga & kGap) != 0, any_b = __ballot(gb & kGap) != 0;
-    pure[p] = (any_a ? 0 : 1) | (any_b ? 0 : 2);   // every lane stores the same value
+    const bool free_a = aff_gap_free(seq + m.off_r, m.lr - 1), free_b = aff_gap_free(seq + m.off_c, m.lc - 1);
+    pure[p] = (free_a ? 1 : 0) | (free_b ? 2 : 0);   // every lane stores the same value
   }
 }
 
@@ -1459,6 +1668,16 @@ __device__ __forceinline__ uint32_t c16_lt01(uint32_t a, uint32_t b) {
   asm("v_pk_min_u16 %0, %1, %2" : "=v"(r) : "v"(c16_sub_sat(b, a)), "s"(kPkRank1));
   return r;
 }
+// per half: 2 where a < b by at least 2, 0 where a >= b
+__device__ __forceinline__ uint32_t c16_lt02(uint32_t a, uint32_t b) {
+  uint32_t r;
+  asm("v_pk_min_u16 %0, %1, %2" : "=v"(r) : "v"(c16_sub_sat(b, a)), "s"(kPkRank2));
+  return r;
+}
+// (a & b) | c at the rate of the plain logic operations, twice v_and_or_b32's
+__device__ __forceinline__ uint32_t and_or(uint32_t a, uint32_t b, uint32_t c) {
+  return __builtin_amdgcn_bitop3_b32(a, b, c, 0xea);
+}
 // two 16-bit table entries at the byte offsets held in the halves of a
 __device__ __forceinline__ uint32_t lds_pair(const uint16_t *t, uint32_t a) {
   const uint32_t lo = *(const uint16_t *)((const char *)t + (a & 0xffffu));
@@ -1599,6 +1818,42 @@ __device__ __forceinline__ uint32_t aff_pk_cell(AffDiag &S, uint32_t eh_l, uint3
   return byte;
 }
 
+// One cell of two pairs without gap-bearing characters under three costs, in
+// packed halves: aff_free_cell's form (ranks inside the states, the closing
+// of cells in per-lane constants, here by saturation).  A group of four steps
+// takes 355 vector instructions against the 592 of gap-free cells with table
+// costs.
+struct PkFreeOut {
+  uint32_t kf, kc, end;   // end: bit 0 where the vertical state is extended, bit 1 the horizontal one
+};
+
+__device__ __forceinline__ PkFreeOut aff_pk_free_cell(AffDiag &S, uint32_t eh_l, uint32_t cb_l, uint32_t ev_u,
+                                                      uint32_t cb_u, uint32_t go_h, uint32_t go_v, uint32_t gap_h,
+                                                      uint32_t gap_v, uint32_t dg, uint32_t shut) {
+  PkFreeOut o;
+  const uint32_t t_v = c16_add_sat(cb_u, go_v), t_h = c16_add_sat(cb_l, go_h);
+  // (the values compared have one rank, so they differ by at least four: the
+  // smaller of the difference and two is the flag already in its place)
+  o.end = c16_lt01(ev_u, t_v) | c16_lt02(eh_l, t_h);
+  const uint32_t ev = c16_add_sat(c16_min(ev_u, t_v), gap_v), eh = c16_add_sat(c16_min(eh_l, t_h), gap_h);
+  o.kc = c16_min(c16_min(c16_add_sat(S.eh2, dg), c16_add_sat(S.ev2, dg)), c16_add_sat(S.cb2, dg | kPkRank2));
+  const uint32_t cb = and_or(o.kc, 0xfffcfffcu, shut);   // shut: the rank, all ones where the cell is closed
+  o.kf = c16_min(c16_min(eh, cb), ev);
+  S.eh2 = S.eh1; S.ev2 = S.ev1; S.cb2 = S.cb1;
+  S.eh1 = (int)eh; S.ev1 = (int)ev; S.cb1 = (int)cb;
+  return o;
+}
+
+// The direction bytes of two steps (even, odd) of both pairs of a lane.
+__device__ __forceinline__ uint32_t aff_pk_free_bytes(const PkFreeOut &a, const PkFreeOut &b, uint32_t keep,
+                                                      uint32_t edge) {
+  const uint32_t f = __builtin_amdgcn_perm(b.kf, a.kf, 0x06020400u) & 0x03030303u;
+  const uint32_t n = ((__builtin_amdgcn_perm(b.kc, a.kc, 0x06020400u) & 0x03030303u) + 0x01010101u) & 0x03030303u;
+  const uint32_t e = __builtin_amdgcn_perm(b.end, a.end, 0x06020400u);
+  const uint32_t bytes = ((n << 5) | ((e << 2) | f)) ^ 0x1c1c1c1cu;
+  return and_or(bytes, keep, edge);
+}
+
 template <int H>
 struct PkLanes {
   AffDiag S[H];
@@ -1620,13 +1875,19 @@ template <bool kBt, int H>
 __global__ __launch_bounds__(kWave * 4, 2) void aff_pk_kernel(
     const PairMeta *__restrict__ meta, const int32_t *__restrict__ order, int n, int *counter,
     const uint8_t *__restrict__ seq, const DevTcm *__restrict__ tcm, uint8_t *dm_base, int32_t *cost_out,
-    uint32_t *sink, const uint8_t *__restrict__ pure, int32_t *redo, int *redo_n, int32_t *tlist, int *tlist_n) {
+    const uint8_t *__restrict__ pure, int32_t *redo, int *redo_n, int32_t *tlist, int *tlist_n,
+    AffUniform uni) {
   __shared__ uint16_t s_c4[32 * 32];   // min(4 cost, 0xffff)
   __shared__ uint16_t s_p4[32];        // min(4 prepend, 0xffff)
   for (int k = threadIdx.x; k < 32 * 32; k += blockDim.x) s_c4[k] = (uint16_t)min(4ll * tcm->cost[k], 0xffffll);
   for (int k = threadIdx.x; k < 32; k += blockDim.x) s_p4[k] = (uint16_t)min(4ll * tcm->prepend[k], 0xffffll);
   __syncthreads();
   const uint32_t go4 = (uint32_t)min(4ll * tcm->gap_open, 0xffffll) * 0x00010001u;
+  // the three-cost form: a rank above and below the opening cost fits beside it
+  const bool three = uni.ok && tcm->gap_open >= 1 && tcm->gap_open < 0x3fff;
+  const uint32_t sub4 = (uint32_t)(4 * uni.sub) * 0x00010001u;
+  const uint32_t ins4 = (uint32_t)min(4ll * uni.ins, 0xffffll) * 0x00010001u;
+  const uint32_t del4 = (uint32_t)min(4ll * uni.del, 0xffffll) * 0x00010001u;
   const int lane = lane_id();
   const int q = lane & 15;
   for (;;) {
@@ -1711,6 +1972,15 @@ __global__ __launch_bounds__(kWave * 4, 2) void aff_pk_kernel(
     uint32_t awin = pk_row_char(AA, AB, 20 + q, laA, laB);
     uint32_t bwin = pk_col_char(BA, BB, 16 * H - 20 + ((q + 1) & 15), lbA, lbB);
     uint32_t anext = 0, bnext = 0;
+    // a lane's H dwords of both pairs' group g: one access each (the plan makes
+    // W a multiple of H, so a lane's dwords are all inside the band's rows or
+    // all outside).  Stored one by one, 12 bytes apart between lanes, they
+    // bound the fill: 65,536 pairs of 50-5,000 took 9.25 ms with them and the
+    // shorter cells, 9.4 ms with the longer ones; 7.0 ms with this.
+    auto store_group = [&](int g, const uint32_t (&dA)[H], const uint32_t (&dB)[H]) {
+      if (actA && g < GsA && H * q < WA) __builtin_memcpy(dmwA + (size_t)g * WA + H * q, dA, sizeof dA);
+      if (actB && g < GsB && H * q < WB) __builtin_memcpy(dmwB + (size_t)g * WB + H * q, dB, sizeof dB);
+    };
     auto group = [&](int g, auto variant_tag) {
       constexpr int kVar = decltype(variant_tag)::value;
       constexpr bool kSt = kVar >= 1, kPu = kVar >= 2, kGF = kVar == 3;
@@ -1803,21 +2073,80 @@ __global__ __launch_bounds__(kWave * 4, 2) void aff_pk_kernel(
           }
         }
         if (kBt) {
-          const bool ginA = actA && g < GsA, ginB = actB && g < GsB;
+          uint32_t dA[H], dB[H];
 #pragma unroll
           for (int k = 0; k < H; ++k) {
             // [even h0, odd h0, even h1, odd h1] of each pair, as
             // aff_quad_kernel stores them
             const uint32_t t0 = __builtin_amdgcn_perm(by[k][1], by[k][0], 0x06020400u);
             const uint32_t t1 = __builtin_amdgcn_perm(by[k][3], by[k][2], 0x06020400u);
-            const uint32_t accA = __builtin_amdgcn_perm(t1, t0, 0x05040100u);
-            const uint32_t accB = __builtin_amdgcn_perm(t1, t0, 0x07060302u);
-            uint32_t *dA = (ginA && Lk[k] < WA) ? dmwA + (size_t)g * WA + Lk[k] : sink + lane;
-            uint32_t *dB = (ginB && Lk[k] < WB) ? dmwB + (size_t)g * WB + Lk[k] : sink + lane;
-            *dA = accA;
-            *dB = accB;
+            dA[k] = __builtin_amdgcn_perm(t1, t0, 0x05040100u);
+            dB[k] = __builtin_amdgcn_perm(t1, t0, 0x07060302u);
+          }
+          store_group(g, dA, dB);
+        }
+      }
+    };
+    // groups of the three-cost form: two pair-steps as above, the characters'
+    // symbols in bits 12-15 of the halves (shared symbols AND to 4,096 or more,
+    // above any four substitution costs)
+    uint32_t shut0[H], shut1[H], gapv0[H], gapv1[H], keep[H], edge[H], gov0 = 0, gaph0 = 0;
+    auto free_group = [&](int g) {
+      if ((g & 7) == 0) {
+        awin = anext;
+        bwin = bnext;
+        anext = (pk_row_char(AA, AB, 2 * g + 16 + 20 + q, laA, laB) & 0x03c003c0u) << 6;
+        bnext = (pk_col_char(BA, BB, 2 * g + 16 + 16 * H - 20 + ((q + 1) & 15), lbA, lbB) & 0x001e001eu) << 11;
+      }
+      PkFreeOut o[H][4];
+      dpp_exec_guard();   // (no branch from here to the stores)
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        {   // even step
+          uint32_t nic = (uint32_t)dpp_row_from_below((int)Q.ic[H - 1], (int)awin);
+          uint32_t eh_l0 = dpp_row_below0((uint32_t)Q.S[H - 1].eh1);
+          uint32_t cb_l0 = dpp_row_below0((uint32_t)Q.S[H - 1].cb1);
+          awin = (uint32_t)dpp_row_rotate_down((int)awin);
+#pragma unroll
+          for (int k = H - 1; k > 0; --k) Q.ic[k] = Q.ic[k - 1];
+          Q.ic[0] = nic;
+#pragma unroll
+          for (int k = H - 1; k >= 0; --k) {
+            const uint32_t eh_l = k == 0 ? eh_l0 : (uint32_t)Q.S[k > 0 ? k - 1 : 0].eh1;
+            const uint32_t cb_l = k == 0 ? cb_l0 : (uint32_t)Q.S[k > 0 ? k - 1 : 0].cb1;
+            o[k][2 * h] = aff_pk_free_cell(Q.S[k], eh_l, cb_l, (uint32_t)Q.S[k].ev1, (uint32_t)Q.S[k].cb1,
+                                           go4 - kPkRank1, k == 0 ? gov0 : go4 + kPkRank1, k == 0 ? gaph0 : ins4,
+                                           gapv0[k], c16_sub_sat(sub4, Q.ic[k] & Q.jc[k]), shut0[k]);
           }
         }
+        {   // odd step
+          uint32_t njc = (uint32_t)dpp_row_from_above((int)Q.jc[0], (int)bwin);
+          uint32_t ev_u0 = dpp_row_above0((uint32_t)Q.S[0].ev1);
+          uint32_t cb_u0 = dpp_row_above0((uint32_t)Q.S[0].cb1);
+          bwin = (uint32_t)dpp_row_rotate_down((int)bwin);
+#pragma unroll
+          for (int k = 0; k < H - 1; ++k) Q.jc[k] = Q.jc[k + 1];
+          Q.jc[H - 1] = njc;
+#pragma unroll
+          for (int k = 0; k < H; ++k) {
+            const uint32_t ev_u = k == H - 1 ? ev_u0 : (uint32_t)Q.S[k < H - 1 ? k + 1 : 0].ev1;
+            const uint32_t cb_u = k == H - 1 ? cb_u0 : (uint32_t)Q.S[k < H - 1 ? k + 1 : 0].cb1;
+            o[k][2 * h + 1] = aff_pk_free_cell(Q.S[k], (uint32_t)Q.S[k].eh1, (uint32_t)Q.S[k].cb1, ev_u, cb_u,
+                                               go4 - kPkRank1, go4 + kPkRank1, ins4, gapv1[k],
+                                               c16_sub_sat(sub4, Q.ic[k] & Q.jc[k]), shut1[k]);
+          }
+        }
+      }
+      if (kBt) {
+        uint32_t dA[H], dB[H];
+#pragma unroll
+        for (int k = 0; k < H; ++k) {
+          const uint32_t t0 = aff_pk_free_bytes(o[k][0], o[k][1], keep[k], edge[k]);
+          const uint32_t t1 = aff_pk_free_bytes(o[k][2], o[k][3], keep[k], edge[k]);
+          dA[k] = __builtin_amdgcn_perm(t1, t0, 0x05040100u);
+          dB[k] = __builtin_amdgcn_perm(t1, t0, 0x07060302u);
+        }
+        store_group(g, dA, dB);
       }
     };
     if (groups >= 1536) __builtin_amdgcn_s_setprio(2);
@@ -1826,7 +2155,54 @@ __global__ __launch_bounds__(kWave * 4, 2) void aff_pk_kernel(
     const int gs_lo = min(g_lo, groups), gs_hi = max(gs_lo, min(g_hi, groups));
     int g = 0;
     for (; g < gs_lo; ++g) group(g, std::integral_constant<int, 0>{});
-    if (all_free) {
+    if (all_free && three && g < gs_hi) {
+      // (a group's first window swap happens in the group: bits both windows here)
+      awin = (awin & 0x03c003c0u) << 6;
+      anext = (anext & 0x03c003c0u) << 6;
+      bwin = (bwin & 0x001e001eu) << 11;
+      bnext = (bnext & 0x001e001eu) << 11;
+#pragma unroll
+      for (int k = 0; k < H; ++k) {
+        const int d0 = 2 * Lk[k] - 40;
+        const bool left = Lk[k] == 0;
+        const uint32_t right0 = halves(d0 >= E0A, d0 >= E0B), right1 = halves(d0 + 1 >= E0A, d0 + 1 >= E0B);
+        const uint32_t closed0 = left ? kPkHigh : right0;
+        shut0[k] = closed0 | kPkRank1;
+        shut1[k] = right1 | kPkRank1;
+        gapv0[k] = right0 | del4;
+        gapv1[k] = right1 | del4;
+        keep[k] = ~((closed0 & 0x00ff00ffu) | (right1 & 0xff00ff00u));
+        edge[k] = ~keep[k] & ((left ? kAffLeft * 0x00010001u : kAffRight * 0x00010001u) | kAffRight * 0x01000100u);
+        Q.ic[k] = (Q.ic[k] & 0x03c003c0u) << 6;
+        Q.jc[k] = (Q.jc[k] & 0x001e001eu) << 11;
+        Q.S[k].ev1 |= (int)kPkRank2;
+        Q.S[k].ev2 |= (int)kPkRank2;
+        Q.S[k].cb1 |= (int)kPkRank1;
+        Q.S[k].cb2 |= (int)kPkRank1;
+      }
+      gov0 = q == 0 ? kPkHigh : go4 + kPkRank1;
+      gaph0 = q == 0 ? kPkHigh : ins4;
+      for (; g < gs_hi; ++g) free_group(g);
+      awin >>= 6;
+      anext >>= 6;
+      bwin >>= 11;
+      bnext >>= 11;
+#pragma unroll
+      for (int k = 0; k < H; ++k) {
+        Q.ic[k] >>= 6;
+        Q.jc[k] >>= 11;
+        Q.ip[k] = Q.ic[k];   // (only its gap bit is read, and it has none)
+        Q.jp[k] = Q.jc[k];
+        Q.S[k].ev1 &= (int)0xfffcfffcu;
+        Q.S[k].ev2 &= (int)0xfffcfffcu;
+        Q.S[k].cb1 &= (int)0xfffcfffcu;
+        Q.S[k].cb2 &= (int)0xfffcfffcu;
+        Q.S[k].eb1 = Q.S[k].eb2 = (int)kPkHigh;
+        Q.si_ge[k] = Q.sive[k] = lds_pair(s_c4, Q.ic[k] + 2u * kGap * 0x00010001u);
+        Q.gap_row[k] = Q.hx[k] = lds_pair(s_p4, Q.jc[k]);
+        Q.si_go[k] = Q.sj_go[k] = go4;
+      }
+    } else if (all_free) {
       for (; g < gs_hi; ++g) group(g, std::integral_constant<int, 3>{});
       // the gap-free groups kept only si_ge and gap_row; for rows and
       // columns without gap-bearing characters the other costs follow
@@ -3391,21 +3767,21 @@ int aff_diag_blocks_per_cu(bool bt, int sets) {
 template <int R>
 static void launch_diag_r(bool bt, int grid, const PairMeta *meta, const int32_t *order, int n, int *counter,
                           const uint8_t *seq, const DevTcm *tcm, uint8_t *dm, int32_t *cost, uint32_t *sink,
-                          const TraceOut *tro, hipStream_t s) {
+                          const TraceOut *tro, const AffUniform &uni, hipStream_t s) {
   if (bt)
     hipLaunchKernelGGL((aff_diag_kernel<true, R>), dim3(grid), dim3(kWave * 4), 0, s, meta, order, n, counter, seq,
-                       tcm, dm, cost, sink, tro);
+                       tcm, dm, cost, sink, tro, uni);
   else
     hipLaunchKernelGGL((aff_diag_kernel<false, R>), dim3(grid), dim3(kWave * 4), 0, s, meta, order, n, counter, seq,
-                       tcm, dm, cost, sink, tro);
+                       tcm, dm, cost, sink, tro, uni);
 }
 
 hipError_t launch_aff_diag(bool bt, int sets, int grid, const PairMeta *meta, const int32_t *order, int n,
                            int *counter, const uint8_t *seq, const DevTcm *tcm, uint8_t *dm, int32_t *cost,
-                           uint32_t *sink, const TraceOut *tro, hipStream_t s) {
-  if (sets == 1) launch_diag_r<1>(bt, grid, meta, order, n, counter, seq, tcm, dm, cost, sink, tro, s);
-  else if (sets == 2) launch_diag_r<2>(bt, grid, meta, order, n, counter, seq, tcm, dm, cost, sink, tro, s);
-  else launch_diag_r<4>(bt, grid, meta, order, n, counter, seq, tcm, dm, cost, sink, tro, s);
+                           uint32_t *sink, const TraceOut *tro, const AffUniform &uni, hipStream_t s) {
+  if (sets == 1) launch_diag_r<1>(bt, grid, meta, order, n, counter, seq, tcm, dm, cost, sink, tro, uni, s);
+  else if (sets == 2) launch_diag_r<2>(bt, grid, meta, order, n, counter, seq, tcm, dm, cost, sink, tro, uni, s);
+  else launch_diag_r<4>(bt, grid, meta, order, n, counter, seq, tcm, dm, cost, sink, tro, uni, s);
   return hipGetLastError();
 }
 
@@ -3448,15 +3824,15 @@ hipError_t launch_aff_quad(bool bt, int grid, const PairMeta *meta, const int32_
 }
 
 hipError_t launch_aff_pk(bool bt, int grid, const PairMeta *meta, const int32_t *order, int n, int *counter,
-                         const uint8_t *seq, const DevTcm *tcm, uint8_t *dm, int32_t *cost, uint32_t *sink,
+                         const uint8_t *seq, const DevTcm *tcm, uint8_t *dm, int32_t *cost,
                          const uint8_t *pure, int32_t *redo, int *redo_n, int32_t *tlist, int *tlist_n,
-                         hipStream_t s) {
+                         const AffUniform &uni, hipStream_t s) {
   if (bt)
     hipLaunchKernelGGL((aff_pk_kernel<true, 3>), dim3(grid), dim3(kWave * 4), 0, s, meta, order, n, counter, seq,
-                       tcm, dm, cost, sink, pure, redo, redo_n, tlist, tlist_n);
+                       tcm, dm, cost, pure, redo, redo_n, tlist, tlist_n, uni);
   else
     hipLaunchKernelGGL((aff_pk_kernel<false, 3>), dim3(grid), dim3(kWave * 4), 0, s, meta, order, n, counter, seq,
-                       tcm, dm, cost, sink, pure, redo, redo_n, tlist, tlist_n);
+                       tcm, dm, cost, pure, redo, redo_n, tlist, tlist_n, uni);
   return hipGetLastError();
 }
 

@@ -169,6 +169,43 @@ def test_affine_block_indels(ctx, oracle, sub, indel, go):
             assert np.array_equal(res.seq(k, slot), want), (k, slot, len(a), len(b))
 
 
+@pytest.mark.parametrize("sub,indel,go", [(1, 1, 3), (2, 3, 1), (63, 2, 4), (64, 2, 4), (0, 1, 2)])
+@pytest.mark.parametrize("alphabet", ["dna", "ambig"])
+def test_affine_three_cost_groups(ctx, oracle, sub, indel, go, alphabet):
+    """The steady groups of sequences without gap-bearing characters: lengths
+    at which the first of them appear and end, bands at the last and first
+    widths of 3 diagonal pairs a lane and of 1, 2 and 4 lane sets, one pair
+    with a gap-bearing character among them, costs at and past the largest
+    the form takes, in batches and per call."""
+    from poyd_amd import engine
+    note(f"affine three-cost groups sub={sub} indel={indel} go={go} alphabet={alphabet}")
+    rng = np.random.default_rng(900 + sub + 7 * indel + 13 * go)
+    pairs = []
+    for n in (99, 100, 101, 102, 103, 107, 108, 109, 110, 116, 124, 250):
+        a = rand_seq(rng, n, alphabet)
+        pairs.append((a, mutate(rng, a, 0.15, 0.06)))
+    for diff in (46, 47, 48, 79, 80, 207, 208):       # E0 = diff + 8
+        a = rand_seq(rng, 420, alphabet)
+        b = np.concatenate([a[:200], rand_seq(rng, diff, alphabet)[1:], a[200:]])
+        pairs.append((a, mutate(rng, b, 0.1, 0.0)))
+    gapped = pairs[11][0].copy()
+    gapped[77] |= GAP
+    A = [p[0] for p in pairs] * 2 + [gapped]
+    B = [p[1] for p in pairs] * 2 + [pairs[11][1]]
+    cm, ref = engine.CostMatrix.of_sub_indel(sub, indel, go), oracle.CM2.sub_indel(sub, indel, go)
+    res = engine.run_pairs(ctx, cm, engine.POYG_MODE_AFFINE_ALIGN, batch_of(A), batch_of(B))
+    cost = engine.run_pairs(ctx, cm, engine.POYG_MODE_AFFINE_COST, batch_of(A), batch_of(B)).cost
+    al = engine.Align(ctx)
+    for k, (a, b) in enumerate(zip(A, B)):
+        med, ri, rj, want, mwg = oracle.align_affine_3(a, b, ref)
+        assert res.cost[k] == want and cost[k] == oracle.cost_affine_3(a, b, ref), k
+        for slot, w in enumerate((med, mwg, ri, rj)):
+            assert np.array_equal(res.seq(k, slot), w), (k, slot)
+        if k < len(pairs):
+            got = al.align_affine_3(a, b, cm)
+            assert got[3] == want and all(np.array_equal(x, y) for x, y in zip(got[:3] + got[4:], (med, ri, rj, mwg))), k
+
+
 @pytest.mark.parametrize("alphabet", ["dna", "any"])
 def test_affine_packed_fill_saturation(ctx, oracle, alphabet):
     """The packed 16-bit narrow-band fill holds values as 4 v saturated at
