@@ -387,6 +387,10 @@ __device__ __forceinline__ int dpp_from_above(int v, int fill) {   // lane l <- 
 
 __device__ __forceinline__ int min3_i32(int a, int b, int c) { return min(min(a, b), c); }
 
+// The first step whose cells all have i >= 1 and j >= 1: on the left edge
+// (d = -40) j = (t - 40) / 2, on the right one (d = E0) i = (t - E0) / 2.
+__device__ __forceinline__ int aff_steady_from(int E0) { return max(42, E0 + 2); }
+
 // Branch-free bounded read: the index is clamped, the value then masked, so
 // no lane is switched off (see aff_diag_kernel).
 __device__ __forceinline__ int load_or0(const uint8_t *s, int idx, int len) {
@@ -403,9 +407,9 @@ struct AffDiag {
 // :2250-2280 with the band rules of :2287-2548).  Returns the direction byte.
 // (eh_l, cb_l) are the states of the left neighbour (i, j-1), (ev_u, cb_u)
 // those of the upper one (i-1, j); the diagonal one is S's step-before-last.
-// kSteady: every cell of the step has 41 <= i <= la and j <= lb, so the band
-// edges are the fixed lanes d == -40 (left) and d == E0 (right), given as
-// flags; no row 0 and no final cell occur.
+// kSteady: every cell of the step has 1 <= i <= la and 1 <= j <= lb, so the
+// band edges are the fixed lanes d == -40 (left) and d == E0 (right), given as
+// flags; no row 0, no column 0 and no final cell occur.
 template <bool kBt, bool kSteady, bool kPure = false, bool kGapFree = false>
 __device__ __forceinline__ uint32_t aff_diag_cell(AffDiag &S, int eh_l, int cb_l, int ev_u, int cb_u, int i, int j,
                                                   int la, int lb, int E0, int go, const int *s_cost, int ic, int ip,
@@ -556,8 +560,10 @@ struct AffDiagLanes {
 // * the moves between lanes are the DPP operands of the sums (zero enters at
 //   the ends, where the constants close the cell);
 // * the direction bytes of four steps are put together byte-wise.
-// One alignment of 1,000 x 1,000, a call: 468 to 254 us (its kernel, with the
-// edge groups and the backtrace, 442 to 225).
+// They run from the first step without row-0 or column-0 cells to the end: what
+// lies past the last row or column reaches no cell inside.
+// One alignment of 1,000 x 1,000, a call: 472 to 225 us (259 with the general
+// groups for the last rows and, until i > 40 on every diagonal, the first).
 struct AffFree {
   uint32_t eh1, ev1, cb1, eh2, ev2, cb2;
 };
@@ -620,13 +626,16 @@ __device__ __forceinline__ uint32_t dpp_above_set(uint32_t v, uint32_t w) {
   return (uint32_t)__builtin_amdgcn_update_dpp(wrap, (int)v, 0x130, 0xf, 0xf, false);
 }
 
-// Four bytes of a sequence from any position, as the positions idx.. of it;
-// outside, some four bytes of it (lanes beyond the band, words not used).
-// len >= 3: the last position.
+// Four bytes of a sequence from any position within it (len >= 3: the last
+// position); clamped to it, some four bytes of it.
 __device__ __forceinline__ uint32_t load_four(const uint8_t *s, int idx, int len) {
   uint32_t v;
   __builtin_memcpy(&v, s + min(max(idx, 0), len - 3), 4);
   return v;
+}
+// What load_four read at idx, with zeros for the positions past the end.
+__device__ __forceinline__ uint32_t four_at(uint32_t v, int idx, int len) {
+  return (uint32_t)((uint64_t)v >> (8 * min(max(idx - (len - 3), 0), 4)));
 }
 
 // Every character of positions 1..len is one or several symbols without the
@@ -730,8 +739,8 @@ __global__ __launch_bounds__(kWave * 4) void aff_diag_kernel(
     const int bbase = 44 + 64 * (R - 1);
     int bwin = load_or0(B, bbase + lane, lb), bnext = load_or0(B, bbase + 64 + lane, lb);
     const int groups = (la + lb + 4) >> 2;   // ceil((la + lb + 1) / 4)
-    // steady steps: t in [E0 + 82, min(2 lb - E0, 2 la - 40)]
-    const int t_lo = E0 + 82, t_hi = min(2 * lb - E0, 2 * la - 40);
+    // steady steps: t in [max(42, E0 + 2), min(2 lb - E0, 2 la - 40)]
+    const int t_lo = aff_steady_from(E0), t_hi = min(2 * lb - E0, 2 * la - 40);
     int g_lo = (t_lo + 3) >> 2, g_hi = t_hi >= 3 ? (t_hi - 3) / 4 + 1 : 0;
     g_lo = min(g_lo, groups);
     g_hi = max(g_lo, min(g_hi, groups));
@@ -827,9 +836,9 @@ __global__ __launch_bounds__(kWave * 4) void aff_diag_kernel(
     };
     int g = 0;
     for (; g < g_lo; ++g) group(g, std::false_type{});
-    // two groups at a time while the words read ahead lie inside the sequences
-    // (the band's lanes: eight pair-steps of steady cells)
-    if (uni.ok && g + 4 <= g_hi && aff_gap_free(A, la) && aff_gap_free(B, lb)) {
+    // two groups at a time to the end: cells past the last row or column
+    // reach no cell inside, and the backtrace does not visit them
+    if (uni.ok && g < groups && min(la, lb) >= 4 && aff_gap_free(A, la) && aff_gap_free(B, lb)) {
       constexpr uint32_t kHigh4 = 4u * kHighNum;
       const uint32_t go4 = 4u * (uint32_t)go, ins4 = 4u * (uint32_t)uni.ins, del4 = 4u * (uint32_t)uni.del;
       AffFree S[R];
@@ -850,18 +859,21 @@ __global__ __launch_bounds__(kWave * 4) void aff_diag_kernel(
         const uint32_t k0 = left || shut0 ? 0 : 0x00ff00ffu, k1 = shut1 ? 0 : 0xff00ff00u;
         keep[r] = k0 | k1;
         edge[r] = ~keep[r] & ((left ? kAffLeft * 0x00010001u : kAffRight * 0x00010001u) | kAffRight * 0x01000100u);
-        a0[r] = load_four(A, i0[r] + 2 * g, la);
-        b0[r] = load_four(B, j0[r] + 2 * g, lb);
+        a0[r] = four_at(load_four(A, i0[r] + 2 * g, la), i0[r] + 2 * g, la);
+        b0[r] = four_at(load_four(B, j0[r] + 2 * g, lb), j0[r] + 2 * g, lb);
         a1[r] = load_four(A, i0[r] + 2 * g + 4, la);
         b1[r] = load_four(B, j0[r] + 2 * g + 4, lb);
       }
       uint32_t *dst[R];
 #pragma unroll
       for (int r = 0; r < R; ++r) dst[r] = dmw[r] + (size_t)g * dmw_step[r];
-      for (; g + 4 <= g_hi; g += 2) {
+      for (; g < groups; g += 2) {
         uint32_t zero[R][2];   // per byte 1 where the characters share no symbol: even and odd steps
 #pragma unroll
         for (int r = 0; r < R; ++r) {
+          // (read a round ago; the positions that hold no character count as mismatches)
+          a1[r] = four_at(a1[r], i0[r] + 2 * g + 4, la);
+          b1[r] = four_at(b1[r], j0[r] + 2 * g + 4, lb);
           const uint32_t xe = a0[r] & b0[r] & 0x0f0f0f0fu,
                          xo = a0[r] & __builtin_amdgcn_alignbyte(b1[r], b0[r], 1) & 0x0f0f0f0fu;
           zero[r][0] = (~(xe + 0x7f7f7f7fu) >> 7) & 0x01010101u;
@@ -898,32 +910,22 @@ __global__ __launch_bounds__(kWave * 4) void aff_diag_kernel(
               o[r][2 * q + 1] = aff_free_cell(S[r], S[r].eh1, S[r].cb1, ev_u[r], cb_u[r], go4 - 1, go4 + 1, ins4,
                                               gap_v1[r], __builtin_amdgcn_udot4(zero[r][1], sub, 0, false), c1[r]);
           }
-          if (kBt) {
+          if (kBt && g + h < groups) {
 #pragma unroll
             for (int r = 0; r < R; ++r) {
               *dst[r] = aff_free_bytes(o[r], keep[r], edge[r]);
               dst[r] += dmw_step[r];
             }
           }
-        }
-      }
-      // the general groups' state
-      const int s = 2 * g - 1, base = 64 * ((g - 1) >> 5);
-      awin = load_or0(A, 20 + base + lane, la);
-      anext = load_or0(A, 84 + base + lane, la);
-      bwin = load_or0(B, bbase + base + lane, lb);
-      bnext = load_or0(B, bbase + base + 64 + lane, lb);
+          if (g + h == groups - 1) {   // the last cell is in the last group
 #pragma unroll
-      for (int r = 0; r < R; ++r) {
-        L.S[r] = AffDiag{(int)(S[r].eh1 >> 2), (int)(S[r].ev1 >> 2), kHigh, (int)(S[r].cb1 >> 2),
-                         (int)(S[r].eh2 >> 2), (int)(S[r].ev2 >> 2), kHigh, (int)(S[r].cb2 >> 2)};
-        L.ic[r] = load_or0(A, i0[r] + s, la);
-        L.ip[r] = load_or0(A, i0[r] + s - 1, la);
-        L.jc[r] = load_or0(B, j0[r] + s + 1, lb);
-        L.jp[r] = load_or0(B, j0[r] + s, lb);
-        L.si_ge[r] = L.sive[r] = s_cost[L.ic[r] * 32 + kGap];
-        L.gap_row[r] = L.hx[r] = s_prep[L.jc[r]];
-        L.si_go[r] = L.sj_go[r] = go;
+            for (int r = 0; r < R; ++r) {
+              const int u = (la + lb) & 3;
+              const uint32_t kf = u == 0 ? o[r][0].kf : u == 1 ? o[r][1].kf : u == 2 ? o[r][2].kf : o[r][3].kf;
+              L.fcost[r] = (int)(kf >> 2);
+            }
+          }
+        }
       }
     }
     for (; g < g_hi; ++g) group(g, std::true_type{});
@@ -1439,7 +1441,7 @@ __global__ __launch_bounds__(kWave * 4, 3) void aff_quad_kernel(
     const int Gs = (la + lb + 4) >> 2;   // groups of 4 steps of this row's pair
     const int pf = active ? pure[p] : 3;
     // steady groups of this row's pair (all cells inside the sequences)
-    const int t_lo = E0 + 82, t_hi = min(2 * lb - E0, 2 * la - 40);
+    const int t_lo = aff_steady_from(E0), t_hi = min(2 * lb - E0, 2 * la - 40);
     const int glo = active ? (t_lo + 3) >> 2 : 0;
     const int ghi = active ? (t_hi >= 3 ? (t_hi - 3) / 4 + 1 : 0) : 0x3fffffff;
     int groups = 0, g_lo = 0, g_hi = 0x3fffffff, all_pure = 1, all_free = 1;
@@ -1949,16 +1951,17 @@ __global__ __launch_bounds__(kWave * 4, 2) void aff_pk_kernel(
     const int pfA = actA ? pure[pA] : 3, pfB = actB ? pure[pB] : 3;
     // steady groups of each pair (all cells inside the sequences)
     auto steady = [&](bool act, int la, int lb, int E0, int &glo, int &ghi) {
-      const int t_lo = E0 + 82, t_hi = min(2 * lb - E0, 2 * la - 40);
+      const int t_lo = aff_steady_from(E0), t_hi = min(2 * lb - E0, 2 * la - 40);
       glo = act ? (t_lo + 3) >> 2 : 0;
       ghi = act ? (t_hi >= 3 ? (t_hi - 3) / 4 + 1 : 0) : 0x3fffffff;
     };
     int gloA, ghiA, gloB, ghiB;
     steady(actA, laA, lbA, E0A, gloA, ghiA);
     steady(actB, laB, lbB, E0B, gloB, ghiB);
-    int groups = 0, g_lo = 0, g_hi = 0x3fffffff, all_pure = 1, all_free = 1;
+    int groups = 0, g_lo = 0, g_hi = 0x3fffffff, g_last = 0x3fffffff, all_pure = 1, all_free = 1;
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
+      g_last = min(g_last, min(__builtin_amdgcn_readlane(GsA, 16 * r), __builtin_amdgcn_readlane(GsB, 16 * r)) - 1);
       const int fA = __builtin_amdgcn_readlane(pfA, 16 * r), fB = __builtin_amdgcn_readlane(pfB, 16 * r);
       all_pure &= fA != 0 && fB != 0;
       all_free &= fA == 3 && fB == 3;
@@ -1976,7 +1979,8 @@ __global__ __launch_bounds__(kWave * 4, 2) void aff_pk_kernel(
     // W a multiple of H, so a lane's dwords are all inside the band's rows or
     // all outside).  Stored one by one, 12 bytes apart between lanes, they
     // bound the fill: 65,536 pairs of 50-5,000 took 9.25 ms with them and the
-    // shorter cells, 9.4 ms with the longer ones; 7.0 ms with this.
+    // shorter cells, 9.4 ms with the longer ones; 7.0 ms with this (6.1 with fewer
+    // general groups at the ends).
     auto store_group = [&](int g, const uint32_t (&dA)[H], const uint32_t (&dB)[H]) {
       if (actA && g < GsA && H * q < WA) __builtin_memcpy(dmwA + (size_t)g * WA + H * q, dA, sizeof dA);
       if (actB && g < GsB && H * q < WB) __builtin_memcpy(dmwB + (size_t)g * WB + H * q, dB, sizeof dB);
@@ -2148,6 +2152,15 @@ __global__ __launch_bounds__(kWave * 4, 2) void aff_pk_kernel(
         }
         store_group(g, dA, dB);
       }
+      if (g >= g_last) {   // some pair's last cell may be in this group
+#pragma unroll
+        for (int k = 0; k < H; ++k)
+#pragma unroll
+          for (int u = 0; u < 4; ++u) {
+            const uint32_t m = halves(4 * g + u == laA + lbA, 4 * g + u == laB + lbB);
+            Q.fcost[k] = (m & o[k][u].kf) | (~m & Q.fcost[k]);
+          }
+      }
     };
     if (groups >= 1536) __builtin_amdgcn_s_setprio(2);
     else if (groups >= 768) __builtin_amdgcn_s_setprio(1);
@@ -2155,7 +2168,7 @@ __global__ __launch_bounds__(kWave * 4, 2) void aff_pk_kernel(
     const int gs_lo = min(g_lo, groups), gs_hi = max(gs_lo, min(g_hi, groups));
     int g = 0;
     for (; g < gs_lo; ++g) group(g, std::integral_constant<int, 0>{});
-    if (all_free && three && g < gs_hi) {
+    if (all_free && three && g < groups) {
       // (a group's first window swap happens in the group: bits both windows here)
       awin = (awin & 0x03c003c0u) << 6;
       anext = (anext & 0x03c003c0u) << 6;
@@ -2182,26 +2195,9 @@ __global__ __launch_bounds__(kWave * 4, 2) void aff_pk_kernel(
       }
       gov0 = q == 0 ? kPkHigh : go4 + kPkRank1;
       gaph0 = q == 0 ? kPkHigh : ins4;
-      for (; g < gs_hi; ++g) free_group(g);
-      awin >>= 6;
-      anext >>= 6;
-      bwin >>= 11;
-      bnext >>= 11;
-#pragma unroll
-      for (int k = 0; k < H; ++k) {
-        Q.ic[k] >>= 6;
-        Q.jc[k] >>= 11;
-        Q.ip[k] = Q.ic[k];   // (only its gap bit is read, and it has none)
-        Q.jp[k] = Q.jc[k];
-        Q.S[k].ev1 &= (int)0xfffcfffcu;
-        Q.S[k].ev2 &= (int)0xfffcfffcu;
-        Q.S[k].cb1 &= (int)0xfffcfffcu;
-        Q.S[k].cb2 &= (int)0xfffcfffcu;
-        Q.S[k].eb1 = Q.S[k].eb2 = (int)kPkHigh;
-        Q.si_ge[k] = Q.sive[k] = lds_pair(s_c4, Q.ic[k] + 2u * kGap * 0x00010001u);
-        Q.gap_row[k] = Q.hx[k] = lds_pair(s_p4, Q.jc[k]);
-        Q.si_go[k] = Q.sj_go[k] = go4;
-      }
+      // to the end: cells past a pair's last row or column reach no cell
+      // inside, and the backtrace does not visit them
+      for (; g < groups; ++g) free_group(g);
     } else if (all_free) {
       for (; g < gs_hi; ++g) group(g, std::integral_constant<int, 3>{});
       // the gap-free groups kept only si_ge and gap_row; for rows and

@@ -181,17 +181,17 @@ def test_affine_three_cost_groups(ctx, oracle, sub, indel, go, alphabet):
     note(f"affine three-cost groups sub={sub} indel={indel} go={go} alphabet={alphabet}")
     rng = np.random.default_rng(900 + sub + 7 * indel + 13 * go)
     pairs = []
-    for n in (99, 100, 101, 102, 103, 107, 108, 109, 110, 116, 124, 250):
+    for n in (3, 4, 5, 20, 21, 22, 24, 29, 31, 38, 41, 42, 60, 99, 100, 101, 102, 103, 250):
         a = rand_seq(rng, n, alphabet)
         pairs.append((a, mutate(rng, a, 0.15, 0.06)))
-    for diff in (46, 47, 48, 79, 80, 207, 208):       # E0 = diff + 8
+    for diff in (46, 47, 48, 79, 80, 207, 208, 463):       # E0 = diff + 8
         a = rand_seq(rng, 420, alphabet)
         b = np.concatenate([a[:200], rand_seq(rng, diff, alphabet)[1:], a[200:]])
         pairs.append((a, mutate(rng, b, 0.1, 0.0)))
-    gapped = pairs[11][0].copy()
+    gapped = pairs[18][0].copy()
     gapped[77] |= GAP
     A = [p[0] for p in pairs] * 2 + [gapped]
-    B = [p[1] for p in pairs] * 2 + [pairs[11][1]]
+    B = [p[1] for p in pairs] * 2 + [pairs[18][1]]
     cm, ref = engine.CostMatrix.of_sub_indel(sub, indel, go), oracle.CM2.sub_indel(sub, indel, go)
     res = engine.run_pairs(ctx, cm, engine.POYG_MODE_AFFINE_ALIGN, batch_of(A), batch_of(B))
     cost = engine.run_pairs(ctx, cm, engine.POYG_MODE_AFFINE_COST, batch_of(A), batch_of(B)).cost
