@@ -36,7 +36,7 @@ hipError_t launch_aff_quad(bool bt, int grid, const PairMeta *meta, const int32_
 hipError_t launch_aff_pk(bool bt, int grid, const PairMeta *meta, const int32_t *order, int n, int *counter,
                          const uint8_t *seq, const DevTcm *tcm, uint8_t *dm, int32_t *cost,
                          const uint8_t *pure, int32_t *redo, int *redo_n, int32_t *tlist, int *tlist_n,
-                         const AffUniform &uni, hipStream_t s);
+                         const AffUniform &uni, bool whole, hipStream_t s);
 int aff_pk_blocks_per_cu(bool bt);
 int aff_trace_list_blocks_per_cu();
 hipError_t launch_aff_trace_list(int grid, const PairMeta *meta, const int32_t *list, const int *list_n, int *counter,
@@ -419,6 +419,7 @@ struct poyg_plan {
   int n_ldiag = 0, grid_ldiag = 0, ldiag_waves = 0;
   LinDiagCosts ldiag_costs{0, 0, 0};
   AffUniform aff_uniform{0, 0, 0, 0};
+  bool whole_lanes = true;   // the packed affine fill's bands are whole lanes wide
   int n_trace = 0;   // linear pairs of the separate backtrace (order_all)
   // the narrow affine bands (order_quad) go to the packed eight-pair fill;
   // its pairs whose cost saturates 16 bits are listed in `redo` for the
@@ -458,6 +459,7 @@ struct poyg_plan {
 
 static int64_t round16(int64_t v) { return (v + 15) & ~(int64_t)15; }
 static constexpr int kPlanCounters = 16;   // work-list counters of a pair plan's run
+static constexpr int64_t kWholeLaneBand = int64_t(32) << 30;   // see poyg_plan_pairs
 static constexpr int kQuadH = 3;   // diagonal pairs per lane of the four-pair kernel
 
 extern "C" {
@@ -895,6 +897,26 @@ static int plan_pairs_impl(poyg_ctx *ctx, const poyg_cm *cm, int mode, int32_t n
     }
     P->cells += cells[k];
   }
+  // Whole lanes cost up to a twentieth more band: a batch of large bands keeps
+  // the exact widths, so that none that fits the device is refused for them
+  // (a lane past the width then stores its dwords one by one).
+  if (affine && align && dm_bytes > kWholeLaneBand) {
+    dm_bytes = 0;
+    P->whole_lanes = false;
+    for (int k = 0; k < n; ++k) {
+      PairMeta &m = meta[k];
+      const int ra = m.lr - 1, cb = m.lc - 1;
+      if (diag[k]) {
+        m.p1 = ((m.p0 + 40) >> 1) + 1;
+        if (ra <= 0) continue;
+        m.dm_off = dm_bytes;
+        dm_bytes += (((int64_t)ra + cb + 4) >> 2) * 4 * m.p1;
+      } else {
+        m.dm_off = dm_bytes;
+        dm_bytes += (int64_t)ra * m.stride;
+      }
+    }
+  }
   // Linear pairs: the diagonal fill, with several waves on a pair where pairs
   // need more than one register per lane and the batch leaves SIMDs idle (a
   // wave's step is shortest with one register; past that the wave per pair
@@ -1302,7 +1324,7 @@ extern "C" int poyg_plan_run(poyg_plan *P, const uint8_t *d_seq, int32_t *d_cost
       if (P->aff_pk)
         return launch_aff_pk(align, grid, meta, (const int32_t *)P->order_quad.p, P->n_quad, ctr + 6, d_seq, tcm, dm,
                              d_cost, (const uint8_t *)P->pure.p, (int32_t *)P->redo.p, ctr + 5,
-                             (int32_t *)P->tlist.p, ctr + 8, P->aff_uniform, st);
+                             (int32_t *)P->tlist.p, ctr + 8, P->aff_uniform, P->whole_lanes, st);
       return launch_aff_quad(align, grid, meta, (const int32_t *)P->order_quad.p, P->n_quad, ctr + 6, d_seq, tcm, dm,
                              d_cost, sink, (const uint8_t *)P->pure.p, (const TraceOut *)P->trout.p, nullptr, st);
     };

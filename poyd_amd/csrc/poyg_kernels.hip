@@ -1873,7 +1873,7 @@ __device__ __forceinline__ uint32_t pk_col_char(const uint8_t *B0, const uint8_t
   return ((uint32_t)load_or0(B0, idx, lb0) << 1) | ((uint32_t)load_or0(B1, idx, lb1) << 17);
 }
 
-template <bool kBt, int H>
+template <bool kBt, int H, bool kWhole = true>
 __global__ __launch_bounds__(kWave * 4, 2) void aff_pk_kernel(
     const PairMeta *__restrict__ meta, const int32_t *__restrict__ order, int n, int *counter,
     const uint8_t *__restrict__ seq, const DevTcm *__restrict__ tcm, uint8_t *dm_base, int32_t *cost_out,
@@ -1975,15 +1975,24 @@ __global__ __launch_bounds__(kWave * 4, 2) void aff_pk_kernel(
     uint32_t awin = pk_row_char(AA, AB, 20 + q, laA, laB);
     uint32_t bwin = pk_col_char(BA, BB, 16 * H - 20 + ((q + 1) & 15), lbA, lbB);
     uint32_t anext = 0, bnext = 0;
-    // a lane's H dwords of both pairs' group g: one access each (the plan makes
-    // W a multiple of H, so a lane's dwords are all inside the band's rows or
-    // all outside).  Stored one by one, 12 bytes apart between lanes, they
-    // bound the fill: 65,536 pairs of 50-5,000 took 9.25 ms with them and the
-    // shorter cells, 9.4 ms with the longer ones; 7.0 ms with this (6.1 with fewer
-    // general groups at the ends).
+    // a lane's H dwords of both pairs' group g: one access each where the plan
+    // made W a multiple of H (kWhole; not if the batch's bands are very large;
+    // told at run time instead, the step of the pairs below was 3% longer).  Stored one by one, 12 bytes apart between
+    // lanes, they bound the fill: 65,536 pairs of 50-5,000 took 9.25 ms with
+    // them and the shorter cells, 9.4 ms with the longer ones; 7.0 ms with this
+    // (6.1 with fewer general groups at the ends).
+    auto store_lane = [&](uint32_t *row, const uint32_t (&d)[H], int W) {
+      if (kWhole) {
+        if (H * q < W) __builtin_memcpy(row + H * q, d, sizeof d);
+      } else {
+#pragma unroll
+        for (int k = 0; k < H; ++k)
+          if (H * q + k < W) row[H * q + k] = d[k];
+      }
+    };
     auto store_group = [&](int g, const uint32_t (&dA)[H], const uint32_t (&dB)[H]) {
-      if (actA && g < GsA && H * q < WA) __builtin_memcpy(dmwA + (size_t)g * WA + H * q, dA, sizeof dA);
-      if (actB && g < GsB && H * q < WB) __builtin_memcpy(dmwB + (size_t)g * WB + H * q, dB, sizeof dB);
+      if (actA && g < GsA) store_lane(dmwA + (size_t)g * WA, dA, WA);
+      if (actB && g < GsB) store_lane(dmwB + (size_t)g * WB, dB, WB);
     };
     auto group = [&](int g, auto variant_tag) {
       constexpr int kVar = decltype(variant_tag)::value;
@@ -3822,8 +3831,11 @@ hipError_t launch_aff_quad(bool bt, int grid, const PairMeta *meta, const int32_
 hipError_t launch_aff_pk(bool bt, int grid, const PairMeta *meta, const int32_t *order, int n, int *counter,
                          const uint8_t *seq, const DevTcm *tcm, uint8_t *dm, int32_t *cost,
                          const uint8_t *pure, int32_t *redo, int *redo_n, int32_t *tlist, int *tlist_n,
-                         const AffUniform &uni, hipStream_t s) {
-  if (bt)
+                         const AffUniform &uni, bool whole, hipStream_t s) {
+  if (bt && !whole)
+    hipLaunchKernelGGL((aff_pk_kernel<true, 3, false>), dim3(grid), dim3(kWave * 4), 0, s, meta, order, n, counter, seq,
+                       tcm, dm, cost, pure, redo, redo_n, tlist, tlist_n, uni);
+  else if (bt)
     hipLaunchKernelGGL((aff_pk_kernel<true, 3>), dim3(grid), dim3(kWave * 4), 0, s, meta, order, n, counter, seq,
                        tcm, dm, cost, pure, redo, redo_n, tlist, tlist_n, uni);
   else

@@ -206,6 +206,37 @@ def test_affine_three_cost_groups(ctx, oracle, sub, indel, go, alphabet):
             assert got[3] == want and all(np.array_equal(x, y) for x, y in zip(got[:3] + got[4:], (med, ri, rj, mwg))), k
 
 
+def test_affine_exact_band_width(ctx, oracle):
+    """A batch whose direction bands pass 32 GiB keeps the exact band width (41
+    diagonal pairs, not 42: the last lane stores its dwords one by one); every
+    copy of the pair gives the oracle's alignment."""
+    from poyd_amd import engine
+    note("affine exact band width")
+    rng = np.random.default_rng(71)
+    a = rand_seq(rng, 5000)
+    b = mutate(rng, a, 0.1, 0.0)
+    n = (32 << 30) // (2501 * 4 * 42) + 1000
+    cm, ref = engine.CostMatrix.of_sub_indel(1, 1, 3), oracle.CM2.sub_indel(1, 1, 3)
+    ln = np.full(n, len(a), np.int32)
+    plan = engine.PairPlan(ctx, cm, engine.POYG_MODE_AFFINE_ALIGN, np.zeros(n, np.int64), ln,
+                           np.full(n, len(a), np.int64), ln)
+    seq = engine.DeviceBuffer.from_array(ctx, np.concatenate([a, b]))
+    cost, out, length = (engine.DeviceBuffer(ctx, size) for size in (4 * n, plan.out_bytes, 16 * n))
+    plan.run(seq.ptr, cost.ptr, out.ptr, length.ptr)
+    assert plan.status() == 0
+    ctx.sync()
+    med, ri, rj, want, mwg = oracle.align_affine_3(a, b, ref)
+    assert (cost.download(np.int32, n) == want).all()
+    lens, rows = length.download(np.int32, 4 * n).reshape(n, 4), out.download(np.uint8, plan.out_bytes).reshape(n, -1)
+    cap = int(plan.cap[0])
+    for slot, w in enumerate((med, mwg, ri, rj)):
+        assert (lens[:, slot] == len(w)).all(), slot
+        bad = (rows[:, (slot + 1) * cap - len(w):(slot + 1) * cap] != w).any(axis=1)
+        assert not bad.any(), (slot, np.flatnonzero(bad)[:10])
+    for buf in (seq, cost, out, length):
+        buf.free()
+
+
 @pytest.mark.parametrize("alphabet", ["dna", "any"])
 def test_affine_packed_fill_saturation(ctx, oracle, alphabet):
     """The packed 16-bit narrow-band fill holds values as 4 v saturated at
