@@ -29,8 +29,10 @@ METRIC = "DP GCUPS (batched NW); TBR joins/s surrogate+exact vs exhaustive, same
 # int32 VALU operations per DP cell counted from the reference recurrences
 # (src/algn.c:1740-1977 affine, :87-453 linear, :2812-3055 cube).
 OPS_PER_CELL = {"affine": 30, "linear": 8, "cube": 20}
-# MI355X: 256 CUs x 4 SIMD x 16 lanes x 2.4 GHz int32 VALU ops; HBM3E 8 TB/s.
-VALU_PEAK_TOPS = 256 * 64 * 2.4e9 / 1e12
+# MI355X: 256 CUs x 4 SIMD x 16 lanes x 2.4 GHz VALU instructions per lane, two
+# operations each in 16-bit halves (v_pk_*), the form most cells of these fills
+# take; HBM3E 8 TB/s.
+VALU_PEAK_TOPS = 2 * 256 * 64 * 2.4e9 / 1e12
 HBM_PEAK_GBS = 8000.0
 
 
@@ -343,8 +345,8 @@ def main() -> int:
               "and the 32-bit fill of the pairs whose cost saturates 16 bits; one span of HIP events on "
               "the main stream (the packed fill's backtraces, aff_trace_list_kernel, are backtrace_ms)") \
         if kind == "affine" \
-        else "cube_rows_kernel (every row class)" if kind == "cube" \
-        else "lin_cost16_kernel (packed 16-bit halves, one pair per wave, 128-row strips)"
+        else "cube_packed_kernel (every row width in one work list)" if kind == "cube" \
+        else "lin_diag_kernel (anti-diagonal wavefront in 16-bit halves, one pair per wave, backtrace fused)"
     out = {
         "metric": METRIC,
         "value": round(gcups, 3),
@@ -377,7 +379,7 @@ def main() -> int:
             "bound": "valu",
             "achieved": round(valu_tops, 3),
             "peak": round(VALU_PEAK_TOPS, 2),
-            "unit": "TOP/s (int32)",
+            "unit": "TOP/s (16-bit halves)",
             "frac": round(valu_tops / VALU_PEAK_TOPS, 4),
             "traffic": measured_traffic(kind),
             "ops_per_cell": ops,
@@ -483,7 +485,7 @@ def bench_tree(args) -> int:
             "bound": "valu",
             "achieved": round(valu, 4),
             "peak": round(VALU_PEAK_TOPS, 2),
-            "unit": "TOP/s (int32)",
+            "unit": "TOP/s (16-bit halves)",
             "frac": round(valu / VALU_PEAK_TOPS, 6),
             "traffic": None,
             "kernel": "whole step (one plan per tree level: a few pairs per launch, each launch as long as "
@@ -869,10 +871,9 @@ def bench_tbr(args) -> int:
     ex_cells, ex_s = r0["exhaustive_cells"], r0["exhaustive_s"]
     valu = ex_cells * OPS_PER_CELL["linear"] / ex_s / 1e12
     out["roofline"] = {"bound": "valu", "achieved": round(valu, 3), "peak": round(VALU_PEAK_TOPS, 2),
-                       "unit": "TOP/s (int32)", "frac": round(valu / VALU_PEAK_TOPS, 4), "traffic": None,
-                       "kernel": "exhaustive round: every linear DP of the round (lin_cost16_kernel / "
-                                 "lin_c16mw_kernel fills, "
-                                 "lin_trace_wave_kernel), 8 ops per band cell over the round's wall time"}
+                       "unit": "TOP/s (16-bit halves)", "frac": round(valu / VALU_PEAK_TOPS, 4), "traffic": None,
+                       "kernel": "exhaustive round: every linear DP of the round (lin_diag_kernel / "
+                                 "lin_diag_group_kernel, their backtraces fused), 8 ops per band cell over the round's wall time"}
     if not args.no_cpu:
         out["cpu_baseline"] = cpu_baseline_tbr(n_taxa, args.cpu_seconds)
     print(json.dumps(out), flush=True)

@@ -1,15 +1,17 @@
 // Three-sequence alignment on gfx950: algn_fill_cube (src/algn.c:2885-3055)
 // and backtrack_3d (:3829-3905).
 //
-// One wavefront fills one cube, row by row (a row = the n3 cells of one
-// (plane, line)), lanes across the s3 axis and the self-gap chain along s3
-// evaluated as a prefix minimum.  The reference walks three row pointers
+// A cube is filled row by row (a row = the n3 cells of one (plane, line)),
+// lanes across the s3 axis and the self-gap chain along s3 evaluated as a
+// prefix minimum: a workgroup of eight waves per triple takes the rows whose
+// inputs are final (the block kernel and its packed form), one wave the
+// triples with rows above 1,024 cells or negative costs.  The reference walks three row pointers
 // that advance n2-1 rows per plane while the output advances n2 rows, so
 // plane p >= 1, line r >= 1 reads its "diagonal", "upper" and "previous"
 // rows at flat row indices out-n2-p, out-n2-p+1 and out-p-1 (and the first
-// line of plane p reads out-n2-p+1).  Those rows are kept in a per-wave ring
-// of n1+n2 rows in global memory.  The direction cube (one code byte per
-// cell) is walked afterwards by one thread per triple.
+// line of plane p reads out-n2-p+1).  Those rows are kept in a ring in
+// global memory.  The direction cube (4 bits per cell; a byte in the one-wave
+// kernel) is walked afterwards by one thread per triple.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -51,7 +53,7 @@ __device__ __forceinline__ void c_lds_sync() {
 }
 
 // Ordering of one wave's own global stores before its later loads of the
-// same rows (every cube kernel runs one wave per workgroup, so workgroup
+// same rows (a triple's rows are written and read by one workgroup, so workgroup
 // scope suffices: no L2 write-back or invalidate is needed).
 __device__ __forceinline__ void c_wave_fence() { __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "workgroup"); }
 
