@@ -52,6 +52,19 @@ inline int lin_diag_regs(int dlo, int dhi) {
     if (pairs <= r * kLinDiagPairsReg) return r;
   return 0;
 }
+// The workgroup form's schedule.  A wave holds the pairs Lw .. Lw + 127 and
+// nothing outside them ("no cell"), so its outermost pairs go wrong, one on
+// each side a time step: an even cell takes a value of the pair below, an odd
+// one of the pair above.  After every sixteenth time step, before an owned pair
+// is wrong, its outer kLinDiagHalo pairs are replaced by the neighbours' own.
+// Time 0 must not cost a pair of them: its odd half step is the first to read
+// the pair above, of which only the origin's holds a cell then
+// (lin_diag_origin_above).
+constexpr int kLinDiagHalo = 16;
+constexpr bool lin_diag_exchange(int group) { return group & 1; }   // behind this group of eight time steps
+// Whether cell (0, 0) is the even cell of pair `above`, the pair above a wave's last.
+constexpr bool lin_diag_origin_above(int dlo, int above) { return !(dlo & 1) && ((-dlo) >> 1) == above; }
+
 // Columns of codes per group of eight time steps, and the bytes of all groups.
 inline int lin_diag_cols(bool group, int k) {
   return group ? kWave + kLinDiagStep / 2 * (k - 1) : kWave * k;

@@ -77,6 +77,9 @@ __device__ __forceinline__ uint32_t lane_below(uint32_t v) {   // lane q <- q - 
 __device__ __forceinline__ uint32_t lane_above(uint32_t v) {   // lane q <- q + 1, lane 63 <- 0
   return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x130, 0xf, 0xf, true);
 }
+__device__ __forceinline__ uint32_t lane_above(uint32_t v, uint32_t last) {   // lane 63 <- last
+  return (uint32_t)__builtin_amdgcn_update_dpp((int)last, (int)v, 0x130, 0xf, 0xf, false);
+}
 __device__ __forceinline__ uint32_t both(uint32_t v) { return v * 0x00010001u; }
 __device__ __forceinline__ uint32_t table_pair(const uint16_t *t, uint32_t a) {
   const uint32_t lo = *(const uint16_t *)((const char *)t + (a & 0xffffu));
@@ -174,8 +177,8 @@ struct DiagFill {
       E[r] = kDm ? best | 0x00030003u : best;
     }
   }
-  __device__ __forceinline__ void odd(bool first) {
-    const uint32_t above = lane_above(E[0]);
+  __device__ __forceinline__ void odd(bool first) { odd(first, lane_above(E[0])); }
+  __device__ __forceinline__ void odd(bool first, uint32_t above) {
 #pragma unroll
     for (int r = 0; r < R; ++r) {
       const uint32_t up = __builtin_amdgcn_alignbit(r < R - 1 ? E[r < R - 1 ? r + 1 : 0] : above, E[r], 16);
@@ -245,7 +248,7 @@ struct DiagFill {
     row_costs();
     col_costs();
     dpp_exec_guard();
-    odd(true);
+    odd(true, lane_above(E[0], lin_diag_origin_above(g.dlo, Lw + 2 * kWave * R) ? 0xffffu : 0u));
     if (g.dlo & 1)
 #pragma unroll
       for (int r = 0; r < R; ++r)
@@ -332,11 +335,10 @@ __device__ __forceinline__ int diag_fill_one(const DiagGeom &g, const LinDiagCos
 }
 
 // One pair on the workgroup's first `waves` waves: wave w holds pairs
-// 96 w .. 96 w + 127, so that neighbours share 32 pairs.  Without exchange a
-// wave's outermost pairs go wrong one diagonal a step; every 16 time steps (32
-// steps) each wave's outer 16 pairs are replaced by the neighbour's, which
-// still are right.  Every wave of the workgroup takes the barriers.
-constexpr int kHaloLanes = 8;   // lanes of 16 pairs
+// 96 w .. 96 w + 127, so that neighbours share 32 pairs, and takes its outer 16
+// pairs from them every 16 time steps (lin_diag_exchange).  Every wave of the
+// workgroup takes the barriers.
+constexpr int kHaloLanes = kLinDiagHalo / 2;   // two pairs a lane
 template <bool kDm, bool kFast>
 __device__ __forceinline__ int diag_fill_group(const DiagGeom &g, const LinDiagCosts &c, bool ins_first,
                                                const uint16_t *tab, uint8_t *dm, int waves,
@@ -356,7 +358,7 @@ __device__ __forceinline__ int diag_fill_group(const DiagGeom &g, const LinDiagC
       f.run8();
       f.store(g, rsrc, k, col, own);
     }
-    if ((k & 1) && waves > 1) {
+    if (lin_diag_exchange(k) && waves > 1) {
       uint2 (*h)[2][kHaloLanes] = halo[(k >> 1) & 1];
       if (on) {
         if (lane >= kHaloLanes && lane < 2 * kHaloLanes) h[wv][0][lane - kHaloLanes] = make_uint2(f.E[0], f.O[0]);

@@ -294,3 +294,71 @@ def test_diagonal_fill_sizes_equal_strips(ctx, sub, indel, alphabet):
                 for k in range(len(A) * (2 if reps > 1 else 1)):
                     for slot in range(3):
                         assert np.array_equal(got[-1].seq(k, slot), got[3].seq(k, slot)), (reps, k, slot)
+
+
+def oracle_align(oracle, a, b, ref, dw):
+    """align_2 with a band parameter: cost and both aligned sequences."""
+    first = len(a) >= len(b)
+    s1, s2 = (a, b) if first else (b, a)
+    cost, dm, lo, hi = oracle.algn_nw(s1, s2, ref, dw, with_dm=True)
+    r1, r2 = oracle.backtrack_2d(dm, lo, hi, s1, s2, ref, first)
+    return (cost, r1, r2) if first else (cost, r2, r1)
+
+
+@pytest.mark.parametrize("sub,indel", [(1, 2), (2, 1), (3, 2)])
+def test_diagonal_fill_long_leading_gaps(ctx, oracle, sub, indel):
+    """Alignments that start (or end) with 33 or more deletions, so that the
+    path runs along column 0 (or ends along the last one), in bands whose
+    origin is the last pair of one of the group's waves, the first of the next,
+    or beside them: first diagonals around -256, -448 and -640, as full bands
+    and as parts.  A single call, a small batch (several waves per pair) and a
+    large one (a wave per pair) equal the oracle."""
+    from poyd_amd import engine
+    rng = np.random.default_rng(170 + sub)
+
+    def block(k, codes):
+        return rng.choice(np.array(codes, np.uint8), k)
+
+    A, B, dws = [], [], []
+
+    def add(extra, cols, dw, tail=False):
+        # `extra` positions that match nothing beside `cols` columns
+        body = block(cols, (1, 2, 4))
+        rows = np.concatenate([body, block(extra, (8,))] if tail else [block(extra, (8,)), body])
+        pair = [np.concatenate([[GAP], x]).astype(np.uint8) for x in (rows, body)]
+        if len(A) % 4 == 3:
+            pair.reverse()
+        A.append(pair[0])
+        B.append(pair[1])
+        dws.append(dw)
+
+    for rows in (253, 254, 255, 256, 257, 258, 446, 447, 448, 449, 450, 640):   # full bands: dlo = -rows
+        add(rows - 60, 60, 3)
+        add(rows - 150, 150, 2)
+        add(rows - 60, 60, 3, tail=True)
+    for reach in (205, 206, 207, 208, 209, 397, 398, 399, 400, 401, 590, 591):   # band parameter and excess: parts
+        add(reach, 2 * reach + 250, 0)
+        add(reach, 2 * reach + 250, 0, tail=True)
+        add(40, 3 * reach + 200, reach - 40)
+        add(40, reach + 50, reach - 40)
+    cm = engine.CostMatrix.of_sub_indel(sub, indel)
+    ref = oracle.CM2.sub_indel(sub, indel)
+    want = [oracle_align(oracle, a, b, ref, dw) for a, b, dw in zip(A, B, dws)]
+    dws = np.array(dws, np.int32)
+    note(f"diagonal fill, leading gaps sub={sub} indel={indel}: {len(A)} pairs")
+    for reps in (1, 24):   # several waves per pair, then one
+        Ar, Br, dr = batch_of(A * reps), batch_of(B * reps), np.tile(dws, reps)
+        cost = engine.run_pairs(ctx, cm, engine.POYG_MODE_LINEAR_COST, Ar, Br, dr).cost
+        res = engine.run_pairs(ctx, cm, engine.POYG_MODE_LINEAR_ALIGN, Ar, Br, dr)
+        for k in range(len(A) * reps):
+            c, oa, ob = want[k % len(A)]
+            assert cost[k] == c and res.cost[k] == c, (reps, k, len(A[k % len(A)]), len(B[k % len(A)]), cost[k], c)
+            if k < len(A) or k % 24 == 5:
+                assert np.array_equal(res.seq(k, 0), oa) and np.array_equal(res.seq(k, 1), ob), (reps, k)
+                assert np.array_equal(res.seq(k, 2), oracle.median_2(oa, ob, ref)), (reps, k)
+    al = engine.Align(ctx)
+    for k in range(0, len(A), 5):
+        assert al.cost_2(A[k], B[k], cm, int(dws[k])) == oracle.cost_2(A[k], B[k], ref, int(dws[k])), k
+        c, oa, ob = oracle.align_2(A[k], B[k], ref)
+        ga, gb, gc = al.align_2(A[k], B[k], cm)
+        assert gc == c and np.array_equal(ga, oa) and np.array_equal(gb, ob), k
