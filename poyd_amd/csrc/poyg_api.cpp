@@ -418,7 +418,8 @@ struct poyg_plan {
   // workgroup per pair, or 0 for one pair per wave
   int n_ldiag = 0, grid_ldiag = 0, ldiag_waves = 0;
   LinDiagCosts ldiag_costs{0, 0, 0};
-  AffUniform aff_uniform{0, 0, 0, 0};
+  AffUniform aff_uniform{0, 0, 0, 0};      // three costs: for the packed fill (32-bit redo past 16 bits)
+  AffUniform aff_uniform_diag{0, 0, 0, 0};   // ... and for the one-pair fill, costs below the closed states'
   bool whole_lanes = true;   // the packed affine fill's bands are whole lanes wide
   int n_trace = 0;   // linear pairs of the separate backtrace (order_all)
   // the narrow affine bands (order_quad) go to the packed eight-pair fill;
@@ -1117,6 +1118,8 @@ static int plan_pairs_impl(poyg_ctx *ctx, const poyg_cm *cm, int mode, int32_t n
                 "less than 2^28 (largest entry %lld, longest pair %lld)", (long long)cmax, (long long)longest);
       return POYG_EINVAL;
     }
+    P->aff_uniform_diag = P->aff_uniform;
+    P->aff_uniform_diag.ok = P->aff_uniform.ok && aff_below_high(P->aff_uniform, dt.gap_open, longest);
   }
   // the cost matrix, the pair descriptors and the work lists travel as one
   // upload: sections of one block at 256-byte offsets
@@ -1331,7 +1334,7 @@ extern "C" int poyg_plan_run(poyg_plan *P, const uint8_t *d_seq, int32_t *d_cost
     auto diag = [&](int q, int grid, hipStream_t st) {
       return launch_aff_diag(align, q == 0 ? 1 : 2 * q, grid, meta, (const int32_t *)P->order_diag[q].p,
                              P->n_diag[q], ctr + 2 + q, d_seq, tcm, dm, d_cost, sink, (const TraceOut *)P->trout.p,
-                             P->aff_uniform, st);
+                             P->aff_uniform_diag, st);
     };
     for (int q = 2; q >= 1; --q)   // the widest bands: 4 and 2 lane sets
       if (P->n_diag[q]) HIP_TRY(diag(q, P->grid_diag[q], rs2));

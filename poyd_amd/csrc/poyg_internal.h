@@ -42,6 +42,17 @@ inline AffUniform uniform_costs(const DevTcm &t) {
   return u;
 }
 
+// Whether every value that an alignment can use stays below kHighNum, the value
+// of the states the reference closes at the band's edges, for pairs of at most
+// `longest` characters.  Every cell of the band has a state of at most one
+// opening and a gap per character, and the next cell adds another opening and a
+// gap; where that can reach kHighNum, a closed state may be the cheaper one, and
+// cells that hold it as any value from kHighNum on do not serve.
+constexpr bool aff_below_high(const AffUniform &u, int gap_open, int64_t longest) {
+  const int gap = u.del > u.ins ? u.del : u.ins, most = u.sub > gap ? u.sub : gap;
+  return (longest + 2) * most + 3 * (int64_t)gap_open < kHighNum;
+}
+
 // Three-dimensional cost matrix block for 5-bit alphabets.
 struct DevTcm3 {
   int cost[32 * 32 * 32];

@@ -553,7 +553,7 @@ struct AffDiagLanes {
 //   constants to rank their candidates;
 // * what closes a cell at the band's edges rides in per-lane constants of the
 //   sums too: a closed cell's states are kHigh or more instead of kHigh (no
-//   path the backtrace follows compares two such values);
+//   path the backtrace follows reads one: aff_below_high, which the plan asks for);
 // * the substitution costs of eight steps come from two words of each
 //   sequence's characters, four bytes at a time (nonzero byte of the AND: the
 //   characters share a symbol), so no character travels between lanes;

@@ -206,6 +206,45 @@ def test_affine_three_cost_groups(ctx, oracle, sub, indel, go, alphabet):
             assert got[3] == want and all(np.array_equal(x, y) for x, y in zip(got[:3] + got[4:], (med, ri, rj, mwg))), k
 
 
+@pytest.mark.parametrize("sub,indel,go", [(1, 1, 1200000), (0, 1, 1000100), (1, 2500, 3), (63, 20000, 1),
+                                          (1, 1, 333000), (1, 1400, 3)])
+def test_affine_costs_past_closed_states(ctx, oracle, sub, indel, go):
+    """Alignments that cost as much as the states the reference closes at the
+    band's edges (HIGH_NUM, src/algn.c:38), and pairs on the other side of the
+    rule for the three-cost groups: one, two and four lane sets, per call and in
+    a batch; costs, and the alignment where the oracle's walk stays in the band."""
+    from poyd_amd import engine
+    note(f"affine costs past the closed states sub={sub} indel={indel} go={go}")
+    rng = np.random.default_rng(910 + sub)
+    A, B = [], []
+    for la, lb in [(30, 30), (60, 75), (80, 110), (60, 160), (61, 300), (60, 505), (200, 290)]:
+        if 2 * (la + lb + 4) * max(indel, go) + 3000000 >= 1 << 29:   # (refused by the plan)
+            continue
+        a = rand_seq(rng, la)
+        A.append(a)
+        B.append(np.concatenate([mutate(rng, a, 0.2, 0.0), rand_seq(rng, lb - la)[1:]]))
+    cm, ref = engine.CostMatrix.of_sub_indel(sub, indel, go), oracle.CM2.sub_indel(sub, indel, go)
+    want = [oracle.cost_affine_3(a, b, ref) for a, b in zip(A, B)]
+    cost = engine.run_pairs(ctx, cm, engine.POYG_MODE_AFFINE_COST, batch_of(A), batch_of(B)).cost
+    assert list(cost) == want
+    res = engine.run_pairs(ctx, cm, engine.POYG_MODE_AFFINE_ALIGN, batch_of(A), batch_of(B), check_band=False)
+    al = engine.Align(ctx)
+    aligned = 0
+    for k, (a, b) in enumerate(zip(A, B)):
+        assert al.cost_2(a, b, cm) == want[k], k
+        try:
+            med, ri, rj, c, mwg = oracle.align_affine_3(a, b, ref)
+        except RuntimeError:   # the reference reads outside its band
+            continue
+        aligned += 1
+        assert res.cost[k] == c, k
+        for slot, w in enumerate((med, mwg, ri, rj)):
+            assert np.array_equal(res.seq(k, slot), w), (k, slot)
+        got = al.align_affine_3(a, b, cm)
+        assert got[3] == c and all(np.array_equal(x, y) for x, y in zip(got[:3] + got[4:], (med, ri, rj, mwg))), k
+    assert aligned
+
+
 def test_affine_exact_band_width(ctx, oracle):
     """A batch whose direction bands pass 32 GiB keeps the exact band width (41
     diagonal pairs, not 42: the last lane stores its dwords one by one); every
