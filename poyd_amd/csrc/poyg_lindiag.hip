@@ -210,9 +210,11 @@ struct DiagFill {
     odd(first);
   }
 
-  // time 0: row 0's and column 0's first cells
+  // time 0: row 0's and column 0's first cells; above: the even value of the
+  // pair above the wave's last (kGroup: the one-wave form has none)
+  template <bool kGroup>
   __device__ __forceinline__ void begin(const DiagGeom &g, int Lw_, const LinDiagCosts &c, bool ins_first,
-                                        const uint16_t *t) {
+                                        const uint16_t *t, uint32_t above = 0u) {
     const int lane = lane_id();
     tab = t;
     Lw = Lw_;
@@ -248,7 +250,7 @@ struct DiagFill {
     row_costs();
     col_costs();
     dpp_exec_guard();
-    odd(true, lane_above(E[0], lin_diag_origin_above(g.dlo, Lw + 2 * kWave * R) ? 0xffffu : 0u));
+    odd(true, kGroup ? lane_above(E[0], above) : lane_above(E[0]));
     if (g.dlo & 1)
 #pragma unroll
       for (int r = 0; r < R; ++r)
@@ -316,7 +318,7 @@ __device__ __forceinline__ int diag_fill_one(const DiagGeom &g, const LinDiagCos
                                              const uint16_t *tab, uint8_t *dm) {
   DiagFill<kDm, kFast, R> f;
   const __amdgpu_buffer_rsrc_t rsrc = __builtin_amdgcn_make_buffer_rsrc(dm, 0, kDm ? 8 * g.groups * g.cols : 0, 0x00020000);
-  f.begin(g, 0, c, ins_first, tab);
+  f.template begin<false>(g, 0, c, ins_first, tab);
   const int col = lane_id() * R;
   int k = 0;
   for (; k < g.groups - 1; ++k) {
@@ -347,7 +349,10 @@ __device__ __forceinline__ int diag_fill_group(const DiagGeom &g, const LinDiagC
   DiagFill<kDm, kFast, 1> f;
   const __amdgpu_buffer_rsrc_t rsrc = __builtin_amdgcn_make_buffer_rsrc(dm, 0, kDm ? 8 * g.groups * g.cols : 0, 0x00020000);
   const bool on = wv < waves;
-  if (on) f.begin(g, kLinDiagStep * wv, c, ins_first, tab);
+  const int first = kLinDiagStep * wv;
+  if (on)
+    f.template begin<true>(g, first, c, ins_first, tab,
+                           lin_diag_origin_above(g.dlo, first + kLinDiagPairsReg) ? 0xffffu : 0u);
   const bool own = (lane >= kHaloLanes || wv == 0) && (lane < kWave - kHaloLanes || wv == waves - 1);
   const int col = kLinDiagStep / 2 * wv + lane;
   int k = 0, cost = -1;
