@@ -19,6 +19,7 @@
 #include <type_traits>
 #include <vector>
 
+#include "poyg_cube.h"
 #include "poyg_internal.h"
 
 namespace poyg {
@@ -322,7 +323,6 @@ __global__ __launch_bounds__(64) void cube_fill_kernel(const TripleMeta *__restr
 // costs that leave the packed kernel's range), 53 in the packed kernel below.
 constexpr int kBig3 = 1 << 28;
 constexpr int kTop3 = 0x7fffffff;
-constexpr int kCubeWaves = 8;
 constexpr int kCubeLines = 2 * kCubeWaves;   // lines of a full chunk
 constexpr int kCubeAhead = 3 * kCubeLines;   // first plane whose chunks' inputs are three chunks old
 
@@ -1263,7 +1263,9 @@ struct TriplePlan {
   std::vector<int64_t> out_off;
   int64_t out_bytes = 0, cells = 0, dm_bytes = 0;
   int64_t scratch_bytes_per_wave = 0;
-  int grid = 1;
+  int grid = 1;        // workgroups of a block kernel launch
+  int fill_grid = 0;   // waves of the chunked fallback; its scratch follows the fill_at rings of the block kernels
+  int fill_at = 0;
   bool narrow = false;   // int16 ring rows
   bool packed = false;   // ... and the packed kernel: one launch for every row class
   bool wide = false;     // ... with triples of more than 512 cells a row
@@ -1422,24 +1424,24 @@ int poyg_triple_plan_create(poyg_ctx *ctx, const poyg_cm3 *cm3, int32_t n, const
   }
   if (n) P->batches.push_back({begin, n});
   const char *wv = getenv("POYG_CUBE_WAVES_PER_CU");
-  const int waves = waves_per_cu > 0 ? waves_per_cu : (wv ? std::max(1, atoi(wv)) : 16);
-  // workgroups of the block kernel (the chunked fallback: waves)
-  P->grid = std::max(1, std::min(n, cus * std::max(1, P->packed && P->wide ? std::min(1, waves / kCubeWaves)
-                                                                           : waves / kCubeWaves)));
+  const CubeGrid shape = cube_grid(n, cus, waves_per_cu > 0 ? waves_per_cu : (wv ? std::max(1, atoi(wv)) : 0),
+                                   P->packed && P->wide);
+  P->grid = shape.rows;
   hipError_t e = hipSuccess;
   auto A = [&](void **p, size_t b) { if (e == hipSuccess) e = hipMalloc(p, b ? b : 16); };
   A(&P->d_tcm, sizeof(DevTcm3));
   A(&P->d_meta, sizeof(TripleMeta) * (size_t)n);
   A(&P->d_order, sizeof(int32_t) * (size_t)n);
   A(&P->d_dm, (size_t)P->dm_bytes);
-  // one scratch region per row class (a batch runs its classes side by side)
-  int n_cls = 0;
+  // one scratch region per row class (a batch runs its classes side by side),
+  // the chunked fallback's, the last in the order, after the others
   {
     bool seen[kCubeClasses] = {};
     for (int k = 0; k < n; ++k) seen[P->group(k)] = true;
-    for (bool x : seen) n_cls += x;
+    if (seen[0]) P->fill_grid = shape.fill;
+    for (int c = 1; c < kCubeClasses; ++c) P->fill_at += seen[c] ? P->grid : 0;
   }
-  A(&P->d_scratch, (size_t)P->scratch_bytes_per_wave * P->grid * std::max(1, n_cls));
+  A(&P->d_scratch, (size_t)P->scratch_bytes_per_wave * (P->fill_at + P->fill_grid));
   A(&P->d_ctr, 64);
   A(&P->d_status, 64);
   for (hipEvent_t *ev : {&P->fork, &P->join, &P->join2})
@@ -1512,10 +1514,10 @@ int poyg_triple_plan_run(void *pp, const uint8_t *d_seq, int32_t *d_cost, uint8_
       const int32_t *o2 = (const int32_t *)P->d_order + q;
       int *ctr = (int *)P->d_ctr + ri;
       if (c == 0) {
-        const int grid = std::max(1, std::min(P->grid, q2 - q));
+        const int grid = std::max(1, std::min(P->fill_grid, q2 - q));
         hipLaunchKernelGGL(cube_fill_kernel, dim3(grid), dim3(64), 0, ls, (const TripleMeta *)P->d_meta, o2,
                            q2 - q, ctr, d_seq, (const DevTcm3 *)P->d_tcm, (uint8_t *)P->d_dm,
-                           (int *)P->d_scratch + (size_t)ri * P->grid * (P->scratch_bytes_per_wave / 4),
+                           (int *)P->d_scratch + (size_t)P->fill_at * (P->scratch_bytes_per_wave / 4),
                            P->scratch_bytes_per_wave / 4, d_cost);
         HIP_TRY3(hipGetLastError());
       } else if (P->packed) {

@@ -542,6 +542,24 @@ def test_three_d_wide_costs(ctx, oracle):
     check_triples(ctx, oracle, 90, 200, shaped_triples(rng, CUBE_SHAPES[:18]))
 
 
+@pytest.mark.parametrize("sub,indel", [(1, 2), (20, 30)])
+def test_three_d_more_long_rows_than_waves(ctx, oracle, sub, indel):
+    """Rows above 1,024 cells, more triples than the chunked kernel has waves
+    (2,048), with every row width of the block kernels beside them."""
+    from poyd_amd import engine
+    note(f"three-dimensional long rows, costs {sub} {indel}")
+    rng = np.random.default_rng(37)
+    some = shaped_triples(rng, [(n1, n2, n3) for n1, n2 in ((2, 3), (4, 2), (3, 3)) for n3 in (1025, 1030, 1089)] +
+                          [(3, 4, 200), (4, 3, 500), (5, 2, 700), (2, 2, 1000)])
+    pick = np.concatenate([np.arange(len(some)), rng.integers(0, 9, 2300)])
+    got = run_triples(ctx, engine.CostMatrix.of_sub_indel(sub, indel), [some[k] for k in pick])
+    ref = oracle.CM3(oracle.CM2.sub_indel(sub, indel))
+    want = [oracle.align_3(*t, ref) for t in some]
+    for q, k in enumerate(pick):
+        assert got[q][0] == want[k][0], (q, k)
+        assert all(np.array_equal(got[q][1][x], want[k][1 + x]) for x in range(3)), (q, k)
+
+
 def test_fitch_matches_oracle(ctx, oracle):
     from poyd_amd import engine
     note("fitch down/up")
