@@ -1686,6 +1686,14 @@ __device__ __forceinline__ uint32_t lds_pair(const uint16_t *t, uint32_t a) {
   const uint32_t hi = *(const uint16_t *)((const char *)t + (a >> 16));
   return lo | (hi << 16);
 }
+// The same in two parts: the entries as read, and put together.
+struct LdsPair {
+  uint32_t lo, hi;
+  __device__ __forceinline__ uint32_t both() const { return lo | (hi << 16); }
+};
+__device__ __forceinline__ LdsPair lds_pair_read(const uint16_t *t, uint32_t a) {
+  return LdsPair{*(const uint16_t *)((const char *)t + (a & 0xffffu)), *(const uint16_t *)((const char *)t + (a >> 16))};
+}
 // 0xffff in the low half if a, in the high half if b
 __device__ __forceinline__ uint32_t halves(bool a, bool b) { return (a ? 0xffffu : 0u) | (b ? 0xffff0000u : 0u); }
 
@@ -1701,9 +1709,9 @@ constexpr uint32_t kPkRowGap = 16u * 64u, kPkColGap = 16u * 2u;
 template <bool kBt, bool kSteady, bool kPure, bool kGapFree>
 __device__ __forceinline__ uint32_t aff_pk_cell(AffDiag &S, uint32_t eh_l, uint32_t cb_l, uint32_t ev_u,
                                                 uint32_t cb_u, int i, int j, int laA, int laB, int lbA, int lbB,
-                                                int E0A, int E0B, uint32_t go4, const uint16_t *s_c4, uint32_t ic,
-                                                uint32_t ip, uint32_t si_ge, uint32_t si_go, uint32_t sive,
-                                                uint32_t jc, uint32_t gap_row, uint32_t sj_go, uint32_t hx,
+                                                int E0A, int E0B, uint32_t go4, uint32_t dg, uint32_t ic, uint32_t ip,
+                                                uint32_t si_ge, uint32_t si_go, uint32_t sive, uint32_t jc,
+                                                uint32_t gap_row, uint32_t sj_go, uint32_t hx,
                                                 uint32_t &fcost, uint32_t open_mask, uint32_t left_mask) {
   if (kGapFree) {
     si_go = go4;
@@ -1729,7 +1737,6 @@ __device__ __forceinline__ uint32_t aff_pk_cell(AffDiag &S, uint32_t eh_l, uint3
     ic_g = c16_bitmask<10>(ic);
     jc_g = c16_bitmask<5>(jc);
   }
-  const uint32_t dg = kGapFree ? lds_pair(s_c4, ic + jc) : lds_pair(s_c4, (ic & 0x03c003c0u) + (jc & 0x001e001eu));
   const uint32_t fv = kGapFree ? c16_add_sat(S.ev2, dg) : c16_add_sat(c16_add_sat(S.ev2, dg), sj_go & ic_g);
   const uint32_t fh = kGapFree ? c16_add_sat(S.eh2, dg) : c16_add_sat(c16_add_sat(S.eh2, dg), si_go & jc_g);
   const uint32_t fc = c16_add_sat(S.cb2, dg);
@@ -1915,15 +1922,13 @@ __global__ __launch_bounds__(kWave * 4, 2) void aff_pk_kernel(
     uint32_t open0[H], open1[H];
     const uint32_t lmask = q == 0 ? kPkHigh : 0u;
     // row constants of both pairs (scaled characters)
-    auto row_consts = [&](uint32_t ic, uint32_t ip, int i, uint32_t &ge, uint32_t &gop, uint32_t &ve) {
-      ge = lds_pair(s_c4, ic + 2u * kGap * 0x00010001u);
+    auto row_consts = [&](uint32_t ic, uint32_t ip, int i, uint32_t ge, uint32_t &gop, uint32_t &ve) {
       const uint32_t ic_g = c16_bitmask<10>(ic), ip_g = c16_bitmask<10>(ip);
       gop = go4 & ~(~ip_g & ic_g);
       const uint32_t m = i > 1 ? (ip_g & ~ic_g) : 0u;
       ve = (m & c16_add_sat(gop, ge)) | (~m & ge);
     };
-    auto col_consts = [&](uint32_t jc, uint32_t jp, int j, uint32_t &gr, uint32_t &gop, uint32_t &x) {
-      gr = lds_pair(s_p4, jc);
+    auto col_consts = [&](uint32_t jc, uint32_t jp, int j, uint32_t gr, uint32_t &gop, uint32_t &x) {
       const uint32_t jc_g = c16_bitmask<5>(jc), jp_g = c16_bitmask<5>(jp);
       gop = go4 & ~(~jp_g & jc_g);
       const uint32_t m = j == 1 ? 0u : (jp_g & ~jc_g);
@@ -1936,9 +1941,11 @@ __global__ __launch_bounds__(kWave * 4, 2) void aff_pk_kernel(
       // the state before step 0: row 19 - L, column L - 20
       Q.ic[k] = pk_row_char(AA, AB, 19 - L, laA, laB);
       Q.ip[k] = pk_row_char(AA, AB, 18 - L, laA, laB);
+      Q.si_ge[k] = lds_pair(s_c4, Q.ic[k] + 2u * kGap * 0x00010001u);
       row_consts(Q.ic[k], Q.ip[k], 19 - L, Q.si_ge[k], Q.si_go[k], Q.sive[k]);
       Q.jc[k] = pk_col_char(BA, BB, L - 20, lbA, lbB);
       Q.jp[k] = pk_col_char(BA, BB, L - 21, lbA, lbB);
+      Q.gap_row[k] = lds_pair(s_p4, Q.jc[k]);
       col_consts(Q.jc[k], Q.jp[k], L - 20, Q.gap_row[k], Q.sj_go[k], Q.hx[k]);
       Q.S[k] = AffDiag{(int)kPkHigh, (int)kPkHigh, (int)kPkHigh, (int)kPkHigh,
                        (int)kPkHigh, (int)kPkHigh, (int)kPkHigh, (int)kPkHigh};
@@ -1994,6 +2001,18 @@ __global__ __launch_bounds__(kWave * 4, 2) void aff_pk_kernel(
       if (actA && g < GsA) store_lane(dmwA + (size_t)g * WA, dA, WA);
       if (actB && g < GsB) store_lane(dmwB + (size_t)g * WB, dB, WB);
     };
+    // The substitution costs of a half step: every read is issued before the
+    // first is waited for.  Left to itself, the compiler put each cell's two
+    // reads before their use, and with few waves on a SIMD every wait showed:
+    // costs of 2,048 pairs of 1,000-2,000 positions with gap-bearing characters
+    // took 1.60 ms, 1.37 this way (4,096 of 200-600: 520 and 450 us).
+    auto read_costs = [&](LdsPair (&dg)[H], auto gap_free) {
+      constexpr uint32_t mi = decltype(gap_free)::value ? 0xffffffffu : 0x03c003c0u;
+      constexpr uint32_t mj = decltype(gap_free)::value ? 0xffffffffu : 0x001e001eu;
+#pragma unroll
+      for (int k = 0; k < H; ++k) dg[k] = lds_pair_read(s_c4, (Q.ic[k] & mi) + (Q.jc[k] & mj));
+      __builtin_amdgcn_sched_barrier(0);
+    };
     auto group = [&](int g, auto variant_tag) {
       constexpr int kVar = decltype(variant_tag)::value;
       constexpr bool kSt = kVar >= 1, kPu = kVar >= 2, kGF = kVar == 3;
@@ -2040,15 +2059,18 @@ __global__ __launch_bounds__(kWave * 4, 2) void aff_pk_kernel(
             }
             Q.ip[0] = old0;
             Q.ic[0] = nic;
-            if (kGF) Q.si_ge[0] = lds_pair(s_c4, nic + 2u * kGap * 0x00010001u);
-            else row_consts(nic, old0, s + 20 - Lg[0], Q.si_ge[0], Q.si_go[0], Q.sive[0]);
+            const LdsPair ge = lds_pair_read(s_c4, nic + 2u * kGap * 0x00010001u);
+            LdsPair dg[H];
+            read_costs(dg, std::integral_constant<bool, kGF>{});
+            Q.si_ge[0] = ge.both();
+            if (!kGF) row_consts(nic, old0, s + 20 - Lg[0], Q.si_ge[0], Q.si_go[0], Q.sive[0]);
 #pragma unroll
             for (int k = H - 1; k >= 0; --k) {
               const uint32_t eh_l = k == 0 ? eh_l0 : (uint32_t)Q.S[k > 0 ? k - 1 : 0].eh1;
               const uint32_t cb_l = k == 0 ? cb_l0 : (uint32_t)Q.S[k > 0 ? k - 1 : 0].cb1;
               by[k][2 * h] = aff_pk_cell<kBt, kSt, kPu, kGF>(
                   Q.S[k], eh_l, cb_l, (uint32_t)Q.S[k].ev1, (uint32_t)Q.S[k].cb1, s + 20 - Lg[k], s - 20 + Lg[k],
-                  laAg, laBg, lbAg, lbBg, E0Ag, E0Bg, go4, s_c4, Q.ic[k], Q.ip[k], Q.si_ge[k], Q.si_go[k],
+                  laAg, laBg, lbAg, lbBg, E0Ag, E0Bg, go4, dg[k].both(), Q.ic[k], Q.ip[k], Q.si_ge[k], Q.si_go[k],
                   Q.sive[k], Q.jc[k], Q.gap_row[k], Q.sj_go[k], Q.hx[k], Q.fcost[k], e0g[k], k == 0 ? lmg : 0u);
             }
           }
@@ -2072,15 +2094,18 @@ __global__ __launch_bounds__(kWave * 4, 2) void aff_pk_kernel(
             }
             Q.jp[H - 1] = oldt;
             Q.jc[H - 1] = njc;
-            if (kGF) Q.gap_row[H - 1] = lds_pair(s_p4, njc);
-            else col_consts(njc, oldt, s - 19 + Lg[H - 1], Q.gap_row[H - 1], Q.sj_go[H - 1], Q.hx[H - 1]);
+            const LdsPair gr = lds_pair_read(s_p4, njc);
+            LdsPair dg[H];
+            read_costs(dg, std::integral_constant<bool, kGF>{});
+            Q.gap_row[H - 1] = gr.both();
+            if (!kGF) col_consts(njc, oldt, s - 19 + Lg[H - 1], Q.gap_row[H - 1], Q.sj_go[H - 1], Q.hx[H - 1]);
 #pragma unroll
             for (int k = 0; k < H; ++k) {
               const uint32_t ev_u = k == H - 1 ? ev_u0 : (uint32_t)Q.S[k < H - 1 ? k + 1 : 0].ev1;
               const uint32_t cb_u = k == H - 1 ? cb_u0 : (uint32_t)Q.S[k < H - 1 ? k + 1 : 0].cb1;
               by[k][2 * h + 1] = aff_pk_cell<kBt, kSt, kPu, kGF>(
                   Q.S[k], (uint32_t)Q.S[k].eh1, (uint32_t)Q.S[k].cb1, ev_u, cb_u, s + 20 - Lg[k], s - 19 + Lg[k],
-                  laAg, laBg, lbAg, lbBg, E0Ag, E0Bg, go4, s_c4, Q.ic[k], Q.ip[k], Q.si_ge[k], Q.si_go[k],
+                  laAg, laBg, lbAg, lbBg, E0Ag, E0Bg, go4, dg[k].both(), Q.ic[k], Q.ip[k], Q.si_ge[k], Q.si_go[k],
                   Q.sive[k], Q.jc[k], Q.gap_row[k], Q.sj_go[k], Q.hx[k], Q.fcost[k], e1g[k], 0u);
             }
           }
