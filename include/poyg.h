@@ -60,12 +60,13 @@ int poyg_ctx_sync(poyg_ctx *ctx);
  * CUs / value compute units), "lin_sys_blocks_per_cu" and
  * "lin_trace_blocks_per_cu" (1..occupancy: resident workgroups per CU of the
  * linear fill and backtrace), "cube_waves_per_cu" (1..64, default
- * 16: resident waves per CU of the three-way fill, whose workgroups have eight),
- * "lin_cost_kernel" (1: the 32-bit systolic linear fill for every pair it
- * takes; 2, the default: the 16-bit fill over the band's diagonals where a
- * pair's costs and band allow it, else the packed 16-bit strips, one wave per
- * pair, or four waves per pair when the batch has at most two such pairs per
- * CU; 3 and 4: the strips with one, four waves per pair whatever the batch
+ * 16: resident waves per CU of the three-way fill, whose workgroups have
+ * eight, and 8 of its form for rows above 1,024 cells and negative costs, whose
+ * workgroups have one), "lin_cost_kernel" (1: the 32-bit systolic linear fill
+ * for every pair it takes; 2, the default: the 16-bit fill over the band's
+ * diagonals where a pair's costs and band allow it and the batch's shapes favour
+ * it, else the packed 16-bit strips, one wave per pair, or four waves per pair
+ * when the batch has at most two such pairs per CU; 3 and 4: the strips with one, four waves per pair whatever the batch
  * size), "aff_narrow_kernel" (1: the 32-bit four-pair affine fill for the
  * narrow bands; 2, the default: the packed eight-pair fill).  A negative
  * value restores the default.  poyd_amd/autotune.py picks them by timed

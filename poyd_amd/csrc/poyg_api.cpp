@@ -774,10 +774,9 @@ static int plan_pairs_impl(poyg_ctx *ctx, const poyg_cm *cm, int mode, int32_t n
                                                  : lin_trace_blocks_per_cu();
   std::vector<PairMeta> meta(n);
   std::vector<int64_t> cells(n);
-  std::vector<char> glb(n, 0), diag(n, 0), quad(n, 0), sys(n, 0), c16(n, 0), ldiag(n, 0);
+  std::vector<char> glb(n, 0), diag(n, 0), quad(n, 0), sys(n, 0), c16(n, 0);
   std::vector<int> widest(affine ? 0 : n);
-  int64_t diag_waves = 0;   // waves the batch's diagonal pairs would take
-  bool diag_multi = false;
+  std::vector<LinDiagPair> shape(affine ? 0 : n, LinDiagPair{1, 0, 0, false});
   DevTcm dt;
   to_dev_tcm(cm, &dt);
   // the packed 16-bit fill: linear plans whose tail costs equal the
@@ -886,14 +885,12 @@ static int plan_pairs_impl(poyg_ctx *ctx, const poyg_cm *cm, int mode, int32_t n
       lin_band_extent(m.lr, m.lc, g, maxw, c);
       cells[k] = c;
       widest[k] = maxw;
+      shape[k].cols = m.lc;
+      shape[k].strips = c16_matrix && m.lc >= 2 && m.lc <= kLinStageHost &&
+                        ((int64_t)m.lr + m.lc + 2) * std::max<int64_t>(c16_cmax, 1) < 0xfff0;
       if (ldiag_matrix && lin_diag_fits(m.lr, m.lc, g) &&
           ((int64_t)m.lr + m.lc + 2) * std::max<int64_t>(c16_cmax, 1) * (align ? 4 : 1) < 0xfff0) {
-        int dlo, dhi;
-        lin_diag_range(m.lr, m.lc, g, dlo, dhi);
-        ldiag[k] = 1;
-        const int w = lin_diag_waves(dlo, dhi);
-        diag_waves += w ? w : 1 << 20;
-        diag_multi = diag_multi || w > 1;
+        lin_diag_range(m.lr, m.lc, g, shape[k].dlo, shape[k].dhi);
       }
     }
     P->cells += cells[k];
@@ -918,37 +915,25 @@ static int plan_pairs_impl(poyg_ctx *ctx, const poyg_cm *cm, int mode, int32_t n
       }
     }
   }
-  // Linear pairs: the diagonal fill, with several waves on a pair where pairs
-  // need more than one register per lane and the batch leaves SIMDs idle (a
-  // wave's step is shortest with one register; past that the wave per pair
-  // wins, which computes no shared diagonals); the strips, the systolic fill or
-  // the row kernels for the pairs it does not take.  Pairs of 1,500-2,000
-  // (2.4 waves each), several waves against one: costs of 256 / 768 / 1,024
-  // pairs 186 / 364 / 442 us against 374 / 382 / 385; alignments of 256 / 512 /
-  // 1,024 pairs 283 / 370 / 398 against 353 / 356 / 361.
-  const bool diag_group = diag_multi && diag_waves <= (align ? 4 : 8) * ctx->cus;
+  // Linear pairs: the diagonal fill for those it is the faster one for, the
+  // strips, the systolic fill or the row kernels for the others.
+  const LinDiagChoice diag_choice = lin_diag_choose(shape, align, P->ldiag_costs.fast != 0, ctx->cus);
+  const bool diag_group = diag_choice.group;
   int max_waves = 0;
   for (int k = 0; !affine && k < n; ++k) {
     PairMeta &m = meta[k];
-    const LinGeom g{m.p0, m.p1, m.p2};
-    if (ldiag[k]) {
-      int dlo, dhi;
-      lin_diag_range(m.lr, m.lc, g, dlo, dhi);
-      const int f = diag_group ? lin_diag_waves(dlo, dhi) : lin_diag_regs(dlo, dhi);
-      ldiag[k] = f > 0;
-      if (f) {
-        m.p0 = dlo;
-        m.p1 = dhi;
-        m.p2 = f;
-        m.p3 = 2;
-        m.stride = lin_diag_cols(diag_group, f);
-        if (align) {
-          m.dm_off = (dm_bytes + 7) & ~(int64_t)7;
-          dm_bytes = m.dm_off + lin_diag_bytes(m.lr, m.lc, dlo, m.stride);
-        }
-        max_waves = std::max(max_waves, f);
-        continue;
+    if (const int f = diag_choice.form[k]) {
+      m.p0 = shape[k].dlo;
+      m.p1 = shape[k].dhi;
+      m.p2 = f;
+      m.p3 = 2;
+      m.stride = lin_diag_cols(diag_group, f);
+      if (align) {
+        m.dm_off = (dm_bytes + 7) & ~(int64_t)7;
+        dm_bytes = m.dm_off + lin_diag_bytes(m.lr, m.lc, m.p0, m.stride);
       }
+      max_waves = std::max(max_waves, f);
+      continue;
     }
     m.stride = lin_dm_stride(widest[k]);   // room for a row start phase of up to 3 bytes (systolic fill)
     if (align && !lin_dm_fits(m.lr, widest[k])) {
@@ -963,8 +948,7 @@ static int plan_pairs_impl(poyg_ctx *ctx, const poyg_cm *cm, int mode, int32_t n
       m.dm_off = dm_bytes;
       dm_bytes += (int64_t)m.lr * m.stride;
     }
-    if (c16_matrix && m.lc >= 2 && m.lc <= kLinStageHost &&
-        ((int64_t)m.lr + m.lc + 2) * std::max<int64_t>(c16_cmax, 1) < 0xfff0) {
+    if (shape[k].strips) {
       c16[k] = 1;
       m.p3 = 1;
     } else if (m.lc <= kLinStageHost) {
@@ -982,7 +966,7 @@ static int plan_pairs_impl(poyg_ctx *ctx, const poyg_cm *cm, int mode, int32_t n
   std::vector<int32_t> o_lds, o_glb, o_sys, o_c16, o_quad, o_diag[3], o_rows, o_ldiag, o_trace;
   int64_t c_quad3 = 0, c_diag1 = 0;
   for (int k : order) {
-    if (ldiag[k]) {
+    if (!affine && diag_choice.form[k]) {
       o_ldiag.push_back(k);
       continue;
     }

@@ -210,3 +210,89 @@ def test_group_schedule_equals_recurrence(tmp_path):
     assert all(r[5] > 0 for r in rows)
     wrong = [r for r in rows if r[6]]
     assert not wrong, (len(wrong), wrong[:5])
+
+
+CHOICE = r'''
+#include <cstdio>
+#include "poyg_lindiag.h"
+using namespace poyg;
+// lines: align fast cus kinds, then per kind: count rows columns band-parameter fill strips
+int main() {
+  int align, fast, cus, kinds;
+  while (scanf("%d %d %d %d", &align, &fast, &cus, &kinds) == 4) {
+    std::vector<LinDiagPair> p;
+    std::vector<int> kind;
+    for (int q = 0; q < kinds; ++q) {
+      int count, m, n, dw, fill, strips;
+      scanf("%d %d %d %d %d %d", &count, &m, &n, &dw, &fill, &strips);
+      const LinGeom g = lin_geom(m, n, dw);
+      LinDiagPair x{1, 0, n, strips != 0};
+      if (fill && lin_diag_fits(m, n, g)) lin_diag_range(m, n, g, x.dlo, x.dhi);
+      p.insert(p.end(), count, x);
+      kind.insert(kind.end(), count, q);
+    }
+    const LinDiagChoice c = lin_diag_choose(p, align != 0, fast != 0, cus);
+    printf("%d", c.group ? 1 : 0);
+    for (int q = 0; q < kinds; ++q)
+      for (size_t k = 0; k < p.size(); ++k)
+        if (kind[k] == q) {
+          printf(" %d", c.form[k]);
+          break;
+        }
+    printf("\n");
+  }
+  return 0;
+}
+'''
+
+
+@pytest.mark.skipif(shutil.which("g++") is None, reason="g++ not available")
+def test_choice_of_fill(tmp_path):
+    """Which batches go to the diagonal fill, with several waves per pair or
+    one, and which to the strips, on both sides of every rule."""
+    src, exe = tmp_path / "choice.cpp", tmp_path / "choice"
+    src.write_text(CHOICE)
+    subprocess.run(["g++", "-O2", "-std=c++17", "-I", CSRC, "-o", str(exe), str(src)], check=True)
+    cost, align, fast, table = 0, 1, 1, 0
+    near, plane, wide, skinny = (1000, 995, 10), (600, 300, 10), (1500, 900, 10), (950, 40, 10)
+    two, long = (300, 150, 10), (3000, 2990, 60)
+    cases = [
+        # one pair each, and batches that several waves per pair fill
+        (cost, fast, [(1, *near, 1, 1)], (0, 1)), (cost, fast, [(1, *plane, 1, 1)], (1, 5)),
+        (cost, fast, [(409, *plane, 1, 1)], (1, 5)), (cost, fast, [(410, *plane, 1, 1)], (0, 4)),
+        (align, fast, [(204, *plane, 1, 1)], (1, 5)), (align, fast, [(205, *plane, 1, 1)], (0, 4)),
+        # tables
+        (cost, table, [(1, *plane, 1, 1)], (1, 0)), (cost, table, [(2000, *plane, 1, 1)], (0, 0)),
+        (cost, table, [(16, *near, 1, 1)], (0, 1)), (cost, table, [(2000, *two, 1, 1)], (0, 2)),
+        (cost, table, [(2000, *near, 1, 1), (2000, *plane, 1, 1)], (0, 1, 4)),
+        (cost, table, [(1999, *near, 1, 1), (2000, *plane, 1, 1)], (0, 0, 0)),
+        (cost, table, [(512, 500, 50, 10, 1, 1)], (1, 3)), (cost, table, [(513, 500, 50, 10, 1, 1)], (1, 0)),
+        (cost, table, [(1024, 200, 100, 10, 1, 1)], (1, 2)),
+        (cost, fast, [(513, 500, 50, 10, 1, 1)], (1, 3)),
+        (cost, table, [(100, *near, 1, 1), (1, *plane, 1, 1)], (1, 0, 0)),
+        (align, table, [(204, *plane, 1, 1)], (1, 5)), (align, table, [(256, *plane, 1, 1)], (0, 0)),
+        (align, table, [(257, *plane, 1, 1)], (0, 4)),
+        # few columns
+        (cost, fast, [(204, *skinny, 1, 1)], (1, 5)), (cost, fast, [(205, *skinny, 1, 1)], (1, 0)), (cost, fast, [(2000, *skinny, 1, 1)], (0, 0)),
+        (cost, fast, [(2000, 900, 65, 10, 1, 1)], (0, 4)),
+        (cost, fast, [(2000, 900, 64, 10, 1, 1), (2001, 900, 65, 10, 1, 1)], (0, 4, 4)),
+        (align, fast, [(2000, *skinny, 1, 1)], (0, 4)),
+        # pairs of more diagonals than the fill holds among others
+        (cost, fast, [(7, *near, 1, 1), (1, *wide, 1, 1)], (0, 0, 0)),
+        (cost, fast, [(511, *near, 1, 1), (1, *wide, 1, 1)], (0, 0, 0)),
+        (cost, fast, [(512, *near, 1, 1), (1, *wide, 1, 1)], (0, 1, 0)),
+        (align, fast, [(900, *near, 1, 1), (300, *wide, 1, 1)], (0, 1, 0)),
+        (align, fast, [(900, *near, 1, 1), (301, *wide, 1, 1)], (0, 0, 0)),
+        (align, fast, [(1024, *near, 1, 1), (1024, *wide, 1, 1)], (0, 1, 0)),
+        # what the strips cannot take stays with the fill
+        (cost, fast, [(7, *long, 1, 0), (1, *wide, 1, 1)], (0, 1, 0)),
+        (cost, table, [(1, *plane, 1, 0)], (1, 5)), (align, fast, [(7, *near, 0, 1), (2, *near, 1, 1)], (0, 0, 0)),
+        (cost, fast, [(7, *near, 0, 0), (2, *near, 1, 1)], (0, 0, 1)),
+    ]
+    text = "".join(f"{mode} {kind} 256 {len(ks)} " + " ".join(" ".join(map(str, k)) for k in ks) + "\n"
+                   for mode, kind, ks, _ in cases)
+    out = subprocess.run([str(exe)], input=text, check=True, capture_output=True, text=True).stdout.splitlines()
+    got = [tuple(map(int, x.split())) for x in out]
+    assert len(got) == len(cases)
+    for c, g in zip(cases, got):
+        assert g == c[3], (c, g)
