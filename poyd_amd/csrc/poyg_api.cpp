@@ -26,7 +26,7 @@ hipError_t launch_prep(bool affine, int grid, const PairMeta *meta, int n, const
 hipError_t launch_aff_fill(bool bt, bool glb, int grid, const PairMeta *meta, const int32_t *order, int n,
                            int *counter, const uint8_t *seq, const DevTcm *tcm, uint8_t *dm, int *aux,
                            int32_t *cost, int *rowscratch, int row_width, hipStream_t s);
-int aff_diag_blocks_per_cu(bool bt, int sets);
+int aff_diag_blocks_per_cu(bool bt, int sets, bool dense);
 int aff_quad_blocks_per_cu(bool bt);
 hipError_t launch_pair_pure(int grid, const PairMeta *meta, const int32_t *order, int n, const uint8_t *seq,
                             uint8_t *pure, hipStream_t s);
@@ -42,7 +42,7 @@ int aff_trace_list_blocks_per_cu();
 hipError_t launch_aff_trace_list(int grid, const PairMeta *meta, const int32_t *list, const int *list_n, int *counter,
                                  const uint8_t *seq, const DevTcm *tcm, const uint8_t *dm, const TraceOut *tro,
                                  hipStream_t s);
-hipError_t launch_aff_diag(bool bt, int sets, int grid, const PairMeta *meta, const int32_t *order, int n,
+hipError_t launch_aff_diag(bool bt, int sets, bool dense, int grid, const PairMeta *meta, const int32_t *order, int n,
                            int *counter, const uint8_t *seq, const DevTcm *tcm, uint8_t *dm, int32_t *cost,
                            uint32_t *sink, const TraceOut *tro, const AffUniform &uni, hipStream_t s);
 hipError_t launch_aff_trace(const PairMeta *meta, const int32_t *order, int n, const uint8_t *seq,
@@ -420,6 +420,7 @@ struct poyg_plan {
   LinDiagCosts ldiag_costs{0, 0, 0};
   AffUniform aff_uniform{0, 0, 0, 0};      // three costs: for the packed fill (32-bit redo past 16 bits)
   AffUniform aff_uniform_diag{0, 0, 0, 0};   // ... and for the one-pair fill, costs below the closed states'
+  bool diag_dense = false;   // the two-set affine fill with three waves a SIMD
   bool whole_lanes = true;   // the packed affine fill's bands are whole lanes wide
   int n_trace = 0;   // linear pairs of the separate backtrace (order_all)
   // the narrow affine bands (order_quad) go to the packed eight-pair fill;
@@ -990,11 +991,12 @@ static int plan_pairs_impl(poyg_ctx *ctx, const poyg_cm *cm, int mode, int32_t n
   P->n_sys = (int)o_sys.size();
   P->n_rows = (int)o_rows.size();
   // persistent grids: exactly the workgroups that can be resident at once
+  // (more pairs than three waves a SIMD hold: the two-set fill's form for three)
+  P->diag_dense = (int64_t)o_diag[1].size() > 12 * (int64_t)ctx->cus;
+  auto diag_bpc = [&](int q) { return aff_diag_blocks_per_cu(align, q == 0 ? 1 : 2 * q, P->diag_dense); };
   for (int q = 0; q < 3; ++q) {
     P->n_diag[q] = (int)o_diag[q].size();
-    if (P->n_diag[q])
-      P->grid_diag[q] = std::max(1, std::min((P->n_diag[q] + 3) / 4,
-                                             ctx->cus * aff_diag_blocks_per_cu(align, q == 0 ? 1 : 2 * q)));
+    if (P->n_diag[q]) P->grid_diag[q] = std::max(1, std::min((P->n_diag[q] + 3) / 4, ctx->cus * diag_bpc(q)));
   }
   P->n_quad = (int)o_quad.size();
   P->aff_pk = P->n_quad > 0 && ctx->tune[kTuneAffNarrow] != 1;
@@ -1041,15 +1043,15 @@ static int plan_pairs_impl(poyg_ctx *ctx, const poyg_cm *cm, int mode, int32_t n
     auto cus_of = [](int grid, int bpc) { return (grid + bpc - 1) / std::max(1, bpc); };
     int side = 0, side2 = 0;   // CUs of the side stream and of the widest-band stream
     for (int q = 1; q < 3; ++q)
-      if (P->n_diag[q]) side2 += cus_of(P->grid_diag[q], aff_diag_blocks_per_cu(align, 2 * q));
+      if (P->n_diag[q]) side2 += cus_of(P->grid_diag[q], diag_bpc(q));
     if (P->n_lds) side2 += cus_of(P->grid_lds, per_cu);
     if (P->n_glb) side2 += cus_of(P->grid_glb, 8);
     if (P->n_quad && P->main_fill != 1) side += cus_of(P->grid_quad, narrow_bpc());
-    if (P->n_diag[0] && P->main_fill != 2) side += cus_of(P->grid_diag[0], aff_diag_blocks_per_cu(align, 1));
+    if (P->n_diag[0] && P->main_fill != 2) side += cus_of(P->grid_diag[0], diag_bpc(0));
     if ((side || side2) && P->main_fill) {
       side = std::min(side, ctx->cus / side_div);
       side2 = std::min(side2, ctx->cus / side_div);
-      const int bpc = P->main_fill == 1 ? narrow_bpc() : aff_diag_blocks_per_cu(align, 1);
+      const int bpc = P->main_fill == 1 ? narrow_bpc() : diag_bpc(0);
       int &grid_main = P->main_fill == 1 ? P->grid_quad : P->grid_diag[0];
       grid_main = std::max(1, std::min(grid_main, (ctx->cus - side - side2) * bpc));
       // a second (third) launch of the main kernel follows the side work on
@@ -1316,7 +1318,7 @@ extern "C" int poyg_plan_run(poyg_plan *P, const uint8_t *d_seq, int32_t *d_cost
                              d_cost, sink, (const uint8_t *)P->pure.p, (const TraceOut *)P->trout.p, nullptr, st);
     };
     auto diag = [&](int q, int grid, hipStream_t st) {
-      return launch_aff_diag(align, q == 0 ? 1 : 2 * q, grid, meta, (const int32_t *)P->order_diag[q].p,
+      return launch_aff_diag(align, q == 0 ? 1 : 2 * q, P->diag_dense, grid, meta, (const int32_t *)P->order_diag[q].p,
                              P->n_diag[q], ctr + 2 + q, d_seq, tcm, dm, d_cost, sink, (const TraceOut *)P->trout.p,
                              P->aff_uniform_diag, st);
     };

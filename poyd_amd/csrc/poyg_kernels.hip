@@ -670,8 +670,13 @@ __device__ __forceinline__ void aff_trace_own(const PairMeta &m, int p, const ui
   aff_trace_pair<K>(m, p, seq, dm_base, s_med, tile, tro.out, tro.out_len, tro.status);
 }
 
-template <bool kBt, int R>
-__global__ __launch_bounds__(kWave * 4) void aff_diag_kernel(
+// kWaves: waves a SIMD must be able to hold.  With the three-cost groups the two
+// sets' alignments need 191 VGPRs (two waves); held to 168 for three they spill
+// ten, which costs small batches (512 pairs of 400-800 and 120 fewer 349 us
+// against 340) and gains large ones (8,192 of them 1.39 ms against 1.45, with
+// gap-bearing characters 2.44 against 2.67).
+template <bool kBt, int R, int kWaves = 1>
+__global__ __launch_bounds__(kWave * 4, kWaves) void aff_diag_kernel(
     const PairMeta *__restrict__ meta, const int32_t *__restrict__ order, int n, int *counter,
     const uint8_t *__restrict__ seq, const DevTcm *__restrict__ tcm, uint8_t *dm_base, int32_t *cost_out,
     uint32_t *sink, const TraceOut *trop, AffUniform uni) {
@@ -3780,16 +3785,17 @@ static int occupancy_cached(int64_t key, F query) {
 
 // Workgroups of aff_diag_kernel<bt, R> one CU holds at once (register and
 // LDS limits), for a persistent grid that is exactly resident.
-template <bool kBt, int R>
+template <bool kBt, int R, int kWaves = 1>
 static int diag_occupancy() {
-  return occupancy_cached(0x100 + 16 * kBt + R, [] {
+  return occupancy_cached(0x100 + 32 * kWaves + 16 * kBt + R, [] {
     int nb = 0;
-    const hipError_t e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, aff_diag_kernel<kBt, R>, kWave * 4, 0);
+    const hipError_t e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, aff_diag_kernel<kBt, R, kWaves>, kWave * 4, 0);
     return (e == hipSuccess && nb > 0) ? nb : 2;
   });
 }
-int aff_diag_blocks_per_cu(bool bt, int sets) {
+int aff_diag_blocks_per_cu(bool bt, int sets, bool dense) {
   if (sets == 1) return bt ? diag_occupancy<true, 1>() : diag_occupancy<false, 1>();
+  if (sets == 2 && bt && dense) return diag_occupancy<true, 2, 3>();
   if (sets == 2) return bt ? diag_occupancy<true, 2>() : diag_occupancy<false, 2>();
   return bt ? diag_occupancy<true, 4>() : diag_occupancy<false, 4>();
 }
@@ -3806,10 +3812,13 @@ static void launch_diag_r(bool bt, int grid, const PairMeta *meta, const int32_t
                        tcm, dm, cost, sink, tro, uni);
 }
 
-hipError_t launch_aff_diag(bool bt, int sets, int grid, const PairMeta *meta, const int32_t *order, int n,
+hipError_t launch_aff_diag(bool bt, int sets, bool dense, int grid, const PairMeta *meta, const int32_t *order, int n,
                            int *counter, const uint8_t *seq, const DevTcm *tcm, uint8_t *dm, int32_t *cost,
                            uint32_t *sink, const TraceOut *tro, const AffUniform &uni, hipStream_t s) {
   if (sets == 1) launch_diag_r<1>(bt, grid, meta, order, n, counter, seq, tcm, dm, cost, sink, tro, uni, s);
+  else if (sets == 2 && bt && dense)
+    hipLaunchKernelGGL((aff_diag_kernel<true, 2, 3>), dim3(grid), dim3(kWave * 4), 0, s, meta, order, n, counter, seq,
+                       tcm, dm, cost, sink, tro, uni);
   else if (sets == 2) launch_diag_r<2>(bt, grid, meta, order, n, counter, seq, tcm, dm, cost, sink, tro, uni, s);
   else launch_diag_r<4>(bt, grid, meta, order, n, counter, seq, tcm, dm, cost, sink, tro, uni, s);
   return hipGetLastError();

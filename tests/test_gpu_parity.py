@@ -206,6 +206,29 @@ def test_affine_three_cost_groups(ctx, oracle, sub, indel, go, alphabet):
             assert got[3] == want and all(np.array_equal(x, y) for x, y in zip(got[:3] + got[4:], (med, ri, rj, mwg))), k
 
 
+def test_affine_wide_pairs_large_batch(ctx, oracle):
+    """More pairs of two lane sets than three waves a SIMD hold (the fill's
+    denser form), with and without gap-bearing characters."""
+    from poyd_amd import engine
+    note("affine wide pairs, large batch")
+    rng = np.random.default_rng(940)
+    A, B = [], []
+    for k in range(40):
+        a = rand_seq(rng, 100, "any" if k % 2 else "dna")
+        A.append(a)
+        B.append(np.concatenate([mutate(rng, a, 0.1, 0.0), rand_seq(rng, 72 + k)[1:]]))
+    pick = np.concatenate([np.arange(40), rng.integers(0, 40, 3400)])
+    cm, ref = engine.CostMatrix.of_sub_indel(1, 1, 3), oracle.CM2.sub_indel(1, 1, 3)
+    res = engine.run_pairs(ctx, cm, engine.POYG_MODE_AFFINE_ALIGN, batch_of([A[k] for k in pick]),
+                           batch_of([B[k] for k in pick]))
+    want = [oracle.align_affine_3(a, b, ref) for a, b in zip(A, B)]
+    assert np.array_equal(res.cost, [want[k][3] for k in pick])
+    for q, k in enumerate(pick):
+        med, ri, rj, _, mwg = want[k]
+        for slot, w in enumerate((med, mwg, ri, rj)):
+            assert np.array_equal(res.seq(q, slot), w), (q, k, slot)
+
+
 @pytest.mark.parametrize("sub,indel,go", [(1, 1, 1200000), (0, 1, 1000100), (1, 2500, 3), (63, 20000, 1),
                                           (1, 1, 333000), (1, 1400, 3)])
 def test_affine_costs_past_closed_states(ctx, oracle, sub, indel, go):
