@@ -296,7 +296,7 @@ __global__ __launch_bounds__(64) void cube_fill_kernel(const TripleMeta *__restr
 }
 
 // ---------------------------------------------------------------------------
-// Block kernel: a workgroup of kCubeWaves waves fills one cube, a wave two
+// Block kernel: a workgroup of kWaves waves (8 or 2) fills one cube, a wave two
 // consecutive rows at a time.  Lane L owns the R consecutive cells k = L*R ..
 // L*R+R-1 of a row (n3 <= 64*R), so a row is one pass: six candidate moves per
 // cell as ranked keys (value*8 + move index; the minimum key is the
@@ -309,11 +309,11 @@ __global__ __launch_bounds__(64) void cube_fill_kernel(const TripleMeta *__restr
 // plane p >= 1 reads rows out-(n2+p-1) ("upper", or "diagonal" on line 0),
 // out-(n2+p) ("diagonal") and out-(p+1) ("previous").  So p + 1 consecutive
 // lines of plane p depend on none of each other: the workgroup computes chunks
-// of min(p + 1, 2 kCubeWaves) lines, one barrier a chunk, and from plane
-// kCubeAhead on the inputs of the next chunk are stored before the current one
+// of min(p + 1, 2 kWaves) lines, one barrier a chunk, and from plane
+// 6 kWaves on the inputs of the next chunk are stored before the current one
 // starts and are loaded while it is computed.  Plane 0 (each line reads the
 // one before) is the first wave's.  Rows live in a ring of n1 + n2 + 2
-// kCubeWaves rows per workgroup (a chunk's stores never reach a row another
+// kWaves rows per workgroup (a chunk's stores never reach a row another
 // wave still reads); T is int16_t when every cell value is provably below 2^15
 // (checked on the host), else int32_t.
 //
@@ -323,8 +323,8 @@ __global__ __launch_bounds__(64) void cube_fill_kernel(const TripleMeta *__restr
 // costs that leave the packed kernel's range), 53 in the packed kernel below.
 constexpr int kBig3 = 1 << 28;
 constexpr int kTop3 = 0x7fffffff;
-constexpr int kCubeLines = 2 * kCubeWaves;   // lines of a full chunk
-constexpr int kCubeAhead = 3 * kCubeLines;   // first plane whose chunks' inputs are three chunks old
+constexpr int cube_lines(int waves) { return 2 * waves; }         // lines of a full chunk
+constexpr int cube_ahead(int waves) { return 3 * cube_lines(waves); }   // first plane whose chunks' inputs are three chunks old
 
 __device__ __forceinline__ int c_shr1(int v, int fill) {
   return __builtin_amdgcn_update_dpp(fill, v, 0x138 /* wave_shr:1 */, 0xf, 0xf, false);
@@ -520,8 +520,8 @@ __device__ __forceinline__ void cube_row_pair(const int (&U0)[R], const int (&D0
   }
 }
 
-template <typename T, int R>
-__global__ __launch_bounds__(64 * kCubeWaves) void cube_block_kernel(
+template <typename T, int R, int kWaves>
+__global__ __launch_bounds__(64 * kWaves) void cube_block_kernel(
     const TripleMeta *__restrict__ meta, const int32_t *__restrict__ order, int n, int *counter,
     const uint8_t *__restrict__ seq, const DevTcm3 *__restrict__ tcm, uint8_t *dm_base, T *scratch,
     int64_t scratch_per_group, int32_t *cost_out) {
@@ -531,11 +531,12 @@ __global__ __launch_bounds__(64 * kCubeWaves) void cube_block_kernel(
   __shared__ int s_z[2][32];
   __shared__ int s_item;
   constexpr int RS = 64 * R;   // ring row stride (elements)
-  constexpr int kPer = 1024 / (64 * kCubeWaves);   // table entries per thread
+  constexpr int kThreads = 64 * kWaves, kLines = cube_lines(kWaves), kAhead = cube_ahead(kWaves);
+  constexpr int kPer = 1024 / kThreads;   // table entries per thread
   const int lane = c_lane(), wv = __builtin_amdgcn_readfirstlane((int)threadIdx.x / 64);
   T *const ring = scratch + (size_t)blockIdx.x * scratch_per_group;
   const int gap = tcm->gap;
-  for (int e = threadIdx.x; e < 1024; e += 64 * kCubeWaves)
+  for (int e = threadIdx.x; e < 1024; e += kThreads)
     s_tab[0][e].x = s_tab[1][e].x = (tcm->cost[gap * 1024 + e] << 3) | kS1;
   for (;;) {
     __syncthreads();   // the previous triple is done in every wave
@@ -556,7 +557,7 @@ __global__ __launch_bounds__(64 * kCubeWaves) void cube_block_kernel(
     else __builtin_amdgcn_s_setprio(0);
     const uint8_t *s1 = seq + off1, *s2 = seq + off2, *s3 = seq + off3;
     uint8_t *dm = dm_base + dm_off;
-    const int W = n1 + n2 + kCubeLines;
+    const int W = n1 + n2 + kLines;
     const int s30 = __builtin_amdgcn_readfirstlane((int)(s3[0] & 31));
     const bool act = lane * R < n3;   // lane holds at least one cell
     // the table of plane p (its part of 1,024 entries per thread)
@@ -564,12 +565,12 @@ __global__ __launch_bounds__(64 * kCubeWaves) void cube_block_kernel(
     auto table_load = [&](int p) {
       const int a = __builtin_amdgcn_readfirstlane((int)(s1[p] & 31));
 #pragma unroll
-      for (int q = 0; q < kPer; ++q) tv[q] = tcm->cost[a * 1024 + q * 64 * kCubeWaves + (int)threadIdx.x];
+      for (int q = 0; q < kPer; ++q) tv[q] = tcm->cost[a * 1024 + q * kThreads + (int)threadIdx.x];
       tz = tcm->cost[(a * 32 + gap) * 32 + (lane & 31)];
     };
     auto table_store = [&](int p) {
 #pragma unroll
-      for (int q = 0; q < kPer; ++q) s_tab[p & 1][q * 64 * kCubeWaves + (int)threadIdx.x].y = (tv[q] << 3) | kS2;
+      for (int q = 0; q < kPer; ++q) s_tab[p & 1][q * kThreads + (int)threadIdx.x].y = (tv[q] << 3) | kS2;
       if (threadIdx.x < 32) s_z[p & 1][lane] = (tz << 3) | kS3;
     };
     if (n1 > 1) table_load(1);
@@ -672,7 +673,7 @@ __global__ __launch_bounds__(64 * kCubeWaves) void cube_block_kernel(
       for (int j = 0; j < R; ++j) z[j] = s_z[buf][yo[j]];
       const int cP3 = __builtin_amdgcn_readfirstlane(s_z[buf][s30]) - (kS3 - kP3);
       if (p + 1 < n1) table_load(p + 1);
-      const int B = min(p + 1, kCubeLines);
+      const int B = min(p + 1, kLines);
       for (int r0 = 0; r0 < n2; r0 += B) {
         const int len = min(B, n2 - r0);
         const int r = r0 + 2 * wv, lines = len - 2 * wv;
@@ -687,9 +688,9 @@ __global__ __launch_bounds__(64 * kCubeWaves) void cube_block_kernel(
           np = p + 1;
           nr0 = 0;
         }
-        ready = np < n1 && np >= kCubeAhead;
+        ready = np < n1 && np >= kAhead;
         if (ready) {
-          const int nlen = min(kCubeLines, n2 - nr0);
+          const int nlen = min(kLines, n2 - nr0);
           int nrr = nrb + 2 * wv;
           nrr -= nrr >= W ? W : 0;
           load_inputs(np, nr0 + 2 * wv, nrr, nlen - 2 * wv);
@@ -863,16 +864,16 @@ struct CubeLds {
   int item;
   uint8_t s2[kPackMax];   // (n2 < kPackMax: every cost bound is at least 1)
 };
-constexpr int kCubePer = 1024 / (64 * kCubeWaves);   // table entries per thread
 
 // One triple by the workgroup; tx: the S1 terms of this thread's table entries.
-template <int R>
+template <int R, int kWaves>
 __device__ __forceinline__ void cube_packed_triple(int t, const TripleMeta *__restrict__ meta,
                                                    const uint8_t *__restrict__ seq, const DevTcm3 *__restrict__ tcm,
                                                    uint8_t *dm_base, uint16_t *const ring, int32_t *cost_out, CubeLds &L,
-                                                   const uint32_t (&tx)[kCubePer], int gap) {
+                                                   const uint32_t (&tx)[1024 / (64 * kWaves)], int gap) {
   constexpr int RS = 64 * R;   // ring row stride (elements)
-  constexpr int kPer = kCubePer;
+  constexpr int kThreads = 64 * kWaves, kLines = cube_lines(kWaves), kAhead = cube_ahead(kWaves);
+  constexpr int kPer = 1024 / kThreads;   // table entries per thread
   uint32_t(&s_tab)[2][32 * 32] = L.tab;
   uint32_t(&s_z)[2][32] = L.z;
   const int lane = c_lane(), wv = __builtin_amdgcn_readfirstlane((int)threadIdx.x / 64);
@@ -888,23 +889,23 @@ __device__ __forceinline__ void cube_packed_triple(int t, const TripleMeta *__re
   else __builtin_amdgcn_s_setprio(0);
   const uint8_t *s1 = seq + off1, *s2 = seq + off2, *s3 = seq + off3;
   uint8_t *dm = dm_base + dm_off;
-  const int W = n1 + n2 + kCubeLines;
+  const int W = n1 + n2 + kLines;
   const int s30 = __builtin_amdgcn_readfirstlane((int)(s3[0] & 31));
   const bool act = lane * R < n3;   // lane holds at least one cell
   int tv[kPer], tz = 0;
   auto table_load = [&](int p) {
     const int a = __builtin_amdgcn_readfirstlane((int)(s1[p] & 31));
 #pragma unroll
-    for (int q = 0; q < kPer; ++q) tv[q] = tcm->cost[a * 1024 + q * 64 * kCubeWaves + (int)threadIdx.x];
+    for (int q = 0; q < kPer; ++q) tv[q] = tcm->cost[a * 1024 + q * kThreads + (int)threadIdx.x];
     tz = tcm->cost[(a * 32 + gap) * 32 + (lane & 31)];
   };
   auto table_store = [&](int p) {
 #pragma unroll
     for (int q = 0; q < kPer; ++q)
-      s_tab[p & 1][q * 64 * kCubeWaves + (int)threadIdx.x] = tx[q] | ((uint32_t)((tv[q] << 3) | kS2) << 16);
+      s_tab[p & 1][q * kThreads + (int)threadIdx.x] = tx[q] | ((uint32_t)((tv[q] << 3) | kS2) << 16);
     if (threadIdx.x < 32) s_z[p & 1][lane] = (uint32_t)((tz << 3) | kS3) & 0xffffu;
   };
-  for (int k = threadIdx.x; k < n2; k += 64 * kCubeWaves) L.s2[k] = s2[k];   // (read after the next barrier)
+  for (int k = threadIdx.x; k < n2; k += kThreads) L.s2[k] = s2[k];   // (read after the next barrier)
   if (n1 > 1) table_load(1);
   // byte offsets of the cells' s3 symbols in a table row (inactive cells:
   // the gap), prefix sums of cost(gap, gap, s3[k]) for k >= 1, S3 terms
@@ -982,7 +983,7 @@ __device__ __forceinline__ void cube_packed_triple(int t, const TripleMeta *__re
   // Planes p >= 1.  Every chunk of every wave issues the same loads and stores
   // (lanes and lines it does not have are dropped by their offsets), so that the
   // waits can count them: with the next chunk's inputs three chunks old (from
-  // plane kCubeAhead on) a wave waits, before its stores, for those of the chunk
+  // plane 6 kWaves on) a wave waits, before its stores, for those of the chunk
   // before -- all older than the loads just issued -- and the barrier waits for
   // nothing else.
   constexpr int kW = R / 2;                  // words of a row per lane
@@ -1078,7 +1079,7 @@ __device__ __forceinline__ void cube_packed_triple(int t, const TripleMeta *__re
       if (p + 1 < n1) table_load(p + 1);
       const __amdgpu_buffer_rsrc_t rcode =
           __builtin_amdgcn_make_buffer_rsrc(dm + (int64_t)p * n2 * dstride, 0, n2 * dstride, 0x00020000);
-      const int B = kPrefetch ? kCubeLines : min(p + 1, kCubeLines);
+      const int B = kPrefetch ? kLines : min(p + 1, kLines);
       for (int r0 = 0; r0 < n2; r0 += B) {
         const int len = min(B, n2 - r0);
         const int r = r0 + 2 * wv, lines = len - 2 * wv;
@@ -1120,14 +1121,14 @@ __device__ __forceinline__ void cube_packed_triple(int t, const TripleMeta *__re
       }
     }
   };
-  planes(std::false_type{}, 1, min(n1, kCubeAhead));
-  if (n1 > kCubeAhead) {
-    load_inputs(kCubeAhead, 2 * wv, down(rb + 2 * wv));
-    planes(std::true_type{}, kCubeAhead, n1);
+  planes(std::false_type{}, 1, min(n1, kAhead));
+  if (n1 > kAhead) {
+    load_inputs(kAhead, 2 * wv, down(rb + 2 * wv));
+    planes(std::true_type{}, kAhead, n1);
     __syncthreads();   // the last stores
   }
   if (n1 > 1) {   // the last row is still in its wave's mm
-    const int at = (n2 - 1) % min(n1, kCubeLines);
+    const int at = (n2 - 1) % min(n1, kLines);
     if (wv == at >> 1) {
       const int c = at & 1 ? last_cell(High{}) : last_cell(Low{});
       cost_out[t] = c;   // every lane stores the same value
@@ -1139,18 +1140,19 @@ __device__ __forceinline__ void cube_packed_triple(int t, const TripleMeta *__re
 // first: workgroups of different row widths in launches of their own, side by
 // side, left a few wide triples waiting for the narrow launch's workgroups (100
 // ms against 70).  kMaxR 8: two workgroups a compute unit, 16: one.
-template <int kMaxR>
-__global__ __launch_bounds__(64 * kCubeWaves, kMaxR <= 8 ? 4 : 2) void cube_packed_kernel(
+template <int kMaxR, int kWaves>
+__global__ __launch_bounds__(64 * kWaves, kMaxR <= 8 ? 4 : 2) void cube_packed_kernel(
     const TripleMeta *__restrict__ meta, const int32_t *__restrict__ order, int n, int *counter,
     const uint8_t *__restrict__ seq, const DevTcm3 *__restrict__ tcm, uint8_t *dm_base, uint16_t *scratch,
     int64_t scratch_per_group, int32_t *cost_out) {
   __shared__ CubeLds L;
   uint16_t *const ring = scratch + (size_t)blockIdx.x * scratch_per_group;
   const int gap = tcm->gap;
-  uint32_t tx[kCubePer];
+  constexpr int kPer = 1024 / (64 * kWaves);
+  uint32_t tx[kPer];
 #pragma unroll
-  for (int q = 0; q < kCubePer; ++q) {
-    const int e = q * 64 * kCubeWaves + (int)threadIdx.x;
+  for (int q = 0; q < kPer; ++q) {
+    const int e = q * 64 * kWaves + (int)threadIdx.x;
     tx[q] = (uint32_t)((tcm->cost[gap * 1024 + e] << 3) | kS1) & 0xffffu;
     L.tab[0][e] = tx[q];   // (plane 0 reads no S2 term that counts)
   }
@@ -1162,11 +1164,11 @@ __global__ __launch_bounds__(64 * kCubeWaves, kMaxR <= 8 ? 4 : 2) void cube_pack
     if (kk >= n) break;
     const int t = __builtin_amdgcn_readfirstlane(order[kk]);
     const int c = (__builtin_amdgcn_readfirstlane(meta[t].l3) + 255) >> 8;   // cube_class
-    if (c <= 1) cube_packed_triple<4>(t, meta, seq, tcm, dm_base, ring, cost_out, L, tx, gap);
-    else if (c == 2) cube_packed_triple<8>(t, meta, seq, tcm, dm_base, ring, cost_out, L, tx, gap);
+    if (c <= 1) cube_packed_triple<4, kWaves>(t, meta, seq, tcm, dm_base, ring, cost_out, L, tx, gap);
+    else if (c == 2) cube_packed_triple<8, kWaves>(t, meta, seq, tcm, dm_base, ring, cost_out, L, tx, gap);
     if constexpr (kMaxR > 8) {
-      if (c == 3) cube_packed_triple<12>(t, meta, seq, tcm, dm_base, ring, cost_out, L, tx, gap);
-      else if (c == 4) cube_packed_triple<16>(t, meta, seq, tcm, dm_base, ring, cost_out, L, tx, gap);
+      if (c == 3) cube_packed_triple<12, kWaves>(t, meta, seq, tcm, dm_base, ring, cost_out, L, tx, gap);
+      else if (c == 4) cube_packed_triple<16, kWaves>(t, meta, seq, tcm, dm_base, ring, cost_out, L, tx, gap);
     }
   }
 }
@@ -1263,6 +1265,7 @@ struct TriplePlan {
   std::vector<int64_t> out_off;
   int64_t out_bytes = 0, cells = 0, dm_bytes = 0;
   int64_t scratch_bytes_per_wave = 0;
+  int waves = kCubeWaves;   // of a block kernel's workgroup: kCubeWaves or kCubeFew
   int grid = 1;        // workgroups of a block kernel launch
   int fill_grid = 0;   // waves of the chunked fallback; its scratch follows the fill_at rings of the block kernels
   int fill_at = 0;
@@ -1287,25 +1290,25 @@ struct TriplePlan {
 static int cube_class(int l3) { return l3 > 1024 ? 0 : (l3 + 255) / 256; }
 
 // Launch ri of a batch uses scratch region ri (launches run side by side).
-template <typename T, int R>
+template <typename T, int R, int kWaves>
 static hipError_t launch_rows(const TriplePlan *P, int ri, const int32_t *ord, int nb, int *ctr,
                               const uint8_t *d_seq, int32_t *d_cost, hipStream_t s) {
   const int grid = std::max(1, std::min(P->grid, nb));
   T *scratch = (T *)((uint8_t *)P->d_scratch + (size_t)ri * P->grid * P->scratch_bytes_per_wave);
-  hipLaunchKernelGGL((cube_block_kernel<T, R>), dim3(grid), dim3(64 * kCubeWaves), 0, s, (const TripleMeta *)P->d_meta, ord, nb, ctr,
+  hipLaunchKernelGGL((cube_block_kernel<T, R, kWaves>), dim3(grid), dim3(64 * kWaves), 0, s, (const TripleMeta *)P->d_meta, ord, nb, ctr,
                      d_seq, (const DevTcm3 *)P->d_tcm, (uint8_t *)P->d_dm, scratch,
                      (int64_t)(P->scratch_bytes_per_wave / (int64_t)sizeof(T)), d_cost);
   return hipGetLastError();
 }
 
-template <typename T>
+template <typename T, int kWaves>
 static hipError_t launch_class(const TriplePlan *P, int c, int ri, const int32_t *ord, int nb, int *ctr,
                                const uint8_t *d_seq, int32_t *d_cost, hipStream_t s) {
   switch (c) {
-    case 1: return launch_rows<T, 4>(P, ri, ord, nb, ctr, d_seq, d_cost, s);
-    case 2: return launch_rows<T, 8>(P, ri, ord, nb, ctr, d_seq, d_cost, s);
-    case 3: return launch_rows<T, 12>(P, ri, ord, nb, ctr, d_seq, d_cost, s);
-    default: return launch_rows<T, 16>(P, ri, ord, nb, ctr, d_seq, d_cost, s);
+    case 1: return launch_rows<T, 4, kWaves>(P, ri, ord, nb, ctr, d_seq, d_cost, s);
+    case 2: return launch_rows<T, 8, kWaves>(P, ri, ord, nb, ctr, d_seq, d_cost, s);
+    case 3: return launch_rows<T, 12, kWaves>(P, ri, ord, nb, ctr, d_seq, d_cost, s);
+    default: return launch_rows<T, 16, kWaves>(P, ri, ord, nb, ctr, d_seq, d_cost, s);
   }
 }
 
@@ -1313,8 +1316,9 @@ static hipError_t launch_packed(const TriplePlan *P, int ri, const int32_t *ord,
                                 int32_t *d_cost, hipStream_t s) {
   const int grid = std::max(1, std::min(P->grid, nb));
   uint16_t *scratch = (uint16_t *)((uint8_t *)P->d_scratch + (size_t)ri * P->grid * P->scratch_bytes_per_wave);
-  auto *k = P->wide ? cube_packed_kernel<16> : cube_packed_kernel<8>;
-  hipLaunchKernelGGL(k, dim3(grid), dim3(64 * kCubeWaves), 0, s, (const TripleMeta *)P->d_meta, ord, nb, ctr, d_seq,
+  auto *k = P->waves == kCubeWaves ? (P->wide ? cube_packed_kernel<16, kCubeWaves> : cube_packed_kernel<8, kCubeWaves>)
+                                   : (P->wide ? cube_packed_kernel<16, kCubeFew> : cube_packed_kernel<8, kCubeFew>);
+  hipLaunchKernelGGL(k, dim3(grid), dim3(64 * P->waves), 0, s, (const TripleMeta *)P->d_meta, ord, nb, ctr, d_seq,
                      (const DevTcm3 *)P->d_tcm, (uint8_t *)P->d_dm, scratch, P->scratch_bytes_per_wave / 2, d_cost);
   return hipGetLastError();
 }
@@ -1388,12 +1392,12 @@ int poyg_triple_plan_create(poyg_ctx *ctx, const poyg_cm3 *cm3, int32_t n, const
     m.flags = c ? 1 : 0;
     dmb[k] = (int64_t)m.l1 * m.l2 * m.dstride;
     const int64_t w = (int64_t)m.l1 + m.l2;
-    const int64_t bytes = c ? (w + kCubeLines) * 64 * 4 * c * (P->narrow ? 2 : 4)
+    const int64_t bytes = c ? (w + cube_lines(kCubeWaves)) * 64 * 4 * c * (P->narrow ? 2 : 4)
                             : 4 * (w * m.l3 + m.l3 + 64);
     need = std::max(need, bytes);
   }
   P->scratch_bytes_per_wave = (need + 255) & ~(int64_t)255;
-  // wave priority: the triples with the most rows (each is one wave's serial work)
+  // wave priority: the triples with the most rows (each is one workgroup's serial work)
   {
     int64_t max_rows = 1;
     for (int k = 0; k < n; ++k) max_rows = std::max(max_rows, (int64_t)P->meta[k].l1 * P->meta[k].l2);
@@ -1424,8 +1428,13 @@ int poyg_triple_plan_create(poyg_ctx *ctx, const poyg_cm3 *cm3, int32_t n, const
   }
   if (n) P->batches.push_back({begin, n});
   const char *wv = getenv("POYG_CUBE_WAVES_PER_CU");
-  const CubeGrid shape = cube_grid(n, cus, waves_per_cu > 0 ? waves_per_cu : (wv ? std::max(1, atoi(wv)) : 0),
-                                   P->packed && P->wide);
+  const int asked = waves_per_cu > 0 ? waves_per_cu : (wv ? std::max(1, atoi(wv)) : 0);
+  const bool one_per_cu = P->packed && P->wide;
+  std::vector<CubeRows> rows;
+  for (int k = 0; k < n; ++k)
+    if (P->cls[k]) rows.push_back(CubeRows{P->meta[k].l1, P->meta[k].l2});
+  P->waves = cube_group_waves(rows, cus, asked, one_per_cu);
+  const CubeGrid shape = cube_grid(n, cus, asked, one_per_cu, P->waves);
   P->grid = shape.rows;
   hipError_t e = hipSuccess;
   auto A = [&](void **p, size_t b) { if (e == hipSuccess) e = hipMalloc(p, b ? b : 16); };
@@ -1522,10 +1531,12 @@ int poyg_triple_plan_run(void *pp, const uint8_t *d_seq, int32_t *d_cost, uint8_
         HIP_TRY3(hipGetLastError());
       } else if (P->packed) {
         HIP_TRY3(launch_packed(P, (int)ri, o2, q2 - q, ctr, d_seq, d_cost, ls));
-      } else if (P->narrow) {
-        HIP_TRY3(launch_class<int16_t>(P, c, ri, o2, q2 - q, ctr, d_seq, d_cost, ls));
+      } else if (P->waves == kCubeWaves) {
+        auto *launch = P->narrow ? launch_class<int16_t, kCubeWaves> : launch_class<int32_t, kCubeWaves>;
+        HIP_TRY3(launch(P, c, ri, o2, q2 - q, ctr, d_seq, d_cost, ls));
       } else {
-        HIP_TRY3(launch_class<int32_t>(P, c, ri, o2, q2 - q, ctr, d_seq, d_cost, ls));
+        auto *launch = P->narrow ? launch_class<int16_t, kCubeFew> : launch_class<int32_t, kCubeFew>;
+        HIP_TRY3(launch(P, c, ri, o2, q2 - q, ctr, d_seq, d_cost, ls));
       }
     }
     if (used_side) {

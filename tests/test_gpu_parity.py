@@ -565,6 +565,33 @@ def test_three_d_wide_costs(ctx, oracle):
     check_triples(ctx, oracle, 90, 200, shaped_triples(rng, CUBE_SHAPES[:18]))
 
 
+# planes around the two-wave workgroup's chunks (min(p + 1, 4) lines; inputs ahead
+# from plane 12 on), lines around multiples of 4, every row width
+FEW_SHAPES = [(n1, n2, n3) for n1, n3 in ((1, 30), (2, 257), (4, 20), (5, 520), (12, 40), (13, 260), (14, 30), (17, 70))
+              for n2 in (1, 2, 3, 4, 5, 8, 9)] + [(20, 21, 60), (26, 7, 300), (15, 12, 790), (13, 3, 1000), (16, 5, 512)]
+
+
+@pytest.mark.parametrize("sub,indel,widest", [(1, 2, 512), (1, 2, 1024), (20, 30, 1024), (90, 200, 1024)])
+def test_three_d_many_small(ctx, oracle, sub, indel, widest):
+    """Batches of small triples, which take workgroups of two waves: packed
+    (costs 1, 2; rows of at most 512 cells and wider ones), 16-bit and 32-bit
+    rows."""
+    note(f"three-dimensional small triples, costs {sub} {indel}")
+    from poyd_amd import engine
+    rng = np.random.default_rng(38)
+    shapes = [s for s in FEW_SHAPES if s[2] <= widest]
+    some = shaped_triples(rng, shapes)
+    pick = np.concatenate([np.arange(len(some)), np.repeat(np.arange(len(some)), 140)])
+    got = run_triples(ctx, engine.CostMatrix.of_sub_indel(sub, indel), [some[k] for k in pick])
+    ref = oracle.CM3(oracle.CM2.sub_indel(sub, indel))
+    want = [oracle.align_3(*t, ref) for t in some]
+    med = [oracle.median_3(*w[1:], ref) for w in want]
+    for q, k in enumerate(pick):
+        assert got[q][0] == want[k][0], (q, shapes[k])
+        assert all(np.array_equal(got[q][1][x], want[k][1 + x]) for x in range(3)), (q, shapes[k])
+        assert np.array_equal(got[q][1][3], med[k]), (q, shapes[k])
+
+
 @pytest.mark.parametrize("sub,indel", [(1, 2), (20, 30)])
 def test_three_d_more_long_rows_than_waves(ctx, oracle, sub, indel):
     """Rows above 1,024 cells, more triples than the chunked kernel has waves
