@@ -521,7 +521,7 @@ __device__ __forceinline__ void cube_row_pair(const int (&U0)[R], const int (&D0
 }
 
 template <typename T, int R, int kWaves>
-__global__ __launch_bounds__(64 * kWaves) void cube_block_kernel(
+__global__ __launch_bounds__(64 * kWaves, kWaves == kCubeWaves || R < 16 ? 2 : 1) void cube_block_kernel(
     const TripleMeta *__restrict__ meta, const int32_t *__restrict__ order, int n, int *counter,
     const uint8_t *__restrict__ seq, const DevTcm3 *__restrict__ tcm, uint8_t *dm_base, T *scratch,
     int64_t scratch_per_group, int32_t *cost_out) {
