@@ -26,14 +26,22 @@ sys.path.insert(0, ROOT)
 
 METRIC = "DP GCUPS (batched NW); TBR joins/s surrogate+exact vs exhaustive, same cost"
 
-# int32 VALU operations per DP cell counted from the reference recurrences
+# Operations per DP cell counted from the reference recurrences
 # (src/algn.c:1740-1977 affine, :87-453 linear, :2812-3055 cube).
 OPS_PER_CELL = {"affine": 30, "linear": 8, "cube": 20}
-# MI355X: 256 CUs x 4 SIMD x 16 lanes x 2.4 GHz VALU instructions per lane, two
-# operations each in 16-bit halves (v_pk_*), the form most cells of these fills
-# take; HBM3E 8 TB/s.
-VALU_PEAK_TOPS = 2 * 256 * 64 * 2.4e9 / 1e12
+# MI355X: 256 CUs x 4 SIMD x 16 lanes x 2.4 GHz VALU instructions per lane, one
+# operation each on 32-bit cells, two in 16-bit halves (v_pk_*); HBM3E 8 TB/s.
+VALU_PEAK_TOPS = {"32-bit": 256 * 64 * 2.4e9 / 1e12, "16-bit halves": 2 * 256 * 64 * 2.4e9 / 1e12}
 HBM_PEAK_GBS = 8000.0
+
+
+def valu_form(kind: str, knobs: dict) -> str:
+    """The form of the cells that the workload's fills take: 16-bit halves,
+    or 32 bits where the launch shapes ask for the 32-bit kernels.  (Of an
+    affine batch, the pairs in wide bands, some per cent of the cells, take
+    32-bit cells either way.)"""
+    asked = {"affine": "aff_narrow_kernel", "linear": "lin_cost_kernel"}.get(kind)
+    return "32-bit" if asked and knobs.get(asked) == 1 else "16-bit halves"
 
 
 def cpu_model() -> str:
@@ -274,7 +282,7 @@ def sub_result(kind: str, steps: int, warmup: int, n_check: int) -> dict:
         ("cube_cells" if r["kind"] == "cube" else "band_cells"): r["cells"],
         "plan_ms": round(r["plan_ms"], 1),
         "fill_ms": round(r["fill_ms"], 3),
-        "valu_frac": round(valu / VALU_PEAK_TOPS, 4),
+        "valu_frac": round(valu / VALU_PEAK_TOPS[valu_form(r["kind"], r["knobs"])], 4),
         **verify(r, want),
     }
 
@@ -328,6 +336,7 @@ def main() -> int:
     gcups = cells / (ms / 1e3) / 1e9
     ops = OPS_PER_CELL[kind]
     valu_tops = cells * ops / (fill_ms / 1e3) / 1e12
+    form = valu_form(kind, r["knobs"])
     # algorithmic HBM bytes of the fill: one direction byte per band cell,
     # both sequences read once, one int32 cost written per pair; the affine
     # fills also run the backtrace of their pairs, which reads both
@@ -378,9 +387,9 @@ def main() -> int:
         "roofline": {
             "bound": "valu",
             "achieved": round(valu_tops, 3),
-            "peak": round(VALU_PEAK_TOPS, 2),
-            "unit": "TOP/s (16-bit halves)",
-            "frac": round(valu_tops / VALU_PEAK_TOPS, 4),
+            "peak": round(VALU_PEAK_TOPS[form], 2),
+            "unit": f"TOP/s ({form})",
+            "frac": round(valu_tops / VALU_PEAK_TOPS[form], 4),
             "traffic": measured_traffic(kind),
             "ops_per_cell": ops,
             "kernel": kernel,
@@ -484,9 +493,9 @@ def bench_tree(args) -> int:
         "roofline": {
             "bound": "valu",
             "achieved": round(valu, 4),
-            "peak": round(VALU_PEAK_TOPS, 2),
+            "peak": round(VALU_PEAK_TOPS["16-bit halves"], 2),
             "unit": "TOP/s (16-bit halves)",
-            "frac": round(valu / VALU_PEAK_TOPS, 6),
+            "frac": round(valu / VALU_PEAK_TOPS["16-bit halves"], 6),
             "traffic": None,
             "kernel": "whole step (one plan per tree level: a few pairs per launch, each launch as long as "
                       "its longest pair takes on one workgroup)",
@@ -870,8 +879,9 @@ def bench_tbr(args) -> int:
     }
     ex_cells, ex_s = r0["exhaustive_cells"], r0["exhaustive_s"]
     valu = ex_cells * OPS_PER_CELL["linear"] / ex_s / 1e12
-    out["roofline"] = {"bound": "valu", "achieved": round(valu, 3), "peak": round(VALU_PEAK_TOPS, 2),
-                       "unit": "TOP/s (16-bit halves)", "frac": round(valu / VALU_PEAK_TOPS, 4), "traffic": None,
+    peak = VALU_PEAK_TOPS["16-bit halves"]
+    out["roofline"] = {"bound": "valu", "achieved": round(valu, 3), "peak": round(peak, 2),
+                       "unit": "TOP/s (16-bit halves)", "frac": round(valu / peak, 4), "traffic": None,
                        "kernel": "exhaustive round: every linear DP of the round (lin_diag_kernel / "
                                  "lin_diag_group_kernel, their backtraces fused), 8 ops per band cell over the round's wall time"}
     if not args.no_cpu:
