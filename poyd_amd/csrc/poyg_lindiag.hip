@@ -35,10 +35,11 @@
 // Bound by VALU issue.  Instructions per time step (four cells a register),
 // from the compiled loops: 29 fast and cost-only, 35 with codes (R = 1), 26 and
 // 32 a register at R = 2, no other instruction but 2-4 wait states.  Measured
-// against the strips with their prefix-sum and backtrace kernels (one MI355X):
-// 16,384 distances of 500-2,000 positions 5.93 to 2.05 ms; 1,000 alignments of
-// 200-400 186 to 71 us; a tree level of 6 medians of 300-1,500 448 to 188 us; one
-// distance of 300 positions 50 to 27 us.
+// against the strips with their prefix-sum and backtrace kernels (one MI355X), a
+// pass: 16,384 distances of 500-2,000 positions 6.0 to 1.95 ms; 1,000 alignments
+// of 200-400 186 to 69 us; a call, its kernels in brackets: a tree level of 6
+// medians of 300-1,500 509 to 255 us (448 to 183), one distance of 300 positions
+// 74 to 51 us (50 to 27).
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
