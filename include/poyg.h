@@ -441,8 +441,9 @@ int poyg_pair_features(poyg_ctx *ctx, const float *d_counts, const int32_t *d_ia
 int poyg_gather_rows(poyg_ctx *ctx, const void *d_src, int64_t row_bytes, const int32_t *d_idx, int64_t n,
                      void *d_dst, void *stream);
 /* C (f32, row stride ldc) = A B over bf16 operands, A(i, k) = a[i*a_rs +
- * k*a_cs], B(k, j) = b[k*b_rs + j*b_cs]: the MFMA tiles the network runs
- * on, exposed for tests. */
+ * k*a_cs], B(k, j) = b[k*b_rs + j*b_cs], for any strides and
+ * 16-byte aligned bases.  The network's own products run in its fused
+ * kernels, not here. */
 int poyg_gemm_bf16_f32(poyg_ctx *ctx, int M, int N, int K, const uint16_t *d_a, int64_t a_rs, int64_t a_cs,
                        const uint16_t *d_b, int64_t b_rs, int64_t b_cs, float *d_c, int64_t ldc, void *stream);
 

@@ -1,7 +1,7 @@
 """Launch shapes of the three-way plans (poyd_amd/csrc/poyg_cube.h): the block
-kernels count workgroups of eight waves, the chunked kernel, whose workgroup is
-one wave, waves.  The header is plain C++; the test compiles a small checker
-with g++."""
+kernels count workgroups of eight waves, or of two for batches of small triples;
+the chunked kernel, whose workgroup is one wave, waves.  The header is plain
+C++; the test compiles a small checker with g++."""
 import os
 import shutil
 import subprocess
